@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "math_f64.hpp"
+
 namespace hexo {
 
 constexpr uint32_t kPhiloxM0 = 0xD2511F53u;
@@ -44,7 +46,7 @@ __device__ __forceinline__ u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_
     return u32x4{c0, c1, c2, c3};
 }
 
-// ---- AS241 coefficients (src/as241.f90:31-44 A/B, :49-63 C/D, :68-82 E/F) ----
+// ---- AS241 coefficients (src/as241.f90:31-44 A/B, :49-63 C/D) ----
 #define HEXO_AS241_A 3.3871328727963666080e0, 1.3314166789178437745e+2, 1.9715909503065514427e+3, \
     1.3731693765509461125e+4, 4.5921953931549871457e+4, 6.7265770927008700853e+4, 3.3430575583588128105e+4, \
     2.5090809287301226727e+3
@@ -55,11 +57,7 @@ __device__ __forceinline__ u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_
     7.74545014278341407640e-4
 #define HEXO_AS241_D 1.0, 2.05319162663775882187e0, 1.67638483018380384940e0, 6.89767334985100004550e-1, \
     1.48103976427480074590e-1, 1.51986665636164571966e-2, 5.47593808499534494600e-4, 1.05075007164441684324e-9
-#define HEXO_AS241_E 6.65790464350110377720e0, 5.46378491116411436990e0, 1.78482653991729133580e0, \
-    2.96560571828504891230e-1, 2.65321895265761230930e-2, 1.24266094738807843860e-3, 2.71155556874348757815e-5, \
-    2.01033439929228813265e-7
-#define HEXO_AS241_F 1.0, 5.99832206555887937690e-1, 1.36929880922735805310e-1, 1.48753612908506148525e-2, \
-    7.86869131145613259100e-4, 1.84631831751005468180e-5, 1.42151175831644588870e-7, 2.04426310338993978564e-15
+
 
 template <typename T>
 struct As241 {
@@ -67,8 +65,6 @@ struct As241 {
     static constexpr T b[8] = {HEXO_AS241_B};
     static constexpr T c[8] = {HEXO_AS241_C};
     static constexpr T d[8] = {HEXO_AS241_D};
-    static constexpr T e[8] = {HEXO_AS241_E};
-    static constexpr T f[8] = {HEXO_AS241_F};
 };
 
 // ((c7 r + c6) r + ...) r + c0 with fused multiply-adds; a leading coefficient of 1 (B, D, F
@@ -94,26 +90,53 @@ __device__ __forceinline__ float uniform_f32(uint32_t k) { return __builtin_fmaf
 __device__ __forceinline__ float one_minus_uniform_f32(uint32_t k) { return uniform_f32(~k); }
 
 // AS241 in FP64, the reference's region logic (src/as241.f90:85-118) on u = (k + 1/2) 2^-32.
-// u never reaches 0 or 1, so the IFAULT branch cannot trigger; 32-bit inputs never reach the
-// far tail (r <= 4.78 < 5), which is kept for completeness.
-__device__ __forceinline__ double normal_f64(uint32_t k) {
-    const double p = uniform_f64(k);
-    const double q = p - 0.5;
-    if (__builtin_fabs(q) <= 0.425) {
-        const double r = 0.180625 - q * q;
-        return q * horner8(As241<double>::a, r) / horner8(As241<double>::b, r);
+// u never reaches 0 or 1, so the IFAULT branch cannot trigger, and sqrt(-ln(min(u, 1 - u))) <= 4.79
+// for 32-bit words, so the far tail (r > 5, the E/F coefficients) is never reached.
+//
+// q = u - 1/2 from the word (exact) and the central region |q| <= 0.425, 85% of the words:
+__device__ __forceinline__ double centred_f64(uint32_t k) { return __builtin_fma((double)k, 0x1p-32, 0x1p-33 - 0.5); }
+__device__ __forceinline__ bool is_tail_f64(double q) { return __builtin_fabs(q) > 0.425; }
+// The tail's |z| from the folded word j = min(k, ~k): p = min(u, 1 - u) = (j + 1/2) 2^-32.
+__device__ __forceinline__ double normal_tail_f64(uint32_t j) {
+    const double r = sqrt_f64(-log_f64(uniform_f64(j))) - 1.6;
+    return div_f64(horner8(As241<double>::c, r), horner8(As241<double>::d, r));
+}
+// The central rational of N words at once: the coefficients are loaded once for all of them, and
+// their reciprocals come from one of the product (the denominators lie in [0.04, 1]); the residual
+// correction leaves each quotient within its last rounding whatever the reciprocal's.
+template <int N>
+__device__ __forceinline__ void normal_central_f64(const double (&q)[N], double (&z)[N]) {
+    static_assert(N == 1 || N == 4, "one word or a counter block's four");
+    double num[N], den[N], rec[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const double r = __builtin_fma(-q[i], q[i], 0.180625);
+        num[i] = q[i] * horner8(As241<double>::a, r);
+        den[i] = horner8(As241<double>::b, r);
     }
-    double r = (q < 0.0) ? p : 1.0 - p;
-    r = ::sqrt(-::log(r));
-    double z;
-    if (r <= 5.0) {
-        r -= 1.6;
-        z = horner8(As241<double>::c, r) / horner8(As241<double>::d, r);
+    if constexpr (N == 4) {
+        const double d01 = den[0] * den[1], d23 = den[2] * den[3], d = d01 * d23;
+        double r = __builtin_amdgcn_rcp(d);
+        r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+        const double r01 = r * d23, r23 = r * d01;
+        rec[0] = r01 * den[1];
+        rec[1] = r01 * den[0];
+        rec[2] = r23 * den[3];
+        rec[3] = r23 * den[2];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const double v = num[i] * rec[i];
+            z[i] = __builtin_fma(__builtin_fma(-den[i], v, num[i]), rec[i], v);
+        }
     } else {
-        r -= 5.0;
-        z = horner8(As241<double>::e, r) / horner8(As241<double>::f, r);
+        z[0] = div_f64(num[0], den[0]);
     }
-    return (q < 0.0) ? -z : z;
+}
+__device__ __forceinline__ double normal_f64(uint32_t k) {
+    const double q[1] = {centred_f64(k)};
+    double z[1];
+    normal_central_f64<1>(q, z);
+    return is_tail_f64(q[0]) ? __builtin_copysign(normal_tail_f64(k ^ (uint32_t)((int32_t)k >> 31)), q[0]) : z[0];
 }
 
 // A value the compiler must keep in a vector register (it cannot prove the result wave-uniform and

@@ -525,6 +525,15 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
             g.fin_count = (uint32_t)S.fins.size();
             g.delta = dl;
             g.dnext = S.dnext;
+            // the FP64 step's constants, each in the reference's own expression (1 - e, not expm1: the
+            // FP64 kernel reproduces its roundings)
+            g.e = dd;
+            g.s2v = e * e * dd / k * (1.0 - dd);
+            g.s2c = th * e * e / (2.0 * k) * (1.0 - dd) * (1.0 - dd);
+            g.dk0 = -rho * k * th / e * dl + d.r_drift * dl;
+            g.dk1 = kc - kd;
+            g.dk2 = kc + kd;
+            g.dk3 = K3;
             for (const HostFin& F : S.fins) {
                 DevFin& f = hf[fin_i++];
                 f.chain = F.chain;

@@ -700,53 +700,105 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 ? 
 }
 #pragma clang fp contract(fast)
 // ------------------------------------------------------------------------------------------
-// Plain FP64 path kernel: the reference's step and policies in FP64, recomputing the step's
-// moments and K0..K4 every step exactly as written in src/HSimulation.tpp:52-86.
+// Plain FP64 path kernel: the reference's step and policies in FP64 (src/HSimulation.tpp:52-86) with
+// the expressions that depend on the run only (e^-kappa dt, the variance's coefficients, K0..K4)
+// taken from the run's record.
+//
+// Bound by FP64 issue (4 cycles per wave instruction, 16 per v_rcp/v_rsq_f64): about 1,200 cycles
+// per wave and step at 3 waves per SIMD. With the constants recomputed every step, the library's
+// division, root, exp and log and the tail normals evaluated for every word it was 2,700: 1e6
+// paths x 252 steps 4.93 -> 2.11 ms, 1e5 x 252 0.715 -> 0.382 ms (kernel, base parameters), a
+// 64-request batch of daily steps 42.9 -> 19.1 ms. Held to 4 waves per SIMD (128 registers) the
+// constants spill and it is 10% slower at 1e6 paths, 25% at 1e5.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ bool qe_step_fp64(const DevReq& R, double delta, double& V, double& logX, uint32_t wv,
-                                             uint32_t wx) {
-    const double theta = R.theta, rho = R.rho, kappa = R.kappa, eps = R.sigma;
-    const double e = ::exp(-kappa * delta);
-    const double m = theta + (V - theta) * e;
-    const double s2 = __builtin_fabs(V * eps * eps * e / kappa * (1.0 - e) +
-                                     theta * eps * eps / (2.0 * kappa) * (1.0 - e) * (1.0 - e));
-    const double psi = s2 / (m * m);
+struct SegD {
+    double e, s2v, s2c, k0, k1, k2, k3, delta;
+};
+
+__device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, double& V, double& logX, uint32_t wv,
+                                             double zv, double zx) {
+    const double m = __builtin_fma(V - R.theta, c.e, R.theta);
+    const double s2 = __builtin_fabs(__builtin_fma(V, c.s2v, c.s2c));
+    const double m2 = m * m;
     const double Vp = V;
-    const bool quad = psi < 1.5;
-    double aq = 0.0, bp2 = 0.0, p = 0.0, beta = 0.0;
+    const bool quad = s2 < 1.5 * m2;  // psi = s2 / m^2 < 1.5
+    double aq = 0.0, bp2 = 0.0, sm = 0.0, arg = 0.0;
     if (quad) {
-        bp2 = 2.0 / psi - 1.0 + ::sqrt(2.0 / psi * (2.0 / psi - 1.0));
-        const double b = ::sqrt(bp2);
-        aq = m / (1.0 + bp2);
-        const double zv = normal_f64(wv);
-        V = aq * (b + zv) * (b + zv);
+        const double tt = div_f64(m2 + m2, s2);  // 2 / psi
+        const double tm1 = tt - 1.0;
+        bp2 = tm1 + sqrt_f64(tt * tm1);
+        aq = div_f64(m, 1.0 + bp2);
+        const double bz = sqrt_f64(bp2) + zv;
+        V = aq * bz * bz;
     } else {
-        p = (psi - 1.0) / (psi + 1.0);
-        beta = 2.0 / (m * (psi + 1.0));
-        const double u = uniform_f64(wv);
-        V = p < u ? ::log((1.0 - p) / (1.0 - u)) / beta : 0.0;
+        // p = (psi - 1)/(psi + 1), beta = 2/(m (psi + 1)): with sm = s2 + m^2, 1 - p = 2 m^2/sm and
+        // 1/beta = sm/(2 m). U > p exactly when arg = (1 - p)/(1 - U) > 1; 1 - U comes from ~k
+        sm = s2 + m2;
+        arg = div_f64(m2 + m2, sm * uniform_f64(~wv));
+        const double v = log_f64(arg) * div_f64(sm, m + m);
+        V = arg > 1.0 ? v : 0.0;
     }
-    double k0 = -rho * kappa * theta / eps * delta + R.r_drift * delta;
-    const double k1 = 0.5 * delta * (kappa * rho / eps - 0.5) - rho / eps;
-    const double k2 = 0.5 * delta * (kappa * rho / eps - 0.5) + rho / eps;
-    const double k3 = 0.5 * delta * (1.0 - rho * rho);
-    const double k4 = 0.5 * delta * (1.0 - rho * rho);
+    double k0 = c.k0;
     if (R.flags & kMartingale) {
         // Andersen's martingale-corrected K0* = -ln E[exp(A V') | V] - (K1 + K3/2) V, A = K2 + K4/2
-        const double A = k2 + 0.5 * k4;
+        const double A = c.k2 + 0.5 * c.k3;
+        const double beta = (m + m) / sm;
         if (quad && 2.0 * A * aq < 1.0) {
             const double lnM = A * bp2 * aq / (1.0 - 2.0 * A * aq) - 0.5 * ::log1p(-2.0 * A * aq);
-            k0 = -lnM - (k1 + 0.5 * k3) * Vp + R.r_drift * delta;
+            k0 = -lnM - (c.k1 + 0.5 * c.k3) * Vp + R.r_drift * c.delta;
         } else if (!quad && A < beta) {
-            const double lnM = ::log(p + beta * (1.0 - p) / (beta - A));
-            k0 = -lnM - (k1 + 0.5 * k3) * Vp + R.r_drift * delta;
+            const double omp = (m2 + m2) / sm;  // 1 - p
+            const double lnM = ::log((1.0 - omp) + beta * omp / (beta - A));
+            k0 = -lnM - (c.k1 + 0.5 * c.k3) * Vp + R.r_drift * c.delta;
         }
     }
-    logX = logX + k0 + k1 * Vp + k2 * V + ::sqrt(k3 * Vp + k4 * V) * normal_f64(wx);
+    // V = V' = 0 makes the diffusion's variance 0: the floor keeps the root finite and moves nothing
+    const double var = __builtin_fmax(__builtin_fma(c.k3, Vp, c.k3 * V), 1e-300);
+    logX = __builtin_fma(sqrt_f64(var), zx, logX + k0 + c.k1 * Vp + c.k2 * V);
     return quad;
 }
 
-__device__ __forceinline__ bool central_f64(uint32_t k) { return __builtin_fabs(uniform_f64(k) - 0.5) <= 0.425; }
+__device__ __forceinline__ bool central_f64(uint32_t k) { return !is_tail_f64(centred_f64(k)); }
+
+// The normals of a counter block's four words. The central rational runs on every lane; the tail
+// (a logarithm, a root and another rational, 15% of the words, so that nearly every wave has a lane
+// in it for every word) runs once for all four words: their tail words are queued in LDS, 38 of
+// the 256 on average, and each lane takes one (`queue`: this wave's 256 slots of 8 bytes).
+__device__ __forceinline__ void normals4_f64(const u32x4& w, double (&z)[4], double* queue, int lane) {
+    const uint32_t k[4] = {w.x, w.y, w.z, w.w};
+    double q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = centred_f64(k[i]);
+    uint32_t* words = reinterpret_cast<uint32_t*>(queue);  // a slot's first half: the folded word
+    uint32_t pos[4], n = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool t = is_tail_f64(q[i]);
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(t);
+        pos[i] = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, n));
+        if (t) words[2 * pos[i]] = k[i] ^ (uint32_t)((int32_t)k[i] >> 31);
+        n += (uint32_t)__builtin_popcountll(mask);
+    }
+    normal_central_f64<4>(q, z);
+    wave_sync_lds();
+    for (uint32_t b = 0; b < n; b += kTile) {  // wave-uniform
+        const uint32_t t = b + (uint32_t)lane;
+        if (t < n) queue[t] = normal_tail_f64(words[2 * t]);
+    }
+    wave_sync_lds();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (is_tail_f64(q[i])) z[i] = __builtin_copysign(queue[pos[i]], q[i]);
+    wave_sync_lds();  // the slots are rewritten by the next block, or by the values of an expiry
+}
+
+// e^y; the fast form covers every price within e^+-700, the library's the rest.
+__device__ __forceinline__ double price_exp_f64(double y) {
+    double x = exp_f64(y);
+    const bool out = !(__builtin_fabs(y) < 700.0);
+    if (__builtin_amdgcn_ballot_w64(out)) x = out ? ::exp(y) : x;
+    return x;
+}
 
 template <bool DEBUG, bool COUNT>
 __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32_t tile, int lane, double4* vals) {
@@ -758,40 +810,40 @@ __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32
     const uint64_t gp = R.path_offset + pl;
     const uint32_t plo = (uint32_t)gp, phi = uniform((uint32_t)((R.path_offset + (uint64_t)tile * kTile) >> 32));
     double V = R.v0, logX = R.log_S0, X = R.S0, Xp = R.S0, acc = 0.0;
-    uint32_t wb0 = 0, wb1 = 0, k = 0;
+    double z[4] = {};  // the counter block's normals: Z_V, Z_X of its two steps
+    u32x4 w{};
+    uint32_t k = 0;
     uint32_t cq = 0, ce = 0, cc = 0, ct = 0;
     for (uint32_t s = 0; s < R.n_segs; ++s) {
         const DevSeg& S = a.segs[R.seg_begin + s];
-        const double delta = S.delta;
+        const SegD c{S.e, S.s2v, S.s2c, S.dk0, S.dk1, S.dk2, S.dk3, S.delta};
         const uint32_t n = S.n_steps;
         for (uint32_t i = 0; i < n; ++i, ++k) {
-            uint32_t wv, wx;
             if ((k & 1u) == 0u) {
-                const u32x4 w = philox4x32_10(k >> 1, plo, phi, 0u, R.seed_lo, R.seed_hi);
-                wv = w.x;
-                wx = w.y;
-                wb0 = w.z;
-                wb1 = w.w;
+                w = philox4x32_10(k >> 1, plo, phi, 0u, R.seed_lo, R.seed_hi);
+                normals4_f64(w, z, reinterpret_cast<double*>(vals), lane);
             } else {
-                wv = wb0;
-                wx = wb1;
+                w.x = w.z;
+                w.y = w.w;
+                z[0] = z[2];
+                z[1] = z[3];
             }
             yp = logX - R.log_S0;
-            const bool quad = qe_step_fp64(R, delta, V, logX, wv, wx);
+            const bool quad = qe_step_fp64(R, c, V, logX, w.x, z[0], z[1]);
             Xp = X;
-            X = ::exp(logX);
+            X = price_exp_f64(logX);
             if constexpr (COUNT) {
                 if (valid) {
                     cq += quad ? 1u : 0u;
                     ce += quad ? 0u : 1u;
-                    const bool cv = central_f64(wv), cx = central_f64(wx);
+                    const bool cv = central_f64(w.x), cx = central_f64(w.y);
                     cc += (quad && cv ? 1u : 0u) + (cx ? 1u : 0u);
                     ct += (quad && !cv ? 1u : 0u) + (cx ? 0u : 1u);
                 }
             }
             if (i + 1u < n) {
-                acc += delta * 0.5 * (X + Xp);  // AAsianCallNonAdaptive::accumulate_value
-                if (geo) accY += delta * 0.5 * ((logX - R.log_S0) + yp);
+                acc += c.delta * 0.5 * (X + Xp);  // AAsianCallNonAdaptive::accumulate_value
+                if (geo) accY += c.delta * 0.5 * ((logX - R.log_S0) + yp);
             }
         }
         for (uint32_t f = 0; f < S.fin_count; ++f) {

@@ -56,6 +56,10 @@ struct DevSeg {
     uint32_t fin_begin, fin_count;
     double delta;  // FP64 kernel: step width
     double dnext;  // FP64 kernel: dt after the finalisations
+    // FP64 kernel: the step's constants as the reference writes them (src/HSimulation.tpp:58-60,
+    // :75-80): e = e^-kappa dt, m = theta + (V - theta) e, s2 = V s2v + s2c, K0 (with the drift
+    // extension), K1, K2, K3 = K4
+    double e, s2v, s2c, dk0, dk1, dk2, dk3;
 };
 
 // Finalisation of one expiry (AAsianCallNonAdaptive / EuropeanCallNonAdaptive

@@ -406,3 +406,34 @@ def test_fp32_over_a_wide_parameter_box(ctx):
         worst = max(worst, float(err.max()))
     say(f"  worst |FP32 - FP64| in units of (1e-4 price + 1e-5 S0): {worst:.3f}; {overflow} beyond the FP32 range")
     assert worst <= 1.0
+
+
+def test_fp64_normals_at_the_region_switch(ctx, oracle):
+    """FP64 normals at the words around |u - 1/2| = 0.425 and at both ends: the central rational and
+    the tail meet within the oracle's own rounding (2e-15 relative, as over random words)."""
+    edge = [int(f * 2**32) + d for f in (0.075, 0.925) for d in range(-3, 4)]
+    w = np.array(edge + [0, 1, 2, 2**31 - 1, 2**31, 2**32 - 2, 2**32 - 1], np.uint32)
+    np.testing.assert_allclose(ctx.normals(w, H.FP64), oracle.normals_f64(w), rtol=2e-15, atol=1e-15)
+
+
+FP64_EDGE = {
+    # V = V' = 0 on consecutive steps (nearly all exponential-branch steps): a zero diffusion variance
+    "zero_variance": dict(v0=0.0, theta=1e-3, rho=-0.5, kappa=0.3, sigma=1.5, S0=100.0, steps=40, n_paths=300),
+    # e^(log X) beyond the fast exponential's range, both ends
+    "huge_spot": dict(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=1e305, steps=9, n_paths=130),
+    "tiny_spot": dict(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=1e-305, steps=9, n_paths=130),
+    # one path, and an odd last step whose counter block is half used
+    "one_path": dict(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, steps=1, n_paths=1),
+}
+
+
+@pytest.mark.parametrize("name", sorted(FP64_EDGE))
+def test_pathwise_fp64_edges(ctx, oracle, name):
+    """The FP64 path against the oracle at the edges of its special functions: 1e-12 relative, or
+    twice the spread of two valid FP64 evaluations (as test_pathwise_fp64)."""
+    req = H.Request(**FP64_EDGE[name], expiries=[0.5], strikes=[[FP64_EDGE[name]["S0"]]], seed=13, precision=H.FP64)
+    g = ctx.paths(req, 0, req.n_paths)
+    o = oracle_for(oracle, req)["finals"]
+    o_fma = oracle_for(oracle, req, kind="fma")["finals"]
+    tol = max(1e-12, 2.0 * (np.abs(o_fma - o) / np.abs(o)).max())
+    assert (np.abs(g - o) / np.abs(o)).max() < tol
