@@ -74,7 +74,7 @@ struct hexo_server_state {
 
     void run();
     void complete_ready();
-    void launch_ready();
+    void launch_ready(std::unique_lock<std::mutex>& lk);  // lk holds mu; released while a batch is built
 };
 
 namespace {
@@ -123,7 +123,7 @@ void hexo_server_state::complete_ready() {
     }
 }
 
-void hexo_server_state::launch_ready() {
+void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
     for (;;) {
         if (queue.empty()) return;
         int slot = -1;
@@ -179,6 +179,14 @@ void hexo_server_state::launch_ready() {
             cv.notify_all();
             continue;
         }
+        // The batch is built and launched without the lock (40 to 70 us of planning, packing and
+        // launch calls), so that requests keep arriving meanwhile and the next batch takes them
+        // together: with the lock held every submission waited for a launch and short requests ran
+        // one or two to a batch (bursts of 2 to 48 requests of 1e3 to 4e5 paths took 1.0 to 1.7 times
+        // as long). The taken tickets are past cancelling, and only this thread touches the flights.
+        const bool fail_launch = inject_launch != 0;
+        for (uint64_t id : ids) tickets[id]->state = 1;
+        lk.unlock();
         std::unique_ptr<hexo::Batch> b;
         std::string err;
         hexo_tuning tun = ctx->tuning_now();
@@ -191,27 +199,33 @@ void hexo_server_state::launch_ready() {
         int rc = hexo::batch_create(ctx, reqs.data(), (uint32_t)reqs.size(), streams[slot], mem, b, err, nullptr, &tun);
         if (rc == HEXO_ERR_NOMEM && !flights.empty()) {
             // fragmentation: put the requests back in arrival order and retry when a batch completes
-            for (uint64_t id : ids) queue.push_back(id);
+            lk.lock();
+            for (uint64_t id : ids) {
+                tickets[id]->state = 0;
+                queue.push_back(id);
+            }
             std::sort(queue.begin(), queue.end());  // ticket ids grow with arrival
             return;
         }
-        if (rc == HEXO_OK && inject_launch) {
-            --inject_launch;
-            rc = HEXO_ERR_INJECTED;
-        }
+        const bool injected = rc == HEXO_OK && fail_launch;
+        if (injected) rc = HEXO_ERR_INJECTED;
         hipEvent_t ev = nullptr;
         if (rc == HEXO_OK) rc = hexo::batch_enqueue(*b, hexo::PathMode::Normal, false, nullptr, err);
         if (rc == HEXO_OK && (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||
                               hipEventRecord(ev, streams[slot]) != hipSuccess))
             rc = HEXO_ERR_HIP;
         const double t_launch = hexo::now_s();
-        ++batch_counter;
         if (rc != HEXO_OK) {
             if (b) {
                 (void)hipStreamSynchronize(streams[slot]);
                 hexo::batch_destroy(*b);
             }
             if (ev) (void)hipEventDestroy(ev);
+        }
+        lk.lock();
+        ++batch_counter;
+        if (rc != HEXO_OK) {
+            if (injected && inject_launch) --inject_launch;
             worker_error = err;
             for (uint64_t id : ids) fail_ticket(*tickets[id], rc);
             cv.notify_all();
@@ -219,7 +233,6 @@ void hexo_server_state::launch_ready() {
         }
         for (uint64_t id : ids) {
             Ticket& t = *tickets[id];
-            t.state = 1;
             t.info.admit_s = t_admit;
             t.info.launch_s = t_launch;
             t.info.batch_id = batch_counter;
@@ -246,7 +259,7 @@ void hexo_server_state::run() {
     std::unique_lock<std::mutex> lk(mu);
     for (;;) {
         complete_ready();
-        if (!stopping || !queue.empty()) launch_ready();
+        if (!stopping || !queue.empty()) launch_ready(lk);
         if (stopping && queue.empty() && flights.empty()) break;
         if (!flights.empty())
             cv.wait_for(lk, std::chrono::microseconds(50));
