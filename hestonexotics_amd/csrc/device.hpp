@@ -193,14 +193,8 @@ __device__ __forceinline__ NormalVregs normal_vregs() {
     return NormalVregs{in_vgpr(NormalF32::c[8]), in_vgpr(0x1p-33f), in_vgpr_u32(0x80000000u)};
 }
 
-// The FP32 normal of word k. `tail` reports l < lc; the tail polynomial is evaluated only where
-// `need` is also set (a caller that does not use the value passes false: it then holds the central
-// polynomial's value, meaningless in the tail).
-__device__ __forceinline__ float normal_word_f32(uint32_t k, bool need, const NormalVregs& nv, bool& tail) {
-    const uint32_t j = k ^ (uint32_t)((int32_t)k >> 31);
-    const float s = __builtin_fmaf((float)j, 0x1p-32f, nv.h33);
-    const float t = __builtin_fmaf(-s, s, s);
-    const float l = __builtin_amdgcn_logf(t);
+// h(l) where l >= lc, and where l < lc.
+__device__ __forceinline__ float normal_central_f32(float l, const NormalVregs& nv) {
     // Horner steps the compiler forms as v_fmamk_f32 / v_fmaak_f32 with the coefficient as the
     // instruction's literal (no scalar-register operand)
     float h = __builtin_fmaf(l, NormalF32::c[9], nv.c8);
@@ -212,21 +206,59 @@ __device__ __forceinline__ float normal_word_f32(uint32_t k, bool need, const No
     h = __builtin_fmaf(h, l, NormalF32::c[2]);
     h = __builtin_fmaf(h, l, NormalF32::c[1]);
     h = __builtin_fmaf(h, l, NormalF32::c[0]);
+    return h;
+}
+__device__ __forceinline__ float normal_tail_f32(float l) {
+    const float y = __builtin_amdgcn_sqrtf(-l) - NormalF32::yc;
+    float g = __builtin_fmaf(y, NormalF32::d[8], NormalF32::d[7]);
+    g = __builtin_fmaf(g, y, NormalF32::d[6]);
+    g = __builtin_fmaf(g, y, NormalF32::d[5]);
+    g = __builtin_fmaf(g, y, NormalF32::d[4]);
+    g = __builtin_fmaf(g, y, NormalF32::d[3]);
+    g = __builtin_fmaf(g, y, NormalF32::d[2]);
+    g = __builtin_fmaf(g, y, NormalF32::d[1]);
+    return __builtin_fmaf(g, y, NormalF32::d[0]);
+}
+
+// The FP32 normal of word k. `tail` reports l < lc; the tail polynomial is evaluated only where
+// `need` is also set (a caller that does not use the value passes false: it then holds the central
+// polynomial's value, meaningless in the tail).
+__device__ __forceinline__ float normal_word_f32(uint32_t k, bool need, const NormalVregs& nv, bool& tail) {
+    const uint32_t j = k ^ (uint32_t)((int32_t)k >> 31);
+    const float s = __builtin_fmaf((float)j, 0x1p-32f, nv.h33);
+    const float t = __builtin_fmaf(-s, s, s);
+    const float l = __builtin_amdgcn_logf(t);
+    float h = normal_central_f32(l, nv);
     tail = l < NormalF32::lc;
-    if (need && tail) {
-        const float y = __builtin_amdgcn_sqrtf(-l) - NormalF32::yc;
-        float g = __builtin_fmaf(y, NormalF32::d[8], NormalF32::d[7]);
-        g = __builtin_fmaf(g, y, NormalF32::d[6]);
-        g = __builtin_fmaf(g, y, NormalF32::d[5]);
-        g = __builtin_fmaf(g, y, NormalF32::d[4]);
-        g = __builtin_fmaf(g, y, NormalF32::d[3]);
-        g = __builtin_fmaf(g, y, NormalF32::d[2]);
-        g = __builtin_fmaf(g, y, NormalF32::d[1]);
-        h = __builtin_fmaf(g, y, NormalF32::d[0]);
-    }
+    if (need && tail) h = normal_tail_f32(l);
     const float pr = h * __builtin_fmaf(-2.0f, s, 1.0f);  // |z| = h (1 - 2s)
     // negative for k < 2^31 (u < 1/2)
     return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pr) ^ (~k & nv.sign));
+}
+// The normals of N words, each as normal_word_f32 gives it: the central polynomials side by side and
+// one test for a tail among the N (in all lanes) instead of N.
+template <int N>
+__device__ __forceinline__ void normals_f32(const uint32_t (&k)[N], float (&z)[N], const NormalVregs& nv) {
+    float s[N], l[N], h[N];
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t j = k[i] ^ (uint32_t)((int32_t)k[i] >> 31);
+        s[i] = __builtin_fmaf((float)j, 0x1p-32f, nv.h33);
+        l[i] = __builtin_amdgcn_logf(__builtin_fmaf(-s[i], s[i], s[i]));
+        h[i] = normal_central_f32(l[i], nv);
+        any |= l[i] < NormalF32::lc;
+    }
+    if (__builtin_amdgcn_ballot_w64(any)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (l[i] < NormalF32::lc) h[i] = normal_tail_f32(l[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float pr = h[i] * __builtin_fmaf(-2.0f, s[i], 1.0f);
+        z[i] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pr) ^ (~k[i] & nv.sign));
+    }
 }
 __device__ __forceinline__ float normal_f32(uint32_t k) {
     bool tail;

@@ -277,6 +277,28 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
     return L;
 }
 
+// Drawing waves per tile of the split kernel for a class of `tiles` 64-path tiles, or 0 for the
+// persistent kernel. FP32 only, and where the launch shape is left to the library (2 paths per
+// thread, no occupancy cap).
+//  * up to 512 tiles (half the SIMDs): two drawing waves; the tile's time is the stepping wave's
+//    (1e4 paths x 126 steps 28.5 -> 20.4 us against one). Beyond, the third wave competes with
+//    other tiles' stepping waves: 5% faster still for quadratic-branch steps at 1,500 tiles, 15%
+//    slower where the stepping wave is the longer one (martingale correction, exponential branch).
+//  * up to 2^17 tiles (1e6 paths for each of the grid workload's 8 maturities): one drawing wave.
+//    At 125,000 tiles the grid takes 1.72 ms against the persistent kernel's 1.80 and 64 uneven
+//    requests 8.6 to 8.8 ms against 8.7; at 370,000 tiles they take 25.8 ms against 25.3: there the
+//    persistent kernel's waves are full and it has no draws to carry through LDS.
+//  * up to 2,048 tiles where the stepping wave is much the longer one, leaving the drawing waves idle:
+//    the martingale correction on a variance that is mostly in the exponential branch
+//    (2 kappa theta / sigma^2 < 0.6). 1,563 tiles x 1,024 steps 0.605 ms against 0.734, 4,096 tiles
+//    1.25 against 1.07; 15,625 tiles x 512 steps at ratios 0.05 to 0.44 1.86-1.90 against 1.73-1.77,
+//    at 0.79 1.38 against 1.52.
+uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, bool long_steps, const hexo_tuning& tun) {
+    if (cls == 0 || tun.paths_per_thread != 2 || tun.waves_per_simd != 0) return 0;
+    if (tiles > (long_steps ? 2048u : 1u << 17)) return 0;
+    return tiles <= 512 ? 2 : 1;
+}
+
 bool plan_request(const hexo_request* r, ReqPlan& p) {
     if (!build_schedule(r->expiries, r->n_expiries, r->n_strikes, r->steps, p.segs, p.total_steps)) return false;
     p.n_opts = n_opts_of(r);
@@ -343,18 +365,12 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         return HEXO_ERR_INVALID;
     }
     const hexo_tuning tun = tuning ? *tuning : ctx->tuning_now();
-    // tiles per work item of each kernel class: 1 for the FP64 kernel, the FP32 kernels' paths per
-    // thread; a wave stores one partial per item and output (layout.hpp, kChunkTiles), or one per
-    // tile when its tiles do not divide a chunk (3 paths per thread)
-    uint32_t cls_ppt[kPathClasses], cls_store[kPathClasses];
-    for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
-        cls_ppt[cls] = cls == 0 ? 1u : tun.paths_per_thread;
-        cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;
-    }
     std::vector<ReqPlan> plans(n);
     uint64_t n_seg = 0, n_fin = 0, n_opt = 0, n_partials = 0, n_groups = 0, n_out = 0;
     uint64_t n_geo_items = 0, n_geo_pts = 0, n_geo_waves = 0;
     uint32_t n_cls[kPathClasses] = {};
+    uint64_t cls_tiles[kPathClasses] = {};
+    bool cls_long[kPathClasses] = {};  // a request with long steps (split_draw_waves)
     for (uint32_t i = 0; i < n; ++i) {
         std::string why = validate(&reqs[i]);
         if (!why.empty()) {
@@ -376,17 +392,33 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         n_seg += p.segs.size();
         n_fin += p.n_fins;
         n_opt += p.n_opts;
-        n_partials += (uint64_t)((p.n_tiles + cls_store[p.cls] - 1) / cls_store[p.cls]) * p.n_out;
         n_groups += (uint64_t)p.n_groups * p.n_out;
         n_out += p.n_out;
         n_cls[p.cls]++;
+        cls_tiles[p.cls] += p.n_tiles;
+        cls_long[p.cls] |= (reqs[i].flags & HEXO_MARTINGALE) &&
+                           2.0 * reqs[i].kappa * reqs[i].theta < 0.6 * reqs[i].sigma * reqs[i].sigma;
     }
+    // Per kernel class: the split kernel's drawing waves (0: the persistent kernel) and the tiles per
+    // work item (1, or the persistent FP32 kernels' paths per thread). A wave stores one partial per item and output (layout.hpp,
+    // kChunkTiles), or one per tile when its tiles do not divide a chunk (3 paths per thread).
+    uint32_t cls_ppt[kPathClasses], cls_store[kPathClasses];
+    uint32_t cls_draw[kPathClasses];
+    for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
+        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_long[cls], tun);
+        cls_ppt[cls] = cls == 0 || cls_draw[cls] ? 1u : tun.paths_per_thread;
+        cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;
+    }
+    for (const ReqPlan& p : plans) n_partials += (uint64_t)((p.n_tiles + cls_store[p.cls] - 1) / cls_store[p.cls]) * p.n_out;
     auto b = std::make_unique<Batch>();
     b->ctx = ctx;
     b->stream = stream;
     b->n_req = n;
     b->n_out_total = n_out;
-    for (uint32_t cls = 0; cls < kPathClasses; ++cls) b->ppt[cls] = cls_ppt[cls];
+    for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
+        b->ppt[cls] = cls_ppt[cls];
+        b->draw_waves[cls] = cls_draw[cls];
+    }
     const uint64_t n_finals = finals_n ? *finals_n : 0;
     const Layout L =
         make_layout(n, n_seg, n_fin, n_opt, n_cls, n_partials, n_groups, n_out, n_finals, n_geo_items, n_geo_pts,
@@ -476,6 +508,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         d.n_exp = q.n_expiries;
         d.n_groups = p.n_groups;
         d.v0_f = (float)q.v0;
+        d.n_steps = (uint32_t)p.total_steps;
         d.store_tiles = cls_store[p.cls];
         // options (chain-major) with their expiry's discount factor
         uint64_t oo = 0;
@@ -755,7 +788,10 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
 }
 
 static int enqueue_body(Batch& b, PathMode mode, bool timed, double* d_finals, std::string& err) {
-    HIP_TRY(launch_fill_u32(b.d_counters, kPathClasses, 0u, b.stream));
+    bool queues = false;  // a class runs the persistent kernel, which takes its work from a counter
+    for (uint32_t cls = 0; cls < kPathClasses; ++cls)
+        queues |= b.has_class[cls] && !(b.draw_waves[cls] && mode == PathMode::Normal);
+    if (queues) HIP_TRY(launch_fill_u32(b.d_counters, kPathClasses, 0u, b.stream));
     if (mode == PathMode::Count) HIP_TRY(launch_zero_u64(b.d_counts, 4, b.stream));
     if (timed) HIP_TRY(hipEventRecord(b.ev[0], b.stream));
     for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
@@ -763,8 +799,11 @@ static int enqueue_body(Batch& b, PathMode mode, bool timed, double* d_finals, s
         PathArgs a = b.pa[cls];
         a.finals = d_finals;
         a.counts = mode == PathMode::Count ? b.d_counts : nullptr;
-        HIP_TRY(launch_paths(class_precision(cls), b.ppt[cls], mode, b.grid[cls], b.block[cls], b.stream, a,
-                             class_martingale(cls), class_geo(cls)));
+        if (b.draw_waves[cls] && mode == PathMode::Normal)
+            HIP_TRY(launch_paths_split(b.draw_waves[cls], a, class_martingale(cls), class_geo(cls), b.stream));
+        else
+            HIP_TRY(launch_paths(class_precision(cls), b.ppt[cls], mode, b.grid[cls], b.block[cls], b.stream, a,
+                                 class_martingale(cls), class_geo(cls)));
         ++b.path_launches;
     }
     if (timed) HIP_TRY(hipEventRecord(b.ev[1], b.stream));

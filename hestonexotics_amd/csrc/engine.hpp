@@ -128,6 +128,7 @@ struct Batch {
     PathArgs pa[kPathClasses]{};
     uint32_t grid[kPathClasses]{}, block[kPathClasses]{}, ppt[kPathClasses]{};
     bool has_class[kPathClasses]{};
+    uint32_t draw_waves[kPathClasses]{};  // of the split kernel (Normal mode); 0: the persistent kernel
     ReduceArgs ra{};
     GeoArgs ga{};  // exact geometric prices, computed once after the upload (n_items 0: none)
     uint64_t n_group_threads = 0, n_out_threads = 0;

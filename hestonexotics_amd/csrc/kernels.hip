@@ -5,6 +5,8 @@
 //              and scheme (src/HSimulation.tpp:23-49, :52-86), the option policies
 //              (src/inc/AsianContract.h:25-47, src/inc/VanillaContract.h:24-39) and the RNG ring
 //              refills (src/RNG.cpp:28-43, src/as241.f90:85-118).
+// k_path_fp32_split  the same paths with the draws and the steps on different waves, for batches
+//              that leave k_path_fp32's persistent grid short of work.
 // k_path_fp64  the plain FP64 kernel: the same path in the reference's own FP64 form.
 // k_reduce_*   cross-tile reduction in a fixed order and the estimator (price, standard error);
 //              replaces the racy `prices[...] +=` of src/HSimulation.tpp:40,47-48.
@@ -372,66 +374,95 @@ __device__ __forceinline__ void qe_moments_fp32(const float (&V)[PPT], const Seg
 // a (b + Z_V)^2 or the exponential branch, then the log-price step (MART: Andersen's
 // martingale-corrected form, falling back per path and step to the plain step where
 // E[exp(A V')] does not exist; GEO: also Y before the step and the run's sum of Y).
-template <int PPT, bool MART, bool GEO>
+//
+// FLAT evaluates the quadratic branch on every lane and enters one branch per step, for the lanes in
+// the exponential one, instead of two per path. The stepping waves of the split kernel run it (1e6
+// stiff paths with the martingale correction x 512 steps: 1.80 ms against 2.05); at the persistent
+// kernel's issue limit it costs 2% (64 uneven requests 5.18 ms against 5.07).
+template <bool FLAT, int PPT, bool MART, bool GEO>
 __device__ __forceinline__ void qe_update_fp32(float (&V)[PPT], float (&Y)[PPT], float (&X)[PPT], float (&Xp)[PPT],
                                                float (&P)[PPT], float (&Yp)[PPT], float (&PY)[PPT],
                                                const uint32_t (&wv)[PPT], const float (&zv)[PPT],
                                                const float (&zx)[PPT], const float (&d0)[PPT], const float (&m)[PPT],
                                                const float (&s2h)[PPT], const float (&m2)[PPT], const float (&tt)[PPT],
                                                const bool (&quad)[PPT], const SegF& c) {
+    // One path's draw: dm = V' - m and, MART: A m - ln E[exp(A V')] = fs f(ft) + corr with
+    // f(t) = t - ln(1 + t), in natural log units; mok: the expectation exists
+    struct Draw {
+        float dm, ft = 0.0f, fs = 0.0f, corr = 0.0f;
+        bool mok = false;
+    };
+    auto quadratic = [&](int j, Draw& o) __attribute__((always_inline)) {
+        const float tm1 = tt[j] - 1.0f;
+        const float b2 = tm1 + __builtin_amdgcn_sqrtf(tt[j] * tm1);
+        const float b = __builtin_amdgcn_sqrtf(b2);
+        // V' = a (b + Z)^2 with a = m / (1 + b^2), taken as V' - m = a (Z (Z + 2 b) - 1): its
+        // mean is 0 whatever the rounding of a and b, so the scheme's E[V'] = m holds exactly
+        // (a biased mean would move the variance's mean-reversion level by (bias) / (kappa dt))
+        const float aq = m[j] * __builtin_amdgcn_rcpf(__builtin_fmaf(b, b, 1.0f));
+        // near b + Z = 0, m + (V' - m) can round a few ulp of m below 0 where a (b + Z)^2 is
+        // >= 0: harmless to the moments, and the diffusion below takes |k3 (V + V')|
+        o.dm = aq * __builtin_fmaf(zv[j], __builtin_fmaf(2.0f, b, zv[j]), -1.0f);
+        if constexpr (MART) {
+            // x = 2 A a < 1: A m - ln E[exp(A V')] = -(f(-x) + x^2 b^2 / (1 - x)) / 2
+            const float x = (c.mA + c.mA) * aq;
+            o.mok = x < 1.0f;
+            o.ft = -x;
+            o.fs = -0.5f;
+            o.corr = -0.5f * (x * x) * b2 * __builtin_amdgcn_rcpf(1.0f - x);
+        }
+    };
+    auto exponential = [&](int j, Draw& o) __attribute__((always_inline)) {
+        // p = (psi-1)/(psi+1), beta = 2/(m (psi+1)); V' = ln((1-p)/(1-U))/beta if U > p, else 0.
+        // With sm = s2 + m^2: 1-p = 2m^2/sm and 1/beta = sm/(2m).
+        const float sm = __builtin_fmaf(2.0f, s2h[j], m2[j]);
+        // (1-U) sm, 1 - U from ~k; the complement is taken here (asm: not hoisted in front of the
+        // branch, where every lane would pay for it; the wait state as at the asm helpers in
+        // device.hpp)
+        uint32_t nk;
+        asm("s_nop 0\n\tv_not_b32 %0, %1" : "=v"(nk) : "v"(wv[j]));
+        const float lhs = uniform_f32(nk) * sm;
+        const float tm2 = m2[j] + m2[j];
+        const float lg = __builtin_amdgcn_logf(tm2 * rcp_refined(lhs));
+        const float ib = sm * rcp_refined(m[j]);  // 2 / beta
+        const float v = ib * (0.5f * 0.693147180559945309f) * lg;
+        // U > p exactly when (1-p)/(1-U) > 1, i.e. when the log is positive: V' = max(v, 0)
+        o.dm = __builtin_fmaxf(v, 0.0f) - m[j];
+        if constexpr (MART) {
+            // cA = A / beta < 1, r1 = (1-p) / (1 - cA) = 2 m^2 / (sm (1 - cA)), y = r1 cA:
+            // A m - ln E[exp(A V')] = f(y) - r1 cA^2
+            const float cA = (0.5f * c.mA) * ib;
+            o.mok = cA < 1.0f;
+            const float r1 = tm2 * __builtin_amdgcn_rcpf(__builtin_fmaf(-cA, sm, sm));
+            o.ft = r1 * cA;
+            o.fs = 1.0f;
+            o.corr = -o.ft * cA;
+        }
+    };
+    Draw dr[PPT];
+    if constexpr (FLAT) {
+        bool any_exp = false;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+            quadratic(j, dr[j]);
+            any_exp |= !quad[j];
+        }
+        if (__builtin_amdgcn_ballot_w64(any_exp)) {
+#pragma unroll
+            for (int j = 0; j < PPT; ++j)
+                if (!quad[j]) exponential(j, dr[j]);
+        }
+    }
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-        float dm;  // V' - m
-        // MART: A m - ln E[exp(A V')] = fs f(ft) + corr with f(t) = t - ln(1 + t), in natural
-        // log units; mok: the expectation exists
-        float ft = 0.0f, fs = 0.0f, corr = 0.0f;
-        bool mok = false;
-        if (quad[j]) {
-            const float tm1 = tt[j] - 1.0f;
-            const float b2 = tm1 + __builtin_amdgcn_sqrtf(tt[j] * tm1);
-            const float b = __builtin_amdgcn_sqrtf(b2);
-            // V' = a (b + Z)^2 with a = m / (1 + b^2), taken as V' - m = a (Z (Z + 2 b) - 1): its
-            // mean is 0 whatever the rounding of a and b, so the scheme's E[V'] = m holds exactly
-            // (a biased mean would move the variance's mean-reversion level by (bias) / (kappa dt))
-            const float aq = m[j] * __builtin_amdgcn_rcpf(__builtin_fmaf(b, b, 1.0f));
-            // near b + Z = 0, m + (V' - m) can round a few ulp of m below 0 where a (b + Z)^2 is
-            // >= 0: harmless to the moments, and the diffusion below takes |k3 (V + V')|
-            dm = aq * __builtin_fmaf(zv[j], __builtin_fmaf(2.0f, b, zv[j]), -1.0f);
-            if constexpr (MART) {
-                // x = 2 A a < 1: A m - ln E[exp(A V')] = -(f(-x) + x^2 b^2 / (1 - x)) / 2
-                const float x = (c.mA + c.mA) * aq;
-                mok = x < 1.0f;
-                ft = -x;
-                fs = -0.5f;
-                corr = -0.5f * (x * x) * b2 * __builtin_amdgcn_rcpf(1.0f - x);
-            }
-        } else {
-            // p = (psi-1)/(psi+1), beta = 2/(m (psi+1)); V' = ln((1-p)/(1-U))/beta if U > p, else 0.
-            // With sm = s2 + m^2: 1-p = 2m^2/sm and 1/beta = sm/(2m).
-            const float sm = __builtin_fmaf(2.0f, s2h[j], m2[j]);
-            // (1-U) sm, 1 - U from ~k; the complement is taken here (asm: not hoisted in front of the
-            // branch, where every lane would pay for it; the wait state as at the asm helpers in
-            // device.hpp)
-            uint32_t nk;
-            asm("s_nop 0\n\tv_not_b32 %0, %1" : "=v"(nk) : "v"(wv[j]));
-            const float lhs = uniform_f32(nk) * sm;
-            const float tm2 = m2[j] + m2[j];
-            const float lg = __builtin_amdgcn_logf(tm2 * rcp_refined(lhs));
-            const float ib = sm * rcp_refined(m[j]);  // 2 / beta
-            const float v = ib * (0.5f * 0.693147180559945309f) * lg;
-            // U > p exactly when (1-p)/(1-U) > 1, i.e. when the log is positive: V' = max(v, 0)
-            dm = __builtin_fmaxf(v, 0.0f) - m[j];
-            if constexpr (MART) {
-                // cA = A / beta < 1, r1 = (1-p) / (1 - cA) = 2 m^2 / (sm (1 - cA)), y = r1 cA:
-                // A m - ln E[exp(A V')] = f(y) - r1 cA^2
-                const float cA = (0.5f * c.mA) * ib;
-                mok = cA < 1.0f;
-                const float r1 = tm2 * __builtin_amdgcn_rcpf(__builtin_fmaf(-cA, sm, sm));
-                ft = r1 * cA;
-                fs = 1.0f;
-                corr = -ft * cA;
-            }
+        if constexpr (!FLAT) {
+            if (quad[j])
+                quadratic(j, dr[j]);
+            else
+                exponential(j, dr[j]);
         }
+        const float dm = dr[j].dm, ft = dr[j].ft, fs = dr[j].fs, corr = dr[j].corr;
+        const bool mok = dr[j].mok;
         // The reference's log-price step multiplies V' - V by rho/sigma and V + V' - 2 th by
         // kappa rho dt / (2 sigma). As differences of FP32 variances they would carry ulp(V) errors
         // amplified by 1/sigma (prices tens of percent off at sigma = 1e-6, or at sigma = 1e-4
@@ -500,7 +531,7 @@ __device__ __forceinline__ void qe_step_fp32(float (&V)[PPT], float (&Y)[PPT], f
         zx[j] = normal_word_f32(wx[j], true, nv, tx);
         if constexpr (COUNT) count_step(cnt, valid[j], quad[j], tv, tx);
     }
-    qe_update_fp32<PPT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, wv, zv, zx, d0, m, s2h, m2, tt, quad, c);
+    qe_update_fp32<false, PPT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, wv, zv, zx, d0, m, s2h, m2, tt, quad, c);
 }
 
 // Philox4x32-10 (device.hpp philox4x32_10) of the path counter {blk, plo, phi, 0} with the step
@@ -564,6 +595,78 @@ __device__ __forceinline__ void philox_block(uint32_t blk, const uint32_t (&plo)
     }
 }
 
+// The end of a run of steps: the Asian accumulation of its interior, the expiries finalised there
+// (payoff sums of the wave's tiles through the wave's LDS region) and the accumulation over the
+// first step of the next run.
+template <int PPT, bool DEBUG, bool GEO>
+__device__ __forceinline__ void end_run_fp32(const PathArgs& a, const DevReq& R, const DevSeg& S, uint32_t tile0, int lane,
+                                             uint32_t* lds, const bool (&valid)[PPT], const float (&X)[PPT],
+                                             const float (&Xp)[PPT], float (&P)[PPT], float (&acc)[PPT],
+                                             float (&Xs)[PPT], const float (&Y)[PPT], const float (&Yp)[PPT],
+                                             float (&PY)[PPT], float (&accY)[PPT], float (&Ys)[PPT]) {
+    // Asian accumulation of the run's interior steps b..e-1:
+    // delta * (X_{b-1}/2 + X_b + ... + X_{e-2} + X_{e-1}/2) = delta * (P - X_e + (Xs - Xp)/2)
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+        acc[j] = __builtin_fmaf(S.delta_f, (P[j] - X[j]) + 0.5f * (Xs[j] - Xp[j]), acc[j]);
+        if constexpr (GEO) accY[j] = __builtin_fmaf(S.delta_f, (PY[j] - Y[j]) + 0.5f * (Ys[j] - Yp[j]), accY[j]);
+    }
+    // per-path values at an expiry: (A, X_T), with GEO (A, X_T, G, -); the wave's LDS region
+    // holds 4 words per path either way
+    using Val = typename std::conditional<GEO, float4, float2>::type;
+    Val* vals = reinterpret_cast<Val*>(lds);
+    for (uint32_t f = 0; f < S.fin_count; ++f) {
+        const DevFin& F = a.fins[S.fin_begin + f];
+        const float w = F.w_f, invT = F.invT_f;
+        NanBits nan;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+            const float dX = X[j] - Xp[j];
+            const float xt = __builtin_fmaf(dX, w, Xp[j]);
+            const float A = (R.flags & kTrapezoid) ? (acc[j] + F.hwdt_f * (Xp[j] + xt)) * invT
+                                                   : __builtin_fmaf(dX, w, acc[j]) * invT;
+            // paths beyond n_paths carry -inf: every payoff max(0, . - K) is then 0
+            if constexpr (GEO) {
+                // the same functional on Y, normalised by its weight sum W: G/S0 = W 2^(L/W)
+                const float dY = Y[j] - Yp[j];
+                const float L = (R.flags & kTrapezoid)
+                                    ? (accY[j] + F.hwdt_f * (Yp[j] + __builtin_fmaf(dY, w, Yp[j]))) * invT
+                                    : __builtin_fmaf(dY, w, accY[j]) * invT;
+                const float G = F.gW_f * __builtin_amdgcn_exp2f(L * F.gInvW_f);
+                vals[j * kTile + lane] =
+                    valid[j] ? make_float4(A, xt, G, 0.0f) : make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+                nan.mark(j, valid[j], A, xt, G);
+            } else {
+                vals[j * kTile + lane] = valid[j] ? make_float2(A, xt) : make_float2(-INFINITY, -INFINITY);
+                nan.mark(j, valid[j], A, xt, 0.0f);
+            }
+            if constexpr (DEBUG) {
+                if (valid[j] && a.finals) {
+                    const uint64_t pl = (uint64_t)(tile0 + (uint32_t)j) * kTile + (uint64_t)lane;
+                    double* out = a.finals + (pl * R.n_exp + F.chain) * 2;
+                    out[0] = (double)A * R.S0;
+                    out[1] = (double)xt * R.S0;
+                }
+            }
+        }
+        wave_sync_lds();
+        reduce_tiles<PPT>(a, R, F, tile0, lane, vals, nan);
+        wave_sync_lds();
+    }
+    const float hn = 0.5f * S.dnext_f;
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+        acc[j] = __builtin_fmaf(hn, X[j] + Xp[j], acc[j]);
+        Xs[j] = X[j];
+        P[j] = 0.0f;
+        if constexpr (GEO) {
+            accY[j] = __builtin_fmaf(hn, Y[j] + Yp[j], accY[j]);
+            Ys[j] = Y[j];
+            PY[j] = 0.0f;
+        }
+    }
+}
+
 template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
 __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32_t tile0, int lane, uint32_t* lds) {
     const DevReq& R = a.reqs[ri];
@@ -618,67 +721,7 @@ __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32
             qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w0, w1, c, valid, cnt, nv);
             ++k;
         }
-        // Asian accumulation of the run's interior steps b..e-1:
-        // delta * (X_{b-1}/2 + X_b + ... + X_{e-2} + X_{e-1}/2) = delta * (P - X_e + (Xs - Xp)/2)
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            acc[j] = __builtin_fmaf(S.delta_f, (P[j] - X[j]) + 0.5f * (Xs[j] - Xp[j]), acc[j]);
-            if constexpr (GEO) accY[j] = __builtin_fmaf(S.delta_f, (PY[j] - Y[j]) + 0.5f * (Ys[j] - Yp[j]), accY[j]);
-        }
-        // per-path values at an expiry: (A, X_T), with GEO (A, X_T, G, -); the wave's LDS region
-        // holds 4 words per path either way
-        using Val = typename std::conditional<GEO, float4, float2>::type;
-        Val* vals = reinterpret_cast<Val*>(lds);
-        for (uint32_t f = 0; f < S.fin_count; ++f) {
-            const DevFin& F = a.fins[S.fin_begin + f];
-            const float w = F.w_f, invT = F.invT_f;
-            NanBits nan;
-#pragma unroll
-            for (int j = 0; j < PPT; ++j) {
-                const float dX = X[j] - Xp[j];
-                const float xt = __builtin_fmaf(dX, w, Xp[j]);
-                const float A = (R.flags & kTrapezoid) ? (acc[j] + F.hwdt_f * (Xp[j] + xt)) * invT
-                                                       : __builtin_fmaf(dX, w, acc[j]) * invT;
-                // paths beyond n_paths carry -inf: every payoff max(0, . - K) is then 0
-                if constexpr (GEO) {
-                    // the same functional on Y, normalised by its weight sum W: G/S0 = W 2^(L/W)
-                    const float dY = Y[j] - Yp[j];
-                    const float L = (R.flags & kTrapezoid)
-                                        ? (accY[j] + F.hwdt_f * (Yp[j] + __builtin_fmaf(dY, w, Yp[j]))) * invT
-                                        : __builtin_fmaf(dY, w, accY[j]) * invT;
-                    const float G = F.gW_f * __builtin_amdgcn_exp2f(L * F.gInvW_f);
-                    vals[j * kTile + lane] =
-                        valid[j] ? make_float4(A, xt, G, 0.0f) : make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-                    nan.mark(j, valid[j], A, xt, G);
-                } else {
-                    vals[j * kTile + lane] = valid[j] ? make_float2(A, xt) : make_float2(-INFINITY, -INFINITY);
-                    nan.mark(j, valid[j], A, xt, 0.0f);
-                }
-                if constexpr (DEBUG) {
-                    if (valid[j] && a.finals) {
-                        const uint64_t pl = (uint64_t)(tile0 + (uint32_t)j) * kTile + (uint64_t)lane;
-                        double* out = a.finals + (pl * R.n_exp + F.chain) * 2;
-                        out[0] = (double)A * R.S0;
-                        out[1] = (double)xt * R.S0;
-                    }
-                }
-            }
-            wave_sync_lds();
-            reduce_tiles<PPT>(a, R, F, tile0, lane, vals, nan);
-            wave_sync_lds();
-        }
-        const float hn = 0.5f * S.dnext_f;
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            acc[j] = __builtin_fmaf(hn, X[j] + Xp[j], acc[j]);
-            Xs[j] = X[j];
-            P[j] = 0.0f;
-            if constexpr (GEO) {
-                accY[j] = __builtin_fmaf(hn, Y[j] + Yp[j], accY[j]);
-                Ys[j] = Y[j];
-                PY[j] = 0.0f;
-            }
-        }
+        end_run_fp32<PPT, DEBUG, GEO>(a, R, S, tile0, lane, lds, valid, X, Xp, P, acc, Xs, Y, Yp, PY, accY, Ys);
     }
     if constexpr (COUNT) count_flush(a.counts, cnt.quad, cnt.exp, cnt.central, cnt.tail, lane);
 }
@@ -696,6 +739,127 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 ? 
         const uint32_t first = sp ? a.item_end[sp - 1] : 0u;
         const uint32_t ri = uniform(a.order[sp]);
         path_fp32<PPT, DEBUG, COUNT, MART, GEO>(a, ri, uniform((item - first) * (uint32_t)PPT), lane, lds);
+    }
+}
+// ------------------------------------------------------------------------------------------
+// FP32 path kernel with drawing and stepping waves
+// ------------------------------------------------------------------------------------------
+// One workgroup per 64-path tile. NP waves draw the normals of a chunk of C steps (Philox and the
+// inverse normals, 57 of a step's 100 instructions) into one LDS buffer while the stepping wave
+// runs the variance and log-price recursion over the chunk before it from the other.
+//
+// Why: a wave alone issues one vector instruction in 6.5 to 7.7 cycles however independent they are
+// (1 or 2 paths per lane: 720 and 670 cycles per path-step, 86 instructions), a SIMD needs four or
+// five waves to reach its 3.1; and a request's time axis cannot be split, so a batch of up to
+// 5 waves x 2 tiles per SIMD (650,000 paths) left k_path_fp32 short of waves or of work for its last
+// round. Here a tile is two or three waves, each with its part of the step. Kernel times, k_path_fp32
+// (2 paths per lane) against this one, base parameters x 252 steps: 1e4 paths 144 -> 34 us,
+// 1e5 159 -> 97, 4e5 323 -> 234, 1e6 593 -> 541; martingale step 2e5 paths 245 -> 176 us;
+// the 8 x 64 grid at 1e6 paths 1802 -> 1718 us. The stepping wave's priority is raised: the tile
+// waits for it (400k paths 240 -> 234 us, the grid at a quarter of its paths 501 -> 478).
+// A chunk's draws, step-major: (Z_V, Z_X) and the word of Z_V (the exponential branch's uniform).
+template <uint32_t C>
+struct DrawChunk {
+    float2 z[C][kTile];
+    uint32_t w[C][kTile];
+};
+
+__device__ __forceinline__ void workgroup_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Drawing wave `part` of NP: counter blocks part, part + NP, ... of every chunk. Every wave of the
+// workgroup meets ceil(n_steps / C) barriers: here after each chunk drawn, in the stepping wave
+// before each chunk stepped, so that a buffer is rewritten only after its chunk has been consumed.
+template <uint32_t NP, uint32_t C>
+__device__ __forceinline__ void draw_fp32(const DevReq& R, uint32_t tile, int lane, uint32_t part, DrawChunk<C>* buf) {
+    static_assert(C % (2 * NP) == 0, "whole counter blocks per wave and chunk");
+    const uint64_t first = R.path_offset + (uint64_t)tile * kTile;  // tiles never straddle 2^32
+    const uint32_t plo = (uint32_t)first + (uint32_t)lane, phi = uniform((uint32_t)(first >> 32));
+    const uint32_t key0 = R.seed_lo, key1 = R.seed_hi, n_steps = R.n_steps;
+    const NormalVregs nv = normal_vregs();
+    for (uint32_t k = 0, c = 0; k < n_steps; k += C, ++c) {
+        DrawChunk<C>& d = buf[c & 1u];
+#pragma unroll
+        for (uint32_t b = 0; b < C / 2; b += NP) {
+            const uint32_t t = 2 * (b + part);  // the block's first step; past n_steps the draws are unused
+            const u32x4 r = philox_path((k + t) >> 1, plo, phi, key0, key1);
+            const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+            float z[4];
+            normals_f32<4>(w, z, nv);
+            d.z[t][lane] = make_float2(z[0], z[1]);
+            d.w[t][lane] = w[0];
+            d.z[t + 1][lane] = make_float2(z[2], z[3]);
+            d.w[t + 1][lane] = w[2];
+        }
+        workgroup_sync_lds();
+    }
+}
+
+template <uint32_t C, bool MART, bool GEO>
+__device__ __forceinline__ void step_fp32(const PathArgs& a, const DevReq& R, uint32_t tile, int lane,
+                                          const DrawChunk<C>* buf, uint32_t* lds) {
+    float V[1] = {R.v0_f}, Y[1] = {0.0f}, X[1] = {1.0f}, Xp[1] = {1.0f}, P[1] = {0.0f}, acc[1] = {0.0f}, Xs[1] = {1.0f};
+    float Yp[1] = {0.0f}, PY[1] = {0.0f}, accY[1] = {0.0f}, Ys[1] = {0.0f};
+    const bool valid[1] = {(uint64_t)tile * kTile + (uint64_t)lane < R.n_paths};
+    uint32_t k = 0;
+    for (uint32_t s = 0; s < R.n_segs; ++s) {
+        const DevSeg& S = a.segs[R.seg_begin + s];
+        const SegF c{S.omd, S.th, S.c1h, S.c2h, S.g0, S.ka, S.kb, S.k3, S.mA, S.ma, S.mh, S.mr};
+        auto step = [&](float2 z, uint32_t w) {
+            float d0[1], m[1], s2h[1], m2[1], tt[1];
+            bool quad[1];
+            qe_moments_fp32<1>(V, c, d0, m, s2h, m2, tt, quad);
+            const uint32_t wv[1] = {w};
+            const float zv[1] = {z.x}, zx[1] = {z.y};
+            qe_update_fp32<true, 1, MART, GEO>(V, Y, X, Xp, P, Yp, PY, wv, zv, zx, d0, m, s2h, m2, tt, quad, c);
+        };
+        for (uint32_t left = S.n_steps; left;) {
+            const uint32_t at = k & (C - 1u);
+            if (at == 0) workgroup_sync_lds();
+            const DrawChunk<C>& d = buf[(k / C) & 1u];
+            if (at == 0 && left >= C) {  // a whole chunk: its draws in registers, no loop
+                float2 z[C];
+                uint32_t w[C];
+#pragma unroll
+                for (uint32_t t = 0; t < C; ++t) {
+                    z[t] = d.z[t][lane];
+                    w[t] = d.w[t][lane];
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < C; ++t) step(z[t], w[t]);
+                k += C;
+                left -= C;
+            } else {
+                const uint32_t end = min(C, at + left);
+                for (uint32_t t = at; t < end; ++t) step(d.z[t][lane], d.w[t][lane]);
+                k += end - at;
+                left -= end - at;
+            }
+        }
+        end_run_fp32<1, false, GEO>(a, R, S, tile, lane, lds, valid, X, Xp, P, acc, Xs, Y, Yp, PY, accY, Ys);
+    }
+}
+
+template <uint32_t NP, uint32_t C, bool MART, bool GEO>
+__global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
+    __shared__ DrawChunk<C> buf[2];
+    __shared__ uint32_t vals[WaveLds<1>::kWords];
+    const int lane = (int)(threadIdx.x & 63u);
+    const uint32_t item = blockIdx.x;
+    const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
+    const uint32_t tile = uniform(item - (sp ? a.item_end[sp - 1] : 0u));
+    const DevReq& R = a.reqs[uniform(a.order[sp])];
+    // the stepping wave's place in the workgroup varies with the tile, so that the waves of one role
+    // do not gather on the same SIMDs
+    const uint32_t role = (uniform(threadIdx.x >> 6) + (uint32_t)__builtin_popcount(item * 0x9E3779B1u >> 16)) % (NP + 1);
+    if (role == 0) {
+        __builtin_amdgcn_s_setprio(2);
+        step_fp32<C, MART, GEO>(a, R, tile, lane, buf, vals);
+    } else {
+        draw_fp32<NP, C>(R, tile, lane, role - 1, buf);
     }
 }
 #pragma clang fp contract(fast)
@@ -1153,6 +1317,27 @@ size_t path_lds_bytes(uint32_t precision, uint32_t ppt, uint32_t block) {
     // FP32: per wave the transpose of the per-path values at expiries (4 words per path, WaveLds);
     // FP64: 64 double4 per wave
     return precision == kPrecFP64 ? waves * kTile * sizeof(double4) : waves * 4 * ppt * kTile * sizeof(uint32_t);
+}
+
+hipError_t launch_paths_split(uint32_t n_draw, const PathArgs& a, bool mart, bool geo, hipStream_t st) {
+#define HEXO_SPLIT(NP, C)                                                                    \
+    if (mart && geo)                                                                         \
+        k_path_fp32_split<NP, C, true, true><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);    \
+    else if (mart)                                                                           \
+        k_path_fp32_split<NP, C, true, false><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);   \
+    else if (geo)                                                                            \
+        k_path_fp32_split<NP, C, false, true><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);   \
+    else                                                                                     \
+        k_path_fp32_split<NP, C, false, false><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);
+    if (n_draw == 2) {
+        HEXO_SPLIT(2, 8)
+    } else if (n_draw == 1) {
+        HEXO_SPLIT(1, 4)
+    } else {
+        return hipErrorInvalidValue;
+    }
+#undef HEXO_SPLIT
+    return hipGetLastError();
 }
 
 hipError_t launch_paths(uint32_t precision, uint32_t ppt, PathMode mode, uint32_t grid, uint32_t block,

@@ -92,6 +92,8 @@ struct DevReq {
     uint32_t precision, n_tiles, opt_begin, out_base;
     uint32_t n_exp, n_groups;
     float v0_f;
+    uint32_t n_steps;      // over all runs
+    uint32_t pad;
     uint32_t store_tiles;  // tiles per stored partial: 1, 2 or kChunkTiles (the kernel's paths per thread)
 };
 

@@ -107,7 +107,9 @@ typedef struct hexo_request {
 } hexo_request;
 
 /* Launch shape of the FP32 path kernel. Results do not depend on it: every 64-path tile is
- * reduced on its own and tiles are combined in a fixed order. */
+ * reduced on its own and tiles are combined in a fixed order. With 2 paths per thread and no cap
+ * (the default) the library runs batches too small to fill the GPU on a kernel with more waves per
+ * tile instead; any other shape is used as given. */
 typedef struct hexo_tuning {
     uint32_t paths_per_thread; /* 1, 2, 3 or 4 */
     uint32_t block_threads;    /* 64, 128 or 256 */

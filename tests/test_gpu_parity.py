@@ -437,3 +437,38 @@ def test_pathwise_fp64_edges(ctx, oracle, name):
     o_fma = oracle_for(oracle, req, kind="fma")["finals"]
     tol = max(1e-12, 2.0 * (np.abs(o_fma - o) / np.abs(o)).max())
     assert (np.abs(g - o) / np.abs(o)).max() < tol
+
+
+SPLIT_SIZES = [  # paths, steps, expiries: chunk remainders, odd blocks at expiries, both drawing-wave counts, and
+    # the first size past the split kernel's range
+    (1, 1, [0.5]), (64, 3, [0.5]), (65, 4, [0.5]), (100, 5, [0.3, 0.31, 0.7]), (130, 7, [0.4, 0.9]), (63, 8, [1.0]),
+    (2000, 9, [0.35, 0.7, 1.05]), (512 * 64, 16, [1.0]), (512 * 64 + 1, 17, [0.5, 1.0]), (200_003, 12, [1.0]),
+    (64 << 17, 2, [1.0]), ((64 << 17) + 1, 2, [1.0]),
+]
+
+
+@pytest.mark.parametrize("n_paths,steps,T", SPLIT_SIZES)
+@pytest.mark.parametrize("precision", [H.FP32, H.FP32_COMPENSATED])
+def test_split_kernel_equals_persistent(ctx, n_paths, steps, T, precision):
+    """The kernel with drawing and stepping waves (the library's choice for batches up to 2^17 tiles)
+    gives the persistent kernel's bits (an explicit launch shape), for every FP32 kernel class, payoff
+    reduction and a variance process in either branch."""
+    base = ctx.get_tuning()
+    K = list(np.linspace(80.0, 120.0, 50 if n_paths == 2000 else 3))
+    for model in (dict(rho=-0.7, kappa=2.0, sigma=0.3), dict(rho=-0.9, kappa=0.5, sigma=0.9)):
+        for flags, payoffs in ((0, H.ASIAN), (H.DRIFT | H.DISCOUNT | H.TRAPEZOID, H.ASIAN | H.EUROPEAN),
+                               (H.MARTINGALE, H.ASIAN | H.EUROPEAN), (0, H.ASIAN | H.GEO_ASIAN),
+                               (H.MARTINGALE, H.GEO_ASIAN | H.EUROPEAN)):
+            if payoffs & H.GEO_ASIAN and steps < 3:
+                continue
+            req = H.Request(v0=0.04, theta=0.04, S0=100.0, expiries=T, strikes=[K] * len(T), steps=steps,
+                            n_paths=n_paths, seed=n_paths, r=0.02, flags=flags, payoffs=payoffs,
+                            precision=precision, path_offset=64 * steps, **model)
+            got = ctx.price(req)
+            try:
+                ctx.set_tuning(1, 64, 0)
+                want = ctx.price(req)
+            finally:
+                ctx.set_tuning(**base)
+            np.testing.assert_array_equal(got[0], want[0])
+            np.testing.assert_array_equal(got[1], want[1])
