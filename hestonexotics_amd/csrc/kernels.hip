@@ -439,30 +439,31 @@ __device__ __forceinline__ void qe_update_fp32(float (&V)[PPT], float (&Y)[PPT],
             o.corr = -o.ft * cA;
         }
     };
-    Draw dr[PPT];
+    Draw flat[FLAT ? PPT : 1];
     if constexpr (FLAT) {
         bool any_exp = false;
 #pragma unroll
         for (int j = 0; j < PPT; ++j) {
-            quadratic(j, dr[j]);
+            quadratic(j, flat[j]);
             any_exp |= !quad[j];
         }
         if (__builtin_amdgcn_ballot_w64(any_exp)) {
 #pragma unroll
             for (int j = 0; j < PPT; ++j)
-                if (!quad[j]) exponential(j, dr[j]);
+                if (!quad[j]) exponential(j, flat[j]);
         }
     }
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-        if constexpr (!FLAT) {
-            if (quad[j])
-                quadratic(j, dr[j]);
-            else
-                exponential(j, dr[j]);
-        }
-        const float dm = dr[j].dm, ft = dr[j].ft, fs = dr[j].fs, corr = dr[j].corr;
-        const bool mok = dr[j].mok;
+        Draw o;
+        if constexpr (FLAT)
+            o = flat[j];
+        else if (quad[j])
+            quadratic(j, o);
+        else
+            exponential(j, o);
+        const float dm = o.dm, ft = o.ft, fs = o.fs, corr = o.corr;
+        const bool mok = o.mok;
         // The reference's log-price step multiplies V' - V by rho/sigma and V + V' - 2 th by
         // kappa rho dt / (2 sigma). As differences of FP32 variances they would carry ulp(V) errors
         // amplified by 1/sigma (prices tens of percent off at sigma = 1e-6, or at sigma = 1e-4
@@ -595,80 +596,27 @@ __device__ __forceinline__ void philox_block(uint32_t blk, const uint32_t (&plo)
     }
 }
 
-// The end of a run of steps: the Asian accumulation of its interior, the expiries finalised there
-// (payoff sums of the wave's tiles through the wave's LDS region) and the accumulation over the
-// first step of the next run.
-template <int PPT, bool DEBUG, bool GEO>
-__device__ __forceinline__ void end_run_fp32(const PathArgs& a, const DevReq& R, const DevSeg& S, uint32_t tile0, int lane,
-                                             uint32_t* lds, const bool (&valid)[PPT], const float (&X)[PPT],
-                                             const float (&Xp)[PPT], float (&P)[PPT], float (&acc)[PPT],
-                                             float (&Xs)[PPT], const float (&Y)[PPT], const float (&Yp)[PPT],
-                                             float (&PY)[PPT], float (&accY)[PPT], float (&Ys)[PPT]) {
-    // Asian accumulation of the run's interior steps b..e-1:
-    // delta * (X_{b-1}/2 + X_b + ... + X_{e-2} + X_{e-1}/2) = delta * (P - X_e + (Xs - Xp)/2)
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-        acc[j] = __builtin_fmaf(S.delta_f, (P[j] - X[j]) + 0.5f * (Xs[j] - Xp[j]), acc[j]);
-        if constexpr (GEO) accY[j] = __builtin_fmaf(S.delta_f, (PY[j] - Y[j]) + 0.5f * (Ys[j] - Yp[j]), accY[j]);
-    }
-    // per-path values at an expiry: (A, X_T), with GEO (A, X_T, G, -); the wave's LDS region
-    // holds 4 words per path either way
-    using Val = typename std::conditional<GEO, float4, float2>::type;
-    Val* vals = reinterpret_cast<Val*>(lds);
-    for (uint32_t f = 0; f < S.fin_count; ++f) {
-        const DevFin& F = a.fins[S.fin_begin + f];
-        const float w = F.w_f, invT = F.invT_f;
-        NanBits nan;
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            const float dX = X[j] - Xp[j];
-            const float xt = __builtin_fmaf(dX, w, Xp[j]);
-            const float A = (R.flags & kTrapezoid) ? (acc[j] + F.hwdt_f * (Xp[j] + xt)) * invT
-                                                   : __builtin_fmaf(dX, w, acc[j]) * invT;
-            // paths beyond n_paths carry -inf: every payoff max(0, . - K) is then 0
-            if constexpr (GEO) {
-                // the same functional on Y, normalised by its weight sum W: G/S0 = W 2^(L/W)
-                const float dY = Y[j] - Yp[j];
-                const float L = (R.flags & kTrapezoid)
-                                    ? (accY[j] + F.hwdt_f * (Yp[j] + __builtin_fmaf(dY, w, Yp[j]))) * invT
-                                    : __builtin_fmaf(dY, w, accY[j]) * invT;
-                const float G = F.gW_f * __builtin_amdgcn_exp2f(L * F.gInvW_f);
-                vals[j * kTile + lane] =
-                    valid[j] ? make_float4(A, xt, G, 0.0f) : make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-                nan.mark(j, valid[j], A, xt, G);
-            } else {
-                vals[j * kTile + lane] = valid[j] ? make_float2(A, xt) : make_float2(-INFINITY, -INFINITY);
-                nan.mark(j, valid[j], A, xt, 0.0f);
-            }
-            if constexpr (DEBUG) {
-                if (valid[j] && a.finals) {
-                    const uint64_t pl = (uint64_t)(tile0 + (uint32_t)j) * kTile + (uint64_t)lane;
-                    double* out = a.finals + (pl * R.n_exp + F.chain) * 2;
-                    out[0] = (double)A * R.S0;
-                    out[1] = (double)xt * R.S0;
-                }
-            }
-        }
-        wave_sync_lds();
-        reduce_tiles<PPT>(a, R, F, tile0, lane, vals, nan);
-        wave_sync_lds();
-    }
-    const float hn = 0.5f * S.dnext_f;
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-        acc[j] = __builtin_fmaf(hn, X[j] + Xp[j], acc[j]);
-        Xs[j] = X[j];
-        P[j] = 0.0f;
-        if constexpr (GEO) {
-            accY[j] = __builtin_fmaf(hn, Y[j] + Yp[j], accY[j]);
-            Ys[j] = Y[j];
-            PY[j] = 0.0f;
-        }
-    }
+// A chunk's draws in the split kernel (below), step-major: (Z_V, Z_X) and the word of Z_V (the
+// exponential branch's uniform).
+template <uint32_t C>
+struct DrawChunk {
+    float2 z[C][kTile];
+    uint32_t w[C][kTile];
+};
+template <>
+struct DrawChunk<0> {};
+
+__device__ __forceinline__ void workgroup_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
-__device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32_t tile0, int lane, uint32_t* lds) {
+// The paths of a lane through the request's runs. C = 0: the draws are made here, a counter block per
+// two steps; else they come in chunks of C steps from the drawing waves (PPT = 1).
+template <uint32_t C, int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
+__device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32_t tile0, int lane, uint32_t* lds,
+                                          const DrawChunk<C>* buf = nullptr) {
     const DevReq& R = a.reqs[ri];
     const uint64_t n_paths = R.n_paths;
     const uint32_t key0 = R.seed_lo, key1 = R.seed_hi;
@@ -703,31 +651,128 @@ __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32
         const DevSeg& S = a.segs[R.seg_begin + s];
         const SegF c{S.omd, S.th, S.c1h, S.c2h, S.g0, S.ka, S.kb, S.k3, S.mA, S.ma, S.mh, S.mr};
         const uint32_t n = S.n_steps;
-        uint32_t i = 0;
-        if ((k & 1u) && n > 0) {  // second half of a block opened by the previous run
-            qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, sv, sx, c, valid, cnt, nv);
-            ++i;
-            ++k;
+        if constexpr (C == 0) {
+            uint32_t i = 0;
+            if ((k & 1u) && n > 0) {  // second half of a block opened by the previous run
+                qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, sv, sx, c, valid, cnt, nv);
+                ++i;
+                ++k;
+            }
+            for (; i + 2 <= n; i += 2, k += 2) {
+                uint32_t w0[PPT], w1[PPT], w2[PPT], w3[PPT];
+                philox_block<PPT>(k >> 1, plo, phi, key0, key1, w0, w1, w2, w3);
+                qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w0, w1, c, valid, cnt, nv);
+                qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w2, w3, c, valid, cnt, nv);
+            }
+            if (i < n) {
+                uint32_t w0[PPT], w1[PPT];
+                philox_block<PPT>(k >> 1, plo, phi, key0, key1, w0, w1, sv, sx);
+                qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w0, w1, c, valid, cnt, nv);
+                ++k;
+            }
+        } else {
+            auto step = [&](float2 z, uint32_t w) {
+                float d0[1], m[1], s2h[1], m2[1], tt[1];
+                bool quad[1];
+                qe_moments_fp32<1>(V, c, d0, m, s2h, m2, tt, quad);
+                const uint32_t wv[1] = {w};
+                const float zv[1] = {z.x}, zx[1] = {z.y};
+                qe_update_fp32<true, 1, MART, GEO>(V, Y, X, Xp, P, Yp, PY, wv, zv, zx, d0, m, s2h, m2, tt, quad, c);
+            };
+            for (uint32_t left = n; left;) {
+                const uint32_t at = k % C;
+                if (at == 0) workgroup_sync_lds();
+                const DrawChunk<C>& d = buf[k / C % 2u];
+                if (at == 0 && left >= C) {  // a whole chunk: its draws in registers, no loop
+                    float2 z[C];
+                    uint32_t w[C];
+#pragma unroll
+                    for (uint32_t t = 0; t < C; ++t) {
+                        z[t] = d.z[t][lane];
+                        w[t] = d.w[t][lane];
+                    }
+#pragma unroll
+                    for (uint32_t t = 0; t < C; ++t) step(z[t], w[t]);
+                    k += C;
+                    left -= C;
+                } else {
+                    const uint32_t end = min(C, at + left);
+                    for (uint32_t t = at; t < end; ++t) step(d.z[t][lane], d.w[t][lane]);
+                    k += end - at;
+                    left -= end - at;
+                }
+            }
         }
-        for (; i + 2 <= n; i += 2, k += 2) {
-            uint32_t w0[PPT], w1[PPT], w2[PPT], w3[PPT];
-            philox_block<PPT>(k >> 1, plo, phi, key0, key1, w0, w1, w2, w3);
-            qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w0, w1, c, valid, cnt, nv);
-            qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w2, w3, c, valid, cnt, nv);
+        // Asian accumulation of the run's interior steps b..e-1:
+        // delta * (X_{b-1}/2 + X_b + ... + X_{e-2} + X_{e-1}/2) = delta * (P - X_e + (Xs - Xp)/2)
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+            acc[j] = __builtin_fmaf(S.delta_f, (P[j] - X[j]) + 0.5f * (Xs[j] - Xp[j]), acc[j]);
+            if constexpr (GEO) accY[j] = __builtin_fmaf(S.delta_f, (PY[j] - Y[j]) + 0.5f * (Ys[j] - Yp[j]), accY[j]);
         }
-        if (i < n) {
-            uint32_t w0[PPT], w1[PPT];
-            philox_block<PPT>(k >> 1, plo, phi, key0, key1, w0, w1, sv, sx);
-            qe_step_fp32<PPT, COUNT, MART, GEO>(V, Y, X, Xp, P, Yp, PY, w0, w1, c, valid, cnt, nv);
-            ++k;
+        // per-path values at an expiry: (A, X_T), with GEO (A, X_T, G, -); the wave's LDS region
+        // holds 4 words per path either way
+        using Val = typename std::conditional<GEO, float4, float2>::type;
+        Val* vals = reinterpret_cast<Val*>(lds);
+        for (uint32_t f = 0; f < S.fin_count; ++f) {
+            const DevFin& F = a.fins[S.fin_begin + f];
+            const float w = F.w_f, invT = F.invT_f;
+            NanBits nan;
+#pragma unroll
+            for (int j = 0; j < PPT; ++j) {
+                const float dX = X[j] - Xp[j];
+                const float xt = __builtin_fmaf(dX, w, Xp[j]);
+                const float A = (R.flags & kTrapezoid) ? (acc[j] + F.hwdt_f * (Xp[j] + xt)) * invT
+                                                       : __builtin_fmaf(dX, w, acc[j]) * invT;
+                // paths beyond n_paths carry -inf: every payoff max(0, . - K) is then 0
+                if constexpr (GEO) {
+                    // the same functional on Y, normalised by its weight sum W: G/S0 = W 2^(L/W)
+                    const float dY = Y[j] - Yp[j];
+                    const float L = (R.flags & kTrapezoid)
+                                        ? (accY[j] + F.hwdt_f * (Yp[j] + __builtin_fmaf(dY, w, Yp[j]))) * invT
+                                        : __builtin_fmaf(dY, w, accY[j]) * invT;
+                    const float G = F.gW_f * __builtin_amdgcn_exp2f(L * F.gInvW_f);
+                    vals[j * kTile + lane] =
+                        valid[j] ? make_float4(A, xt, G, 0.0f) : make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+                    nan.mark(j, valid[j], A, xt, G);
+                } else {
+                    vals[j * kTile + lane] = valid[j] ? make_float2(A, xt) : make_float2(-INFINITY, -INFINITY);
+                    nan.mark(j, valid[j], A, xt, 0.0f);
+                }
+                if constexpr (DEBUG) {
+                    if (valid[j] && a.finals) {
+                        const uint64_t pl = (uint64_t)(tile0 + (uint32_t)j) * kTile + (uint64_t)lane;
+                        double* out = a.finals + (pl * R.n_exp + F.chain) * 2;
+                        out[0] = (double)A * R.S0;
+                        out[1] = (double)xt * R.S0;
+                    }
+                }
+            }
+            wave_sync_lds();
+            reduce_tiles<PPT>(a, R, F, tile0, lane, vals, nan);
+            wave_sync_lds();
         }
-        end_run_fp32<PPT, DEBUG, GEO>(a, R, S, tile0, lane, lds, valid, X, Xp, P, acc, Xs, Y, Yp, PY, accY, Ys);
+        const float hn = 0.5f * S.dnext_f;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+            acc[j] = __builtin_fmaf(hn, X[j] + Xp[j], acc[j]);
+            Xs[j] = X[j];
+            P[j] = 0.0f;
+            if constexpr (GEO) {
+                accY[j] = __builtin_fmaf(hn, Y[j] + Yp[j], accY[j]);
+                Ys[j] = Y[j];
+                PY[j] = 0.0f;
+            }
+        }
     }
     if constexpr (COUNT) count_flush(a.counts, cnt.quad, cnt.exp, cnt.central, cnt.tail, lane);
 }
 
+// Registers for 5 waves per SIMD at 2 paths per lane (96), 4 with the martingale step: it needs 114,
+// and held to 96 it spilled 22 (4e6 paths x 252 steps 2.58 -> 2.48 ms, 2^20 stiff paths x 2,048 steps
+// 7.15 -> 6.90).
 template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 && !MART ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
     extern __shared__ uint32_t lds_u32[];
     const int lane = (int)(threadIdx.x & 63u);
     // the wave's LDS region, at a wave-uniform address
@@ -738,7 +783,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 ? 
         const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
         const uint32_t first = sp ? a.item_end[sp - 1] : 0u;
         const uint32_t ri = uniform(a.order[sp]);
-        path_fp32<PPT, DEBUG, COUNT, MART, GEO>(a, ri, uniform((item - first) * (uint32_t)PPT), lane, lds);
+        path_fp32<0, PPT, DEBUG, COUNT, MART, GEO>(a, ri, uniform((item - first) * (uint32_t)PPT), lane, lds);
     }
 }
 // ------------------------------------------------------------------------------------------
@@ -757,19 +802,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 ? 
 // 1e5 159 -> 97, 4e5 323 -> 234, 1e6 593 -> 541; martingale step 2e5 paths 245 -> 176 us;
 // the 8 x 64 grid at 1e6 paths 1802 -> 1718 us. The stepping wave's priority is raised: the tile
 // waits for it (400k paths 240 -> 234 us, the grid at a quarter of its paths 501 -> 478).
-// A chunk's draws, step-major: (Z_V, Z_X) and the word of Z_V (the exponential branch's uniform).
-template <uint32_t C>
-struct DrawChunk {
-    float2 z[C][kTile];
-    uint32_t w[C][kTile];
-};
-
-__device__ __forceinline__ void workgroup_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Drawing wave `part` of NP: counter blocks part, part + NP, ... of every chunk. Every wave of the
 // workgroup meets ceil(n_steps / C) barriers: here after each chunk drawn, in the stepping wave
 // before each chunk stepped, so that a buffer is rewritten only after its chunk has been consumed.
@@ -798,51 +830,6 @@ __device__ __forceinline__ void draw_fp32(const DevReq& R, uint32_t tile, int la
     }
 }
 
-template <uint32_t C, bool MART, bool GEO>
-__device__ __forceinline__ void step_fp32(const PathArgs& a, const DevReq& R, uint32_t tile, int lane,
-                                          const DrawChunk<C>* buf, uint32_t* lds) {
-    float V[1] = {R.v0_f}, Y[1] = {0.0f}, X[1] = {1.0f}, Xp[1] = {1.0f}, P[1] = {0.0f}, acc[1] = {0.0f}, Xs[1] = {1.0f};
-    float Yp[1] = {0.0f}, PY[1] = {0.0f}, accY[1] = {0.0f}, Ys[1] = {0.0f};
-    const bool valid[1] = {(uint64_t)tile * kTile + (uint64_t)lane < R.n_paths};
-    uint32_t k = 0;
-    for (uint32_t s = 0; s < R.n_segs; ++s) {
-        const DevSeg& S = a.segs[R.seg_begin + s];
-        const SegF c{S.omd, S.th, S.c1h, S.c2h, S.g0, S.ka, S.kb, S.k3, S.mA, S.ma, S.mh, S.mr};
-        auto step = [&](float2 z, uint32_t w) {
-            float d0[1], m[1], s2h[1], m2[1], tt[1];
-            bool quad[1];
-            qe_moments_fp32<1>(V, c, d0, m, s2h, m2, tt, quad);
-            const uint32_t wv[1] = {w};
-            const float zv[1] = {z.x}, zx[1] = {z.y};
-            qe_update_fp32<true, 1, MART, GEO>(V, Y, X, Xp, P, Yp, PY, wv, zv, zx, d0, m, s2h, m2, tt, quad, c);
-        };
-        for (uint32_t left = S.n_steps; left;) {
-            const uint32_t at = k & (C - 1u);
-            if (at == 0) workgroup_sync_lds();
-            const DrawChunk<C>& d = buf[(k / C) & 1u];
-            if (at == 0 && left >= C) {  // a whole chunk: its draws in registers, no loop
-                float2 z[C];
-                uint32_t w[C];
-#pragma unroll
-                for (uint32_t t = 0; t < C; ++t) {
-                    z[t] = d.z[t][lane];
-                    w[t] = d.w[t][lane];
-                }
-#pragma unroll
-                for (uint32_t t = 0; t < C; ++t) step(z[t], w[t]);
-                k += C;
-                left -= C;
-            } else {
-                const uint32_t end = min(C, at + left);
-                for (uint32_t t = at; t < end; ++t) step(d.z[t][lane], d.w[t][lane]);
-                k += end - at;
-                left -= end - at;
-            }
-        }
-        end_run_fp32<1, false, GEO>(a, R, S, tile, lane, lds, valid, X, Xp, P, acc, Xs, Y, Yp, PY, accY, Ys);
-    }
-}
-
 template <uint32_t NP, uint32_t C, bool MART, bool GEO>
 __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
     __shared__ DrawChunk<C> buf[2];
@@ -851,15 +838,15 @@ __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
     const uint32_t item = blockIdx.x;
     const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
     const uint32_t tile = uniform(item - (sp ? a.item_end[sp - 1] : 0u));
-    const DevReq& R = a.reqs[uniform(a.order[sp])];
+    const uint32_t ri = uniform(a.order[sp]);
     // the stepping wave's place in the workgroup varies with the tile, so that the waves of one role
     // do not gather on the same SIMDs
     const uint32_t role = (uniform(threadIdx.x >> 6) + (uint32_t)__builtin_popcount(item * 0x9E3779B1u >> 16)) % (NP + 1);
     if (role == 0) {
         __builtin_amdgcn_s_setprio(2);
-        step_fp32<C, MART, GEO>(a, R, tile, lane, buf, vals);
+        path_fp32<C, 1, false, false, MART, GEO>(a, ri, tile, lane, vals, buf);
     } else {
-        draw_fp32<NP, C>(R, tile, lane, role - 1, buf);
+        draw_fp32<NP, C>(a.reqs[ri], tile, lane, role - 1, buf);
     }
 }
 #pragma clang fp contract(fast)
