@@ -278,8 +278,8 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
 }
 
 // Drawing waves per tile of the split kernel for a class of `tiles` 64-path tiles, or 0 for the
-// persistent kernel. FP32 only, and where the launch shape is left to the library (2 paths per
-// thread, no occupancy cap).
+// persistent kernel. FP32, where the launch shape is left to the library (2 paths per thread, no
+// occupancy cap):
 //  * up to 512 tiles (half the SIMDs): two drawing waves; the tile's time is the stepping wave's
 //    (1e4 paths x 126 steps 28.5 -> 20.4 us against one). Beyond, the third wave competes with
 //    other tiles' stepping waves: 5% faster still for quadratic-branch steps at 1,500 tiles, 15%
@@ -293,8 +293,15 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
 //    (2 kappa theta / sigma^2 < 0.6). 1,563 tiles x 1,024 steps 0.605 ms against 0.734, 4,096 tiles
 //    1.25 against 1.07; 15,625 tiles x 512 steps at ratios 0.05 to 0.44 1.86-1.90 against 1.73-1.77,
 //    at 0.79 1.38 against 1.52.
-uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, bool long_steps, const hexo_tuning& tun) {
-    if (cls == 0 || tun.paths_per_thread != 2 || tun.waves_per_simd != 0) return 0;
+// FP64 (whose kernels take the martingale correction at run time, with the library's log and log1p
+// on the stepping wave):
+//  * up to 512 tiles: two drawing waves (32,768 paths x 252 steps 165 us, 198 with one, 280
+//    persistent; 50,000 paths 214, 195, 286); up to 3,328: one (k_path_fp64_split).
+//  * with the correction up to 256 tiles (1e4 paths: 223 us against 392, stiff parameters 332 against
+//    500; at 313 tiles stiff 521 against 501, at 1,563 and one drawing wave 610 against 561).
+uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, bool martingale, bool long_steps, const hexo_tuning& tun) {
+    if (cls == 0) return tiles > (martingale ? 256u : 3328u) ? 0 : tiles <= 512 ? 2 : 1;
+    if (tun.paths_per_thread != 2 || tun.waves_per_simd != 0) return 0;
     if (tiles > (long_steps ? 2048u : 1u << 17)) return 0;
     return tiles <= 512 ? 2 : 1;
 }
@@ -370,7 +377,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint64_t n_geo_items = 0, n_geo_pts = 0, n_geo_waves = 0;
     uint32_t n_cls[kPathClasses] = {};
     uint64_t cls_tiles[kPathClasses] = {};
-    bool cls_long[kPathClasses] = {};  // a request with long steps (split_draw_waves)
+    bool cls_mart[kPathClasses] = {}, cls_long[kPathClasses] = {};  // requests with longer steps (split_draw_waves)
     for (uint32_t i = 0; i < n; ++i) {
         std::string why = validate(&reqs[i]);
         if (!why.empty()) {
@@ -396,8 +403,9 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         n_out += p.n_out;
         n_cls[p.cls]++;
         cls_tiles[p.cls] += p.n_tiles;
-        cls_long[p.cls] |= (reqs[i].flags & HEXO_MARTINGALE) &&
-                           2.0 * reqs[i].kappa * reqs[i].theta < 0.6 * reqs[i].sigma * reqs[i].sigma;
+        const bool mart = (reqs[i].flags & HEXO_MARTINGALE) != 0;
+        cls_mart[p.cls] |= mart;
+        cls_long[p.cls] |= mart && 2.0 * reqs[i].kappa * reqs[i].theta < 0.6 * reqs[i].sigma * reqs[i].sigma;
     }
     // Per kernel class: the split kernel's drawing waves (0: the persistent kernel) and the tiles per
     // work item (1, or the persistent FP32 kernels' paths per thread). A wave stores one partial per item and output (layout.hpp,
@@ -405,7 +413,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint32_t cls_ppt[kPathClasses], cls_store[kPathClasses];
     uint32_t cls_draw[kPathClasses];
     for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
-        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_long[cls], tun);
+        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_mart[cls], cls_long[cls], tun);
         cls_ppt[cls] = cls == 0 || cls_draw[cls] ? 1u : tun.paths_per_thread;
         cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;
     }
@@ -800,7 +808,8 @@ static int enqueue_body(Batch& b, PathMode mode, bool timed, double* d_finals, s
         a.finals = d_finals;
         a.counts = mode == PathMode::Count ? b.d_counts : nullptr;
         if (b.draw_waves[cls] && mode == PathMode::Normal)
-            HIP_TRY(launch_paths_split(b.draw_waves[cls], a, class_martingale(cls), class_geo(cls), b.stream));
+            HIP_TRY(launch_paths_split(class_precision(cls), b.draw_waves[cls], a, class_martingale(cls), class_geo(cls),
+                                       b.stream));
         else
             HIP_TRY(launch_paths(class_precision(cls), b.ppt[cls], mode, b.grid[cls], b.block[cls], b.stream, a,
                                  class_martingale(cls), class_geo(cls)));

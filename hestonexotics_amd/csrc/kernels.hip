@@ -7,7 +7,8 @@
 //              refills (src/RNG.cpp:28-43, src/as241.f90:85-118).
 // k_path_fp32_split  the same paths with the draws and the steps on different waves, for batches
 //              that leave k_path_fp32's persistent grid short of work.
-// k_path_fp64  the plain FP64 kernel: the same path in the reference's own FP64 form.
+// k_path_fp64, k_path_fp64_split  the plain FP64 kernel, the same path in the reference's own FP64
+//              form, and its division into drawing and stepping waves for small batches.
 // k_reduce_*   cross-tile reduction in a fixed order and the estimator (price, standard error);
 //              replaces the racy `prices[...] +=` of src/HSimulation.tpp:40,47-48.
 //
@@ -830,6 +831,12 @@ __device__ __forceinline__ void draw_fp32(const DevReq& R, uint32_t tile, int la
     }
 }
 
+// A wave's role in its workgroup of n waves: 0 steps, the others draw. The stepping wave's place
+// varies with the tile, so that the waves of one role do not gather on the same SIMDs.
+__device__ __forceinline__ uint32_t stepping_first(uint32_t wave, uint32_t item, uint32_t n) {
+    return (wave + (uint32_t)__builtin_popcount(item * 0x9E3779B1u >> 16)) % n;
+}
+
 template <uint32_t NP, uint32_t C, bool MART, bool GEO>
 __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
     __shared__ DrawChunk<C> buf[2];
@@ -839,9 +846,7 @@ __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
     const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
     const uint32_t tile = uniform(item - (sp ? a.item_end[sp - 1] : 0u));
     const uint32_t ri = uniform(a.order[sp]);
-    // the stepping wave's place in the workgroup varies with the tile, so that the waves of one role
-    // do not gather on the same SIMDs
-    const uint32_t role = (uniform(threadIdx.x >> 6) + (uint32_t)__builtin_popcount(item * 0x9E3779B1u >> 16)) % (NP + 1);
+    const uint32_t role = stepping_first(uniform(threadIdx.x >> 6), item, NP + 1);
     if (role == 0) {
         __builtin_amdgcn_s_setprio(2);
         path_fp32<C, 1, false, false, MART, GEO>(a, ri, tile, lane, vals, buf);
@@ -951,8 +956,18 @@ __device__ __forceinline__ double price_exp_f64(double y) {
     return x;
 }
 
-template <bool DEBUG, bool COUNT>
-__device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32_t tile, int lane, double4* vals) {
+// A chunk's draws in the FP64 split kernel (below), as DrawChunk.
+template <uint32_t C>
+struct DrawChunk64 {
+    double2 z[C][kTile];
+    uint32_t w[C][kTile];
+};
+template <>
+struct DrawChunk64<0> {};
+
+template <uint32_t C, bool DEBUG, bool COUNT>
+__device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32_t tile, int lane, double4* vals,
+                                          const DrawChunk64<C>* buf = nullptr) {
     const DevReq& R = a.reqs[ri];
     const bool geo = (R.payoffs & (kAsianGeoCV | kGeoAsian)) != 0;  // wave-uniform
     double accY = 0.0, yp = 0.0;  // the Asian accumulation on y = ln(X/S0); y before the last step
@@ -970,7 +985,14 @@ __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32
         const SegD c{S.e, S.s2v, S.s2c, S.dk0, S.dk1, S.dk2, S.dk3, S.delta};
         const uint32_t n = S.n_steps;
         for (uint32_t i = 0; i < n; ++i, ++k) {
-            if ((k & 1u) == 0u) {
+            if constexpr (C != 0) {
+                if (k % C == 0) workgroup_sync_lds();
+                const DrawChunk64<C>& d = buf[k / C % 2u];
+                const double2 zz = d.z[k % C][lane];
+                z[0] = zz.x;
+                z[1] = zz.y;
+                w.x = d.w[k % C][lane];
+            } else if ((k & 1u) == 0u) {
                 w = philox4x32_10(k >> 1, plo, phi, 0u, R.seed_lo, R.seed_hi);
                 normals4_f64(w, z, reinterpret_cast<double*>(vals), lane);
             } else {
@@ -1041,7 +1063,65 @@ __global__ __launch_bounds__(256) void k_path_fp64(PathArgs a) {
         const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
         const uint32_t first = sp ? a.item_end[sp - 1] : 0u;
         const uint32_t ri = uniform(a.order[sp]);
-        path_fp64<DEBUG, COUNT>(a, ri, uniform(item - first), lane, vals);
+        path_fp64<0, DEBUG, COUNT>(a, ri, uniform(item - first), lane, vals);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// FP64 path kernel with drawing and stepping waves (k_path_fp32_split's division of a tile's work)
+// ------------------------------------------------------------------------------------------
+// A lone wave of k_path_fp64 takes 2,600 cycles per step, of which its SIMD needs 1,200 for the
+// instructions: up to a few tiles per SIMD the time is the wave's. Drawing (half of the work) on
+// waves of their own: 1e4 paths x 252 steps 272 -> 120 us, 5e4 286 -> 195, 1e5 385 -> 314,
+// 2e5 593 -> 502. Beyond 13 tiles per CU (3,328) k_path_fp64 is as fast (3e5 716 against 734 us,
+// stiff parameters 938 against 845): its three waves per SIMD are full, and the LDS traffic is not
+// free.
+constexpr uint32_t kChunkSteps64 = 4;
+
+template <uint32_t NP>
+__device__ __forceinline__ void draw_fp64(const DevReq& R, uint32_t tile, int lane, uint32_t part,
+                                          DrawChunk64<kChunkSteps64>* buf, double* queue) {
+    constexpr uint32_t C = kChunkSteps64;
+    static_assert(C % (2 * NP) == 0, "whole counter blocks per wave and chunk");
+    const uint64_t first = R.path_offset + (uint64_t)tile * kTile;  // tiles never straddle 2^32
+    const uint32_t plo = (uint32_t)first + (uint32_t)lane, phi = uniform((uint32_t)(first >> 32));
+    const uint32_t n_steps = R.n_steps;
+    for (uint32_t k = 0, c = 0; k < n_steps; k += C, ++c) {
+        DrawChunk64<C>& d = buf[c & 1u];
+        for (uint32_t b = 0; b < C / 2; b += NP) {
+            const uint32_t t = 2 * (b + part);
+            const u32x4 w = philox4x32_10((k + t) >> 1, plo, phi, 0u, R.seed_lo, R.seed_hi);
+            double z[4];
+            normals4_f64(w, z, queue, lane);
+            d.z[t][lane] = make_double2(z[0], z[1]);
+            d.w[t][lane] = w.x;
+            d.z[t + 1][lane] = make_double2(z[2], z[3]);
+            d.w[t + 1][lane] = w.z;
+        }
+        workgroup_sync_lds();  // as in draw_fp32: ceil(n_steps / C) barriers in every wave
+    }
+}
+
+// One drawing wave: 4 waves per SIMD (128 registers, 18 spilled constants) against the 3 of an
+// unconstrained build: 2e5 paths x 252 steps 552 -> 516 us. Two, for at most half a tile per SIMD,
+// have no use for them.
+template <uint32_t NP>
+__global__ __launch_bounds__(64 * (NP + 1)) __attribute__((amdgpu_waves_per_eu(NP == 1 ? 4 : 3))) void k_path_fp64_split(
+    PathArgs a) {
+    __shared__ DrawChunk64<kChunkSteps64> buf[2];
+    __shared__ double queue[NP][4 * kTile];
+    __shared__ double4 vals[kTile];
+    const int lane = (int)(threadIdx.x & 63u);
+    const uint32_t item = blockIdx.x;
+    const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
+    const uint32_t tile = uniform(item - (sp ? a.item_end[sp - 1] : 0u));
+    const uint32_t ri = uniform(a.order[sp]);
+    const uint32_t role = stepping_first(uniform(threadIdx.x >> 6), item, NP + 1);
+    if (role == 0) {
+        __builtin_amdgcn_s_setprio(2);
+        path_fp64<kChunkSteps64, false, false>(a, ri, tile, lane, vals, buf);
+    } else {
+        draw_fp64<NP>(a.reqs[ri], tile, lane, role - 1, buf, queue[role - 1]);
     }
 }
 
@@ -1306,22 +1386,29 @@ size_t path_lds_bytes(uint32_t precision, uint32_t ppt, uint32_t block) {
     return precision == kPrecFP64 ? waves * kTile * sizeof(double4) : waves * 4 * ppt * kTile * sizeof(uint32_t);
 }
 
-hipError_t launch_paths_split(uint32_t n_draw, const PathArgs& a, bool mart, bool geo, hipStream_t st) {
-#define HEXO_SPLIT(NP, C)                                                                    \
-    if (mart && geo)                                                                         \
-        k_path_fp32_split<NP, C, true, true><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);    \
-    else if (mart)                                                                           \
-        k_path_fp32_split<NP, C, true, false><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);   \
-    else if (geo)                                                                            \
-        k_path_fp32_split<NP, C, false, true><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);   \
-    else                                                                                     \
-        k_path_fp32_split<NP, C, false, false><<<a.total_items, 64 * (NP + 1), 0, st>>>(a);
-    if (n_draw == 2) {
-        HEXO_SPLIT(2, 8)
-    } else if (n_draw == 1) {
-        HEXO_SPLIT(1, 4)
+hipError_t launch_paths_split(uint32_t precision, uint32_t n_draw, const PathArgs& a, bool mart, bool geo,
+                              hipStream_t st) {
+    if (n_draw != 1 && n_draw != 2) return hipErrorInvalidValue;
+    if (precision == kPrecFP64) {
+        if (n_draw == 2)
+            k_path_fp64_split<2><<<a.total_items, 192, 0, st>>>(a);
+        else
+            k_path_fp64_split<1><<<a.total_items, 128, 0, st>>>(a);
+        return hipGetLastError();
+    }
+#define HEXO_SPLIT(M, G)                                                           \
+    if (n_draw == 2)                                                               \
+        k_path_fp32_split<2, 8, M, G><<<a.total_items, 192, 0, st>>>(a);           \
+    else                                                                           \
+        k_path_fp32_split<1, 4, M, G><<<a.total_items, 128, 0, st>>>(a);
+    if (mart && geo) {
+        HEXO_SPLIT(true, true)
+    } else if (mart) {
+        HEXO_SPLIT(true, false)
+    } else if (geo) {
+        HEXO_SPLIT(false, true)
     } else {
-        return hipErrorInvalidValue;
+        HEXO_SPLIT(false, false)
     }
 #undef HEXO_SPLIT
     return hipGetLastError();

@@ -16,9 +16,10 @@ const void* path_kernel_symbol(uint32_t precision, uint32_t ppt, PathMode mode, 
 size_t path_lds_bytes(uint32_t precision, uint32_t ppt, uint32_t block);
 hipError_t launch_paths(uint32_t precision, uint32_t ppt, PathMode mode, uint32_t grid, uint32_t block,
                         hipStream_t st, const PathArgs& a, bool mart = false, bool geo = false);
-// The FP32 kernel with n_draw (1 or 2) drawing waves and a stepping wave per 64-path tile
+// The kernels with n_draw (1 or 2) drawing waves and a stepping wave per 64-path tile
 // (PathArgs.total_items tiles; partials stored per tile).
-hipError_t launch_paths_split(uint32_t n_draw, const PathArgs& a, bool mart, bool geo, hipStream_t st);
+hipError_t launch_paths_split(uint32_t precision, uint32_t n_draw, const PathArgs& a, bool mart, bool geo,
+                              hipStream_t st);
 // Exact prices of the geometric control variates (geo.hip); GeoArgs.state holds
 // geo_state_doubles(n_items) doubles.
 hipError_t launch_geo(const GeoArgs& a, hipStream_t st);

@@ -472,3 +472,24 @@ def test_split_kernel_equals_persistent(ctx, n_paths, steps, T, precision):
                 ctx.set_tuning(**base)
             np.testing.assert_array_equal(got[0], want[0])
             np.testing.assert_array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n_paths,steps,T", [s for s in SPLIT_SIZES if s[0] <= 512 * 64 + 1] + [(3328 * 64, 5, [1.0])])
+def test_fp64_split_kernel_equals_persistent(ctx, n_paths, steps, T):
+    """The FP64 kernel with drawing and stepping waves (batches up to 3,328 tiles, 256 with the
+    martingale correction) gives the persistent kernel's bits: the same request alone and beside one
+    that takes the batch past that size."""
+    K = list(np.linspace(80.0, 120.0, 50 if n_paths == 2000 else 3))
+    filler = H.Request(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, expiries=[1.0],
+                       strikes=[[100.0]], steps=1, n_paths=3329 * 64, seed=1, precision=H.FP64)
+    for model in (dict(rho=-0.7, kappa=2.0, sigma=0.3), dict(rho=-0.9, kappa=0.5, sigma=0.9)):
+        for flags, payoffs in ((0, H.ASIAN | H.EUROPEAN), (H.DRIFT | H.DISCOUNT | H.TRAPEZOID, H.ASIAN),
+                               (H.MARTINGALE, H.EUROPEAN), (0, H.ASIAN | H.GEO_ASIAN)):
+            if payoffs & H.GEO_ASIAN and steps < 3:
+                continue
+            req = H.Request(v0=0.04, theta=0.04, S0=100.0, expiries=T, strikes=[K] * len(T), steps=steps,
+                            n_paths=n_paths, seed=n_paths, r=0.02, flags=flags, payoffs=payoffs,
+                            precision=H.FP64, path_offset=64 * steps, **model)
+            got, want = ctx.price(req), ctx.price_batch([req, filler])[0]
+            np.testing.assert_array_equal(got[0], want[0])
+            np.testing.assert_array_equal(got[1], want[1])
