@@ -159,7 +159,12 @@ int hexo_ctx_destroy(hexo_ctx* ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipStreamDestroy(ctx->stream);
     }
+    if (ctx->swift_stream) {
+        (void)hipStreamSynchronize(ctx->swift_stream);
+        (void)hipStreamDestroy(ctx->swift_stream);
+    }
     if (ctx->swift_dev) (void)hipFree(ctx->swift_dev);
+    if (ctx->swift_roots) (void)hipFree(ctx->swift_roots);
     delete ctx;
     return HEXO_OK;
 }

@@ -162,16 +162,19 @@ struct hexo_ctx {
     std::mutex server_mu;
     std::shared_ptr<struct hexo_server_state> server;
     std::unordered_set<struct hexo_batch*> batches;  // live batches; released by hexo_ctx_destroy
-    // SWIFT pricer workspace, grown on demand and kept for the context's lifetime (no per-call
-    // allocation, which would also synchronise the device). The kernels read their inputs from
-    // and write their results to the two fine-grained pinned buffers in place: the grid kernel's
-    // inputs, strikes and outputs in swift_in_host; the pricing kernels' tables (which a first
-    // kernel copies to the device) and results in swift_host. No copy-engine transfer, whose
-    // hand-offs with the kernels would cost more than the transfers themselves.
+    // SWIFT pricer, grown on demand and kept for the context's lifetime (no per-call allocation, which
+    // would also synchronise the device): two fine-grained pinned stages, which the kernels read their
+    // inputs from and write the grids and results to in place (no copy-engine transfer, whose
+    // hand-offs with the kernels would cost more than the transfers themselves); the roots of unity
+    // of the transforms, made at the first call; the work arrays; and a stage for the tables of
+    // chains too large for transforms in LDS.
+    hexo::PinnedBuf swift_in_host{nullptr, 0, hipHostMallocCoherent};
+    hexo::PinnedBuf swift_host{nullptr, 0, hipHostMallocCoherent};
+    void* swift_roots = nullptr;
+    hipStream_t swift_stream = nullptr;  // of the longest chains of a large call
     void* swift_dev = nullptr;
     size_t swift_dev_bytes = 0;
-    hexo::PinnedBuf swift_host{nullptr, 0, hipHostMallocCoherent};
-    hexo::PinnedBuf swift_in_host{nullptr, 0, hipHostMallocCoherent};
+    hexo::PinnedBuf swift_large_host{nullptr, 0, hipHostMallocCoherent};
     // the synchronous pricing calls' device arena and staging buffer, likewise grown on demand and
     // resident (guarded by mu): hexo_price and hexo_price_batch allocate nothing once they fit
     hexo::Arena sync_arena;

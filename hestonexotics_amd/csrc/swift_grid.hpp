@@ -13,14 +13,10 @@
 namespace hexo {
 
 // One chain's inputs to the grid choice: model, expiry, rate, spot, the extreme strikes and the
-// truncation precision. The GPU grid kernel finds the extreme strikes itself, from the chain's
-// n_strikes strikes at strike_off of the call's strike array (checking them on the way).
+// truncation precision.
 struct SwiftGridIn {
     double p[5];  // v0, theta, rho, kappa, sigma
     double T, r, S0, kmin, kmax, trunc;
-    uint64_t strike_off;
-    uint32_t n_strikes;
-    uint32_t pad;
 };
 
 // One chain's grid and its status: kSwiftGridOk, or which check of the choice failed.
@@ -76,15 +72,19 @@ __host__ __device__ inline double swift_cumulant4(const double p[5], double t) {
     return (3 * sigma2 * theta) / (64 * ::pow(kappa, 7)) * (b4 + b3 + b2 + b1 + b0);
 }
 
-// The rest of the grid once the scale m is known (src/SWIFT.cpp:24-34): the truncation range from
-// the strikes and the cumulants, the wavelet index range k1..k2 and J = 2^(ceil(log2(pi |k2 - k1|)) - 2).
-__host__ __device__ inline int32_t swift_grid_finish(const SwiftGridIn& q, uint32_t m, hexo_swift_grid& g,
+// Half-width of the truncation range around the strikes, from the cumulants (src/SWIFT.cpp:24-27).
+__host__ __device__ inline double swift_grid_width(const double p[5], double T) {
+    return ::fabs(swift_cumulant1(p, T)) +
+           10.0 * ::sqrt(::fabs(swift_cumulant2(p, T)) + ::sqrt(::fabs(swift_cumulant4(p, T))));
+}
+
+// The rest of the grid once the scale m and the half-width c are known (src/SWIFT.cpp:24-34): the
+// truncation range, the wavelet index range k1..k2 and J = 2^(ceil(log2(pi |k2 - k1|)) - 2).
+__host__ __device__ inline int32_t swift_grid_finish(const SwiftGridIn& q, double c, uint32_t m, hexo_swift_grid& g,
                                                      double& J_wanted) {
     const double pi = 3.14159265358979323846;
     const double hi = q.r * q.T + ::log(q.S0 / q.kmin);
     const double lo = q.r * q.T + ::log(q.S0 / q.kmax);
-    const double c = ::fabs(swift_cumulant1(q.p, q.T)) +
-                     10.0 * ::sqrt(::fabs(swift_cumulant2(q.p, q.T)) + ::sqrt(::fabs(swift_cumulant4(q.p, q.T))));
     g.m = m;
     g.exp2_m = 1u << m;
     g.sqrt_exp2_m = ::sqrt((double)g.exp2_m);
@@ -102,11 +102,5 @@ __host__ __device__ inline int32_t swift_grid_finish(const SwiftGridIn& q, uint3
     g.reserved = 0;
     return kSwiftGridOk;
 }
-
-// The grid of chains in[0..n) on the GPU (one wavefront per chain; the scales m = 0..30 are tried
-// in parallel and the first that reaches the truncation precision is taken, as the reference's
-// loop takes it), with each chain's extreme strikes from `strikes`.
-hipError_t launch_swift_grid(const SwiftGridIn* in, const double* strikes, SwiftGridOut* out, uint32_t n,
-                             hipStream_t st);
 
 }  // namespace hexo

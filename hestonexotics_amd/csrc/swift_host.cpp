@@ -1,14 +1,14 @@
 // swift_host.cpp -- host side of the SWIFT European pricer: validation, the dynamic grid (the
 // reference's SwiftParameters constructor, src/SWIFT.cpp:21-35) for hexo_swift_grid_for (a call's
-// grids are chosen on the GPU, swift_grid.hpp), the layout of one call's chains in the context's
-// pinned stages and device workspace, and the C entry points hexo_swift_grid_for /
-// hexo_swift_price.
+// grids are chosen on the GPU, swift.hip), the layout of one call's chains in the context's
+// pinned stages, and the C entry points hexo_swift_grid_for / hexo_swift_price.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -105,8 +105,7 @@ int check_grid(const hexo_swift_grid& g, std::string& err) {
 // SwiftParameters constructor (src/SWIFT.cpp:21-35).
 // The extreme strikes and the rest of a chain's grid-choice inputs.
 hexo::SwiftGridIn grid_input(const hexo_swift_request& q) {
-    hexo::SwiftGridIn in{{q.v0, q.theta, q.rho, q.kappa, q.sigma}, q.T, q.r, q.S0, q.strikes[0], q.strikes[0], q.trunc,
-                         0, q.n_strikes, 0};
+    hexo::SwiftGridIn in{{q.v0, q.theta, q.rho, q.kappa, q.sigma}, q.T, q.r, q.S0, q.strikes[0], q.strikes[0], q.trunc};
     for (uint32_t i = 1; i < q.n_strikes; ++i) {
         in.kmin = std::min(in.kmin, q.strikes[i]);
         in.kmax = std::max(in.kmax, q.strikes[i]);
@@ -134,7 +133,7 @@ int dynamic_grid(const hexo_swift_request& q, hexo_swift_grid& g, std::string& e
     while (int_error(in.p, q.T, m++) > q.trunc)
         if (m > 30) return grid_status(hexo::kSwiftGridNoScale, 0.0, err);
     double J = 0.0;
-    return grid_status(hexo::swift_grid_finish(in, m, g, J), J, err);
+    return grid_status(hexo::swift_grid_finish(in, hexo::swift_grid_width(in.p, in.T), m, g, J), J, err);
 }
 
 // Grows one of the context's SWIFT device buffers to at least `bytes` (kept for the context's
@@ -173,65 +172,37 @@ extern "C" int hexo_swift_grid_for(const hexo_swift_request* req, hexo_swift_gri
     return grid_of(*req, *out, err);
 }
 
-extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, uint32_t n, double* prices, double* grads,
-                                hexo_swift_grid* grids_used) {
-    if (!ctx) return HEXO_ERR_INVALID;
-    if (!reqs || !prices || n == 0) return ctx->set_error(HEXO_ERR_INVALID, "requests and prices must be non-NULL");
-    std::string err;
-    std::vector<uint64_t> strike_off(n);
-    std::vector<uint32_t> dyn;  // chains whose grid is chosen here (not HEXO_SWIFT_FIXED_GRID)
-    uint64_t n_strk = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        if (int rc = check_chain(reqs[i], err))
-            return ctx->set_error(rc, "swift request " + std::to_string(i) + ": " + err);
-        strike_off[i] = n_strk;
-        n_strk += reqs[i].n_strikes;
-        if (!(reqs[i].flags & HEXO_SWIFT_FIXED_GRID)) dyn.push_back(i);
-    }
-    std::lock_guard<std::recursive_mutex> lock(ctx->mu);
-    if (hipSetDevice(ctx->device) != hipSuccess) return ctx->set_error(HEXO_ERR_HIP, "hipSetDevice failed");
+namespace {
+
+// A chain's J up to a factor (J / 1.3, mostly within a factor of 2): the frequency where the
+// characteristic function, e^{-u sqrt(1 - rho^2) (v0 + kappa theta T) / sigma} far out, has fallen to
+// trunc, times the width of the log-price range, about 20 standard deviations and the strikes'. Only
+// the order and the class of a chain's workgroup depend on it.
+double size_estimate(const hexo_swift_request& q) {
+    if (q.flags & HEXO_SWIFT_FIXED_GRID) return 0.6 * q.grid.J;  // 1,024 below the line at 630, 2,048 above it
+    const double u = -std::log(q.trunc) * q.sigma / ((q.v0 + q.kappa * q.theta * q.T) * std::sqrt(1.0 - q.rho * q.rho));
+    const double size = u * (0.5 + 20.0 * std::sqrt(std::max(q.v0, q.theta) * q.T));
+    return std::isfinite(size) ? size : 1e300;  // ordered in any case
+}
+
+// Chains whose transforms exceed the LDS (J > kSwiftFftMaxJ), given their grids, through the direct
+// sums. idx: the chains; results go to their places in the pinned arrays.
+// Called with the context locked, its stream idle.
+int price_large(hexo_ctx* ctx, const hexo_swift_request* reqs, const std::vector<uint32_t>& idx,
+                const std::vector<hexo_swift_grid>& grids, const std::vector<uint64_t>& strike_off, uint64_t n_strk,
+                const double* h_strikes, double* h_prices, double* h_grads) {
     auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
     hipStream_t st = ctx->stream;
-    // ---- first phase: the grid kernel reads the strikes and grid inputs from the fine-grained
-    // pinned stage and writes the grids back into it (a wavefront per dynamic chain, which also
-    // finds the chain's extreme strikes and checks them). Stage layout:
-    // [strikes | grid inputs | grid outputs].
-    const size_t nd = dyn.size();
-    const size_t b_strk = align(8 * n_strk), b_gin = align(sizeof(hexo::SwiftGridIn) * nd),
-                 b_gout = sizeof(hexo::SwiftGridOut) * nd;
-    if (!ctx->swift_in_host.reserve(b_strk + b_gin + b_gout)) return ctx->set_error(HEXO_ERR_NOMEM, "hipHostMalloc failed");
-    unsigned char* in_host = reinterpret_cast<unsigned char*>(ctx->swift_in_host.p);
-    const double* h_strikes = reinterpret_cast<const double*>(in_host);
-    {
-        double* ks = reinterpret_cast<double*>(in_host);
-        for (uint32_t i = 0; i < n; ++i) std::memcpy(ks + strike_off[i], reqs[i].strikes, 8 * reqs[i].n_strikes);
-    }
-    hexo::SwiftGridOut* gout = reinterpret_cast<hexo::SwiftGridOut*>(in_host + b_strk + b_gin);
-    bool ok = true;
-    if (nd) {
-        hexo::SwiftGridIn* gin = reinterpret_cast<hexo::SwiftGridIn*>(in_host + b_strk);
-        for (size_t k = 0; k < nd; ++k) {
-            const hexo_swift_request& q = reqs[dyn[k]];
-            gin[k] = hexo::SwiftGridIn{{q.v0, q.theta, q.rho, q.kappa, q.sigma}, q.T, q.r, q.S0, 0.0, 0.0, q.trunc,
-                                       strike_off[dyn[k]], q.n_strikes, 0};
-        }
-        ok = hexo::launch_swift_grid(gin, h_strikes, gout, (uint32_t)nd, st) == hipSuccess;
-    }
-    auto fail = [&](int code, const std::string& msg) {
-        // drain what was queued before the pinned stages are reused
-        (void)hipStreamSynchronize(st);
-        return ctx->set_error(code, msg);
-    };
-    if (!ok) return fail(HEXO_ERR_HIP, "SWIFT grid launch failed");
-    // while the GPU chooses the grids: the strikes of the fixed-grid chains (the grid kernel checks
-    // the others') and the records' grid-independent fields
-    for (uint32_t i = 0; i < n; ++i)
-        if (reqs[i].flags & HEXO_SWIFT_FIXED_GRID)
-            if (int rc = check_strikes(reqs[i], err)) return fail(rc, "swift request " + std::to_string(i) + ": " + err);
-    const uint32_t rows = grads ? 6u : 1u;
+    const uint32_t n = (uint32_t)idx.size(), rows = h_grads ? 6u : 1u;
     std::vector<hexo::DevSwift> recs(n);
+    std::vector<hexo::SwiftTable> tables;
+    std::vector<uint64_t> ends(2 * (size_t)n);  // j, dens
+    std::vector<uint32_t> blk_chain, blk_strike;
+    uint64_t n_pay = 0, n_dens = 0, n_pm = 0;
+    hexo::SwiftTotals tot{0, 0, 0};
     for (uint32_t i = 0; i < n; ++i) {
-        const hexo_swift_request& q = reqs[i];
+        const hexo_swift_request& q = reqs[idx[i]];
+        const hexo_swift_grid& g = grids[idx[i]];
         hexo::DevSwift& R = recs[i];
         std::memset(&R, 0, sizeof(R));
         R.p[0] = q.v0;
@@ -245,34 +216,8 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
         R.disc = std::exp(-q.r * q.T);
         R.n_strikes = q.n_strikes;
         R.rows = rows;
-        R.strike_off = strike_off[i];
-        R.out_off = strike_off[i];
-    }
-    if (nd && hipStreamSynchronize(st) != hipSuccess) return fail(HEXO_ERR_HIP, "SWIFT grid launch failed");
-    std::vector<hexo_swift_grid> grids(n);
-    {
-        size_t k = 0;
-        for (uint32_t i = 0; i < n; ++i) {
-            if (reqs[i].flags & HEXO_SWIFT_FIXED_GRID) {
-                grids[i] = reqs[i].grid;
-            } else {
-                if (int rc = grid_status(gout[k].status, gout[k].J_wanted, err))
-                    return fail(rc, "swift request " + std::to_string(i) + ": " + err);
-                grids[i] = gout[k++].g;
-            }
-            if (int rc = check_grid(grids[i], err)) return fail(rc, "swift request " + std::to_string(i) + ": " + err);
-        }
-    }
-    // ---- second phase: the grid-dependent fields, tables, FFT chain list and prefix sums, then
-    // the work arrays
-    std::vector<hexo::SwiftTable> tables;
-    std::vector<uint32_t> fft_chains;
-    std::vector<uint64_t> ends(4 * (size_t)n);  // j, dens, dcoef, strike blocks
-    uint64_t n_pay = 0, n_dens = 0, n_pm = 0;
-    hexo::SwiftTotals tot{0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t i = 0; i < n; ++i) {
-        const hexo_swift_grid& g = grids[i];
-        hexo::DevSwift& R = recs[i];
+        R.strike_off = strike_off[idx[i]];
+        R.out_off = strike_off[idx[i]];
         R.exp2_m = (double)g.exp2_m;
         R.sqrt_exp2_m = g.sqrt_exp2_m;
         R.lower = g.lower;
@@ -280,7 +225,6 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
         R.k1 = g.k1;
         R.k2 = g.k2;
         R.J = g.J;
-        R.log2_2J = 1u + (uint32_t)__builtin_ctz(g.J);
         // one twiddle table per distinct J
         size_t t = 0;
         while (t < tables.size() && tables[t].J != g.J) ++t;
@@ -294,39 +238,31 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
         R.dens_off = n_dens;
         R.pm_off = n_pm;
         const uint64_t nk = (uint64_t)((int64_t)g.k2 - (int64_t)g.k1 + 1);
-        const bool fft = g.J <= hexo::kSwiftFftMaxJ;
-        if (fft) {
-            fft_chains.push_back(i);
-            tot.fft_lds_bytes = std::max(tot.fft_lds_bytes, (uint32_t)(sizeof(hexo::Cplx) * 2 * g.J));
-        } else {
-            tot.dens += nk;
-            tot.dcoef += g.J;
-        }
+        tot.dens += nk;
         n_pay += g.J;
         n_dens += nk;
         n_pm += (uint64_t)rows * g.J;
         tot.j += g.J;
-        tot.sblocks += (reqs[i].n_strikes + hexo::kSwiftStrikeBlock - 1) / hexo::kSwiftStrikeBlock;
+        for (uint32_t o = 0; o < q.n_strikes; o += hexo::kSwiftStrikeBlock) {
+            blk_chain.push_back(i);
+            blk_strike.push_back(o);
+        }
         ends[i] = tot.j;
         ends[n + i] = tot.dens;
-        ends[2 * (size_t)n + i] = tot.dcoef;
-        ends[3 * (size_t)n + i] = tot.sblocks;
     }
-    tot.n_fft = (uint32_t)fft_chains.size();
     std::vector<uint64_t> tab_end(tables.size());
     for (size_t t = 0; t < tables.size(); ++t) tab_end[t] = tables[t].off + 4ull * tables[t].J;
     const uint32_t n_tab = (uint32_t)tables.size();
-    const size_t b_recs = align(sizeof(hexo::DevSwift) * n), b_tabs = align(sizeof(hexo::SwiftTable) * n_tab),
-                 b_tabend = align(8 * (size_t)n_tab), b_fft = align(4 * fft_chains.size()),
-                 b_ends = align(sizeof(uint64_t) * 4 * (size_t)n), b_tw = align(16 * tot.tw),
-                 b_pay = align(16 * n_pay), b_dens = align(8 * n_dens), b_coeff = align(16 * n_pay),
-                 b_pm = align(16 * n_pm), b_prices = align(8 * n_strk), b_grads = grads ? align(40 * n_strk) : 0;
-    const size_t in_bytes = b_recs + b_tabs + b_tabend + b_fft + b_ends;
-    // device: [tables | strikes | work arrays]; pinned stage: [tables | prices | grads]
+    const size_t b_strk = align(8 * n_strk), b_recs = align(sizeof(hexo::DevSwift) * n),
+                 b_tabs = align(sizeof(hexo::SwiftTable) * n_tab), b_tabend = align(8 * (size_t)n_tab),
+                 b_ends = align(sizeof(uint64_t) * 2 * (size_t)n), b_blk = align(4 * blk_chain.size()), b_tw = align(16 * tot.tw), b_pay = align(16 * n_pay),
+                 b_dens = align(8 * n_dens), b_coeff = align(16 * n_pay), b_pm = align(16 * n_pm);
+    const size_t in_bytes = b_recs + b_tabs + b_tabend + b_ends + 2 * b_blk;
+    // device: [tables | strikes | work arrays]
     const size_t total = in_bytes + b_strk + b_tw + b_pay + b_dens + b_coeff + b_pm;
-    if (!ctx->swift_host.reserve(in_bytes + b_prices + b_grads)) return fail(HEXO_ERR_NOMEM, "hipHostMalloc failed");
+    if (!ctx->swift_large_host.reserve(in_bytes)) return ctx->set_error(HEXO_ERR_NOMEM, "hipHostMalloc failed");
     if (int rc = grow_device(ctx, ctx->swift_dev, ctx->swift_dev_bytes, total)) return rc;
-    unsigned char* host = reinterpret_cast<unsigned char*>(ctx->swift_host.p);
+    unsigned char* host = reinterpret_cast<unsigned char*>(ctx->swift_large_host.p);
     std::memset(host, 0, in_bytes);
     size_t off = 0;
     std::memcpy(host + off, recs.data(), sizeof(hexo::DevSwift) * n);
@@ -335,9 +271,11 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
     off += b_tabs;
     std::memcpy(host + off, tab_end.data(), 8 * (size_t)n_tab);
     off += b_tabend;
-    if (!fft_chains.empty()) std::memcpy(host + off, fft_chains.data(), 4 * fft_chains.size());
-    off += b_fft;
-    std::memcpy(host + off, ends.data(), sizeof(uint64_t) * 4 * (size_t)n);
+    std::memcpy(host + off, ends.data(), sizeof(uint64_t) * 2 * (size_t)n);
+    off += b_ends;
+    std::memcpy(host + off, blk_chain.data(), 4 * blk_chain.size());
+    off += b_blk;
+    std::memcpy(host + off, blk_strike.data(), 4 * blk_strike.size());
     unsigned char* dev = reinterpret_cast<unsigned char*>(ctx->swift_dev);
     hexo::SwiftArgs a{};
     off = 0;
@@ -349,14 +287,17 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
     off += b_tabs;
     a.tab_end = reinterpret_cast<const uint64_t*>(dev + off);
     off += b_tabend;
-    a.fft_chains = reinterpret_cast<const uint32_t*>(dev + off);
-    off += b_fft;
     const uint64_t* d_ends = reinterpret_cast<const uint64_t*>(dev + off);
     a.j_end = d_ends;
     a.dens_end = d_ends + n;
-    a.dcoef_end = d_ends + 2 * (size_t)n;
-    a.sblk_end = d_ends + 3 * (size_t)n;
     off += b_ends;
+    a.block_chain = reinterpret_cast<const uint32_t*>(dev + off);
+    off += b_blk;
+    a.block_strike = reinterpret_cast<const uint32_t*>(dev + off);
+    a.n_blocks = (uint32_t)blk_chain.size();
+    a.strike_block = hexo::kSwiftStrikeBlock;
+    a.split_rows = true;
+    off += b_blk;
     double* d_strikes = reinterpret_cast<double*>(dev + off);
     a.strikes = d_strikes;
     off += b_strk;
@@ -369,14 +310,186 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
     a.coeff = reinterpret_cast<hexo::Cplx*>(dev + off);
     off += b_coeff;
     a.pm = reinterpret_cast<hexo::Cplx*>(dev + off);
-    // the contraction writes the results straight into the pinned stage
-    double* h_prices = reinterpret_cast<double*>(host + in_bytes);
-    double* h_grads = reinterpret_cast<double*>(host + in_bytes + b_prices);
     a.prices = h_prices;
-    a.grads = grads ? h_grads : nullptr;
-    ok = hexo::launch_swift_stage(host, dev, in_bytes, h_strikes, d_strikes, b_strk, st) == hipSuccess &&
-         hexo::launch_swift(a, tot, st) == hipSuccess && hipStreamSynchronize(st) == hipSuccess;
-    if (!ok) return fail(HEXO_ERR_HIP, "SWIFT launch failed");
+    a.grads = h_grads;
+    if (hexo::launch_swift_stage(host, dev, in_bytes, h_strikes, d_strikes, b_strk, st) != hipSuccess ||
+        hexo::launch_swift_large(a, tot, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
+        (void)hipStreamSynchronize(st);
+        return ctx->set_error(HEXO_ERR_HIP, "SWIFT launch failed");
+    }
+    return HEXO_OK;
+}
+
+}  // namespace
+
+extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, uint32_t n, double* prices, double* grads,
+                                hexo_swift_grid* grids_used) {
+    if (!ctx) return HEXO_ERR_INVALID;
+    if (!reqs || !prices || n == 0) return ctx->set_error(HEXO_ERR_INVALID, "requests and prices must be non-NULL");
+    std::string err;
+    std::vector<uint64_t> strike_off(n);
+    uint64_t n_strk = 0, n_blocks = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        int rc = check_chain(reqs[i], err);
+        if (!rc && (reqs[i].flags & HEXO_SWIFT_FIXED_GRID)) rc = check_grid(reqs[i].grid, err);
+        if (rc) return ctx->set_error(rc, "swift request " + std::to_string(i) + ": " + err);
+        strike_off[i] = n_strk;
+        n_strk += reqs[i].n_strikes;
+        n_blocks += (reqs[i].n_strikes + hexo::kSwiftStrikeBlock - 1u) / hexo::kSwiftStrikeBlock;
+    }
+    if (n_blocks >= (1ull << 31)) return ctx->set_error(HEXO_ERR_INVALID, "too many strikes in one call");
+    std::lock_guard<std::recursive_mutex> lock(ctx->mu);
+    if (hipSetDevice(ctx->device) != hipSuccess) return ctx->set_error(HEXO_ERR_HIP, "hipSetDevice failed");
+    auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    hipStream_t st = ctx->stream;
+    // The kernels read their inputs from and write the grids and results to two fine-grained pinned
+    // stages, in place: [strikes | chains | chain order] and [grids | prices | gradients].
+    const size_t b_strk = align(8 * n_strk), b_chain = align(sizeof(hexo::SwiftChainIn) * n), b_blk = align(4 * n_blocks);
+    const size_t b_grid = align(sizeof(hexo::SwiftGridOut) * n), b_prices = align(8 * n_strk);
+    if (!ctx->swift_in_host.reserve(b_strk + b_chain + 4 * (size_t)n) ||
+        !ctx->swift_host.reserve(b_grid + b_prices + (grads ? 40 * n_strk : 0)))
+        return ctx->set_error(HEXO_ERR_NOMEM, "hipHostMalloc failed");
+    unsigned char* in = reinterpret_cast<unsigned char*>(ctx->swift_in_host.p);
+    unsigned char* out = reinterpret_cast<unsigned char*>(ctx->swift_host.p);
+    double* h_strikes = reinterpret_cast<double*>(in);
+    hexo::SwiftChainIn* chains = reinterpret_cast<hexo::SwiftChainIn*>(in + b_strk);
+    uint32_t* order = reinterpret_cast<uint32_t*>(in + b_strk + b_chain);
+    hexo::SwiftGridOut* gout = reinterpret_cast<hexo::SwiftGridOut*>(out);
+    double* h_prices = reinterpret_cast<double*>(out + b_grid);
+    double* h_grads = grads ? reinterpret_cast<double*>(out + b_grid + b_prices) : nullptr;
+    for (uint32_t i = 0; i < n; ++i) {
+        const hexo_swift_request& q = reqs[i];
+        std::memcpy(h_strikes + strike_off[i], q.strikes, 8 * q.n_strikes);
+        hexo::SwiftChainIn& c = chains[i];
+        c = hexo::SwiftChainIn{{q.v0, q.theta, q.rho, q.kappa, q.sigma}, q.T, q.r, q.S0, q.trunc, std::exp(-q.r * q.T),
+                               strike_off[i], 0, q.n_strikes, (q.flags & HEXO_SWIFT_FIXED_GRID) ? 1u : 0u, q.grid};
+    }
+    // More chains than CUs: by size, the longest transforms first (J ranges over a factor of 32 in a
+    // calibration batch, and one of 4,096 begun last holds up the rest), and those that will not
+    // exceed kSwiftSmallJ several to a CU. The others' chain of kernels is as long as the rest of the
+    // batch takes, so it runs beside it on a stream of its own.
+    const bool sorted = n > (uint32_t)ctx->prop.multiProcessorCount;
+    uint32_t n_big = n;
+    if (sorted) {
+        std::vector<double> size(n);
+        for (uint32_t i = 0; i < n; ++i) {
+            size[i] = size_estimate(reqs[i]);
+            order[i] = i;
+        }
+        std::stable_sort(order, order + n, [&](uint32_t x, uint32_t y) { return size[x] > size[y]; });
+        // The estimate is within a factor of 2 of J / 1.3 for nearly all: of 6,000 calibration chains
+        // none with J = 2,048 was below 678. One that is after all runs once more (below).
+        n_big = (uint32_t)(std::lower_bound(order, order + n, 630.0, [&](uint32_t x, double v) { return size[x] >= v; }) - order);
+    }
+    auto fail = [&](int code, const std::string& msg) {
+        // drain what was queued before the pinned stages are reused
+        (void)hipStreamSynchronize(st);
+        if (ctx->swift_stream) (void)hipStreamSynchronize(ctx->swift_stream);
+        return ctx->set_error(code, msg);
+    };
+    if (!ctx->swift_roots) {
+        if (hipMalloc(&ctx->swift_roots, sizeof(hexo::Cplx) * 4 * hexo::kSwiftFftMaxJ) != hipSuccess) {
+            ctx->swift_roots = nullptr;
+            return ctx->set_error(HEXO_ERR_NOMEM, "hipMalloc failed");
+        }
+        // (read on both streams, so it has to be complete)
+        if (hexo::launch_swift_roots(static_cast<hexo::Cplx*>(ctx->swift_roots), st) != hipSuccess ||
+            hipStreamSynchronize(st) != hipSuccess) {
+            (void)hipFree(ctx->swift_roots);
+            ctx->swift_roots = nullptr;
+            return fail(HEXO_ERR_HIP, "SWIFT launch failed");
+        }
+    }
+    if (n_big && n_big < n && !ctx->swift_stream &&
+        hipStreamCreateWithFlags(&ctx->swift_stream, hipStreamNonBlocking) != hipSuccess) {
+        ctx->swift_stream = nullptr;
+        return ctx->set_error(HEXO_ERR_HIP, "hipStreamCreate failed");
+    }
+    // Work arrays of each class for a pass of up to 256 or 1,024 chains, each chain with room for the
+    // largest J of its class: no second look at J, and the two streams share nothing that is written.
+    const uint32_t rows = grads ? 6u : 1u;
+    constexpr uint32_t kBigPass = 256, kSmallPass = 1024;
+    const size_t row_bytes[2] = {sizeof(hexo::Cplx) * hexo::kSwiftFftMaxJ * std::min(n, kBigPass),
+                                 n_big < n ? sizeof(hexo::Cplx) * hexo::kSwiftSmallJ * kSmallPass : 0};
+    const size_t b_recs = align(sizeof(hexo::DevSwift) * kSmallPass);
+    if (int rc = grow_device(ctx, ctx->swift_dev, ctx->swift_dev_bytes,
+                             b_strk + 2 * b_blk + 2 * b_recs + (row_bytes[0] + row_bytes[1]) * (1 + rows)))
+        return rc;
+    unsigned char* dev = reinterpret_cast<unsigned char*>(ctx->swift_dev);
+    double* dev_strikes = reinterpret_cast<double*>(dev);
+    uint32_t* block_chain = reinterpret_cast<uint32_t*>(dev + b_strk);
+    uint32_t* block_strike = reinterpret_cast<uint32_t*>(dev + b_strk + b_blk);
+    // one class of chains, order[k0 .. k1), its contraction workgroups numbered from blk on
+    auto run = [&](int small, uint32_t k0, uint32_t k1, uint32_t& blk, hipStream_t s) {
+        // Two strikes a thread in the contraction where one would already fill the device (2 workgroups
+        // a CU) and most of the second ones exist; not for long chains, which are bound by their own
+        // serial sums. 1,000 chains of J = 512 and 64 strikes with gradients: 107 us instead of 147.
+        const bool two = small && n_blocks > 2ull * ctx->prop.multiProcessorCount && n_strk > 16ull * n;
+        hexo::SwiftChainArgs c{};
+        c.chains = chains;
+        c.strikes = h_strikes;
+        c.roots = static_cast<const hexo::Cplx*>(ctx->swift_roots);
+        c.grids = gout;
+        c.dev_strikes = dev_strikes;
+        c.block_chain = block_chain;
+        c.block_strike = block_strike;
+        c.recs = reinterpret_cast<hexo::DevSwift*>(dev + b_strk + 2 * b_blk + small * b_recs);
+        c.coeff = reinterpret_cast<hexo::Cplx*>(dev + b_strk + 2 * b_blk + 2 * b_recs + (small ? row_bytes[0] * (1 + rows) : 0));
+        c.max_J = small ? hexo::kSwiftSmallJ : hexo::kSwiftFftMaxJ;
+        c.rows = rows;
+        c.strike_block = two ? hexo::kSwiftStrikeBlock2 : hexo::kSwiftStrikeBlock;
+        hexo::SwiftArgs a{};
+        a.reqs = c.recs;
+        a.strikes = dev_strikes;
+        a.strike_block = c.strike_block;
+        a.split_rows = !small && sorted;
+        a.coeff = c.coeff;
+        a.pm = c.coeff + row_bytes[small] / sizeof(hexo::Cplx);
+        a.prices = h_prices;
+        a.grads = h_grads;
+        for (uint32_t k = k0, m; k < k1; k += m) {
+            m = std::min(k1 - k, small ? kSmallPass : kBigPass);
+            const uint32_t b0 = blk;
+            for (uint32_t i = k; i < k + m; ++i) {
+                hexo::SwiftChainIn& q = chains[sorted ? order[i] : i];
+                q.block_off = blk;
+                blk += (q.n_strikes + c.strike_block - 1u) / c.strike_block;
+            }
+            c.order = sorted ? order + k : nullptr;
+            c.n_req = a.n_req = m;
+            a.block_chain = block_chain + b0;
+            a.block_strike = block_strike + b0;
+            a.n_blocks = blk - b0;
+            if (hexo::launch_swift_transform(c, s) != hipSuccess ||
+                hexo::launch_swift_prices(a, c.max_J, s) != hipSuccess)
+                return false;
+        }
+        return true;
+    };
+    const bool beside = n_big && n_big < n;
+    uint32_t blk = 0;
+    if (!run(0, 0, n_big, blk, beside ? ctx->swift_stream : st) || !run(1, n_big, n, blk, st) ||
+        (beside && hipStreamSynchronize(ctx->swift_stream) != hipSuccess) || hipStreamSynchronize(st) != hipSuccess)
+        return fail(HEXO_ERR_HIP, "SWIFT launch failed");
+    // chains that were larger than their class
+    uint32_t missed = 0;
+    for (uint32_t k = n_big; k < n; ++k)
+        if (gout[order[k]].status == hexo::kSwiftGridOk && gout[order[k]].g.J > hexo::kSwiftSmallJ &&
+            gout[order[k]].g.J <= hexo::kSwiftFftMaxJ)
+            order[missed++] = order[k];
+    blk = 0;
+    if (missed && (!run(0, 0, missed, blk, st) || hipStreamSynchronize(st) != hipSuccess))
+        return fail(HEXO_ERR_HIP, "SWIFT launch failed");
+    std::vector<hexo_swift_grid> grids(n);
+    std::vector<uint32_t> large;
+    for (uint32_t i = 0; i < n; ++i) {
+        int rc = grid_status(gout[i].status, gout[i].J_wanted, err);
+        if (!rc) rc = check_grid(grids[i] = gout[i].g, err);
+        if (rc) return ctx->set_error(rc, "swift request " + std::to_string(i) + ": " + err);
+        if (grids[i].J > hexo::kSwiftFftMaxJ) large.push_back(i);
+    }
+    if (!large.empty())
+        if (int rc = price_large(ctx, reqs, large, grids, strike_off, n_strk, h_strikes, h_prices, h_grads)) return rc;
     std::memcpy(prices, h_prices, 8 * n_strk);
     if (grads) std::memcpy(grads, h_grads, 40 * n_strk);
     if (grids_used) std::memcpy(grids_used, grids.data(), sizeof(hexo_swift_grid) * n);

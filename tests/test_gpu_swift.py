@@ -216,3 +216,60 @@ def test_swift_calibration_batch_within_conditioning(ctx, oracle):
         assert np.abs(p - op).max() <= 1e-11 * ch.S0 + 8 * cond
         assert np.abs(g - og).max() <= 1e-10 * ch.S0 + 64 * cond * (1 + np.abs(og).max() / ch.S0)
     say("  max |gpu - oracle| / (eps S e^upper):", worst)
+
+
+@pytest.mark.parametrize("J", [1, 2, 4, 8, 32, 64, 256, 512, 1024, 2048, 4096, 8192])
+def test_swift_every_transform_size(ctx, oracle, J):
+    """Every transform length in LDS (both parities of log2, one to sixteen chunks of the pricing
+    matrix) and the first by direct sums, against the oracle's direct DFTs
+    with the tolerance of its dynamic grids; a chain gives the same bits alone, without gradients
+    and beside others of every strike-block shape (1-130 strikes)."""
+    say("gpu swift transform size", J)
+    kw = dict(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, T=1.0, r=0.02)
+    if J >= 256:  # the chain's own range, oversampled
+        g = list(H.swift_grid(H.SwiftChain(**kw, strikes=[80.0, 120.0])))[:7]
+        assert g[6] - g[5] + 1 <= 4 * J
+    else:  # a range of 4 J wavelets at scale 1
+        g = [1, 2, 2 ** 0.5, -0.75, 0.75, -2 * J, 2 * J - 1]
+    chains = [H.SwiftChain(**kw, strikes=np.linspace(85.0, 115.0, n), grid=g + [J])
+              for n in (1, 15, 16, 17, 32, 33, 64, 65, 130)]
+    res = ctx.swift_price(chains, grads=True)
+    for ch, (p, gr, _) in zip(chains, res):
+        op, _, og = oracle.swift_price([ch.v0, ch.theta, ch.rho, ch.kappa, ch.sigma], ch.S0, ch.r, ch.T, ch.strikes,
+                                       swift_params=ch.grid, grads=True)
+        np.testing.assert_allclose(p, op, rtol=1e-10, atol=1e-11 * ch.S0)
+        np.testing.assert_allclose(gr, og, rtol=1e-9, atol=1e-10 * ch.S0)
+        for alone in (ctx.swift_price([ch], grads=True)[0], ctx.swift_price([ch])[0]):
+            np.testing.assert_array_equal(alone[0], p)
+            if alone[1] is not None:
+                np.testing.assert_array_equal(alone[1], gr)
+
+
+def test_swift_call_beyond_the_compute_units(ctx):
+    """A call of more chains than compute units sorts them by their expected transform length, runs the
+    long ones beside the others and repeats those that turn out longer than expected (here: strikes
+    far out, which the expectation does not look at). Every chain of the device sums has the bits
+    that it has alone, with and without gradients."""
+    rng = np.random.default_rng(5)
+    kw = dict(v0=0.04, theta=0.05, rho=-0.6, kappa=1.5, S0=100.0, r=0.02)
+    g = list(H.swift_grid(H.SwiftChain(**kw, sigma=0.3, T=1.0, strikes=[80.0, 120.0])))[:7]
+    special = [H.SwiftChain(**kw, sigma=0.3, T=1.0, strikes=np.linspace(85.0, 115.0, 33), grid=g + [J])
+               for J in (512, 1024, 2048, 4096, 8192)]
+    special += [H.SwiftChain(**kw, sigma=s, T=T, strikes=np.array([1e-3, 90.0, 100.0, 110.0, 1e6]))
+                for s, T in ((0.2, 1.0), (0.5, 2.0), (0.8, 0.5))]
+    special += [H.SwiftChain(**kw, sigma=0.8, T=T, strikes=np.linspace(60.0, 150.0, n)) for T, n in ((0.05, 16), (5.0, 70))]
+    chains = [H.SwiftChain(**kw, sigma=float(rng.uniform(0.2, 0.8)), T=float(rng.choice([0.1, 0.5, 1.0, 3.0])),
+                           strikes=np.sort(rng.uniform(70.0, 130.0, int(rng.integers(1, 41))))) for _ in range(600)]
+    for k, c in enumerate(special):
+        chains.insert(61 * k, c)
+    say("gpu swift call of", len(chains), "chains")
+    J = np.array([H.swift_grid(c)[7] if c.grid is None else c.grid[7] for c in chains])
+    assert (J > 1024).any() and (J <= 1024).any()
+    for grads in (True, False):
+        res = ctx.swift_price(chains, grads=grads)
+        for k in [61 * k for k in range(len(special))] + list(range(0, len(chains), 7)):
+            p, gr, used = ctx.swift_price([chains[k]], grads=grads)[0]
+            np.testing.assert_array_equal(res[k][0], p)
+            assert res[k][2] == used
+            if grads:
+                np.testing.assert_array_equal(res[k][1], gr)
