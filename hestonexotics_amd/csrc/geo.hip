@@ -15,11 +15,11 @@
 // starting at u0 (the integral's remaining tail is then below 1e-15).
 //
 // Work items are (request, expiry, block of <= 64 strikes), in up to three rounds. Pass 1 of a
-// round evaluates the next p0 panels of every unconverged item at once, one wavefront per panel
+// round evaluates the next p0 panels of every unconverged item at once, one workgroup per panel
 // (lane q: node q, a recursion over the expiry's grid, a few hundred to a few thousand steps;
-// lane i: strike i's panel sum over the 64 nodes in node order), plus E[e^L] in the first round;
+// lane i: strike i's panel sum over the 64 nodes in a fixed order), plus E[e^L] in the first round;
 // p0 is the host's estimate of where the characteristic function has decayed. Pass 2 gives each
-// item one wavefront: lane i adds strike i's panel sums in panel order, keeps them for the next
+// item one workgroup: lane i adds strike i's panel sums in panel order, keeps them for the next
 // round if the decay was not reached, and in the last round evaluates further panels itself;
 // every price is therefore the same fixed-order sum whatever p0 is. Runs once per batch, before
 // the path kernels.
@@ -28,46 +28,97 @@
 #include "cplx_device.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
+#include "math_f64.hpp"
 
 namespace hexo {
 namespace {
 
 constexpr double kPi = 3.14159265358979323846;
-constexpr int kGeoWaves = 4;  // wavefronts per workgroup
+// The recursion over an expiry's grid is one chain of steps, and 87 panels (one expiry) leave a wavefront
+// alone on its SIMD, where it issues an instruction every 7 cycles or so: 0.9 us a step when one
+// wavefront did all of it. Most of a step does not depend on the running B: a is known from the
+// weights, and with it beta, d, B-, e and Z below; and log(1 + z) only adds to A. So 7 wavefronts
+// prepare the steps of a chunk (one each) and take the logarithms of an earlier one, and the eighth
+// runs the rest, B' = B- - (B- - B) e / (1 + z): 35 instructions in place of 500. 252 steps, one
+// expiry, 87 panels: 450 -> 106 us for the first pass; 2,000 steps 2.9 -> 0.65 ms; 40 expiries, where
+// the chip is full either way, 3.6 -> 2.9 ms.
+constexpr int kGeoHelpers = 7;
+constexpr int kGeoWaves = kGeoHelpers + 1;
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+struct GeoShared {
+    Cplx pre[2][kGeoHelpers][3][64];  // B-, e, Z of a chunk's steps, lane by lane
+    Cplx z[2][kGeoHelpers][64];
+    Cplx A[kGeoHelpers][64];
+    double node[3][64];  // weighted phi and u of a panel's nodes
+    double part[kGeoWaves][64];
+    double mag;
+};
 
 __device__ __forceinline__ double cabs_(Cplx z) { return hypot(z.re, z.im); }
+__device__ __forceinline__ double norm2(Cplx z) { return __builtin_fma(z.re, z.re, z.im * z.im); }
+// z / w, inv_w2 = 1 / |w|^2: the operands here are far from the ends of the range
+__device__ __forceinline__ Cplx div_by(Cplx z, Cplx w, double inv_w2) { return inv_w2 * (z * conj(w)); }
 
-// phi(s) over points 0..n of pts = (t_j, v_j) pairs.
+// phi(s) over points 0..n of pts = (t_j, v_j) pairs, by a whole workgroup, lane by lane; wavefront
+// kGeoHelpers returns it.
 // With beta = kappa - rho sigma a, d = sqrt(beta^2 - sigma^2 (a^2 - a)), the stable root
-// B- = (a^2 - a)/(beta + d) (or (beta - d)/sigma^2 when beta + d is the smaller) and
-// e = e^{-d tau}, om = 1 - e:
-//   B(tau) = B- + (B - B-) e 2d / D,   D = (beta + d - sigma^2 B) - sigma^2 (B- - B) e,
-//   A(tau) = A + r a tau + kappa theta (B- tau - (2/sigma^2) log(1 + sigma^2 (B- - B) om / (2d))).
-__device__ Cplx geo_cf(const DevReq& R, const double* pts, uint32_t n, Cplx s) {
-    const double rho = R.rho, kap = R.kappa, sig = R.sigma, s2 = sig * sig, kth = R.kappa * R.theta;
-    Cplx a = cx(0.0), A = cx(0.0), B = cx(0.0);
-    for (uint32_t j = n; j >= 1; --j) {
-        const double tau = pts[2 * j] - pts[2 * (j - 1)];
-        a = a + pts[2 * j + 1] * s;
-        const Cplx bt = cx(kap) - (rho * sig) * a;
-        const Cplx q = a * a - a;
-        const Cplx d = csqrt(bt * bt - s2 * q);
-        const Cplx bp = bt + d, bm = bt - d;
-        const Cplx Bm = cabs_(bp) >= cabs_(bm) ? q / bp : (1.0 / s2) * bm;
-        const Cplx om = -1.0 * cexpm1(-tau * d);
-        const Cplx e = cx(1.0) - om;
-        const Cplx D = (bp - s2 * B) - s2 * ((Bm - B) * e);
-        const Cplx Bn = Bm + ((B - Bm) * e) * ((2.0 * d) / D);
-        const Cplx z = (s2 * ((Bm - B) * om)) / (2.0 * d);
-        A = A + (R.r_drift * tau) * a + kth * (tau * Bm - (2.0 / s2) * clog1p(z));
-        B = Bn;
+// B- = (a^2 - a)/(beta + d) (or (beta - d)/sigma^2 when beta + d is the smaller),
+// e = e^{-d tau}, Z = sigma^2 (1 - e) / (2d) and z = Z (B- - B):
+//   B(tau) = B- - (B- - B) e / (1 + z),   A(tau) = A + r a tau + kappa theta (B- tau - (2/sigma^2) log(1 + z)).
+__device__ Cplx geo_cf(const DevReq& R, const double* pts, uint32_t n, Cplx s, GeoShared& sh, int w, int lane) {
+    const double s2 = R.sigma * R.sigma, kth = R.kappa * R.theta, rs = R.rho * R.sigma, kap = R.kappa;
+    const double k2 = 2.0 * kth / s2;
+    const uint32_t chunks = (n + kGeoHelpers - 1) / kGeoHelpers;
+    Cplx A = cx(0.0), B = cx(0.0);
+    double S = 0.0;     // sum of the weights from point n down to jn + 1
+    uint32_t jn = n;
+    if (w == kGeoHelpers) __builtin_amdgcn_s_setprio(2);  // the others wait for it
+    for (uint32_t it = 0; it < chunks + 2; ++it) {
+        if (w < kGeoHelpers) {
+            if (it >= 2 && (it - 2) * kGeoHelpers + w < n) A = A - k2 * clog1p(sh.z[it & 1][w][lane]);
+            const uint32_t i = it * kGeoHelpers + w;
+            if (i < n) {
+                const uint32_t j = n - i;  // the step from point j to j - 1
+                for (; jn >= j; --jn) S += pts[2 * jn + 1];
+                const double tau = pts[2 * j] - pts[2 * (j - 1)];
+                const Cplx a = S * s;
+                const Cplx bt = cx(kap) - rs * a;
+                const Cplx q = a * a - a;
+                // d = principal root of d2, |d|^2 = |d2|
+                const Cplx d2 = bt * bt - s2 * q;
+                const double r = sqrt(norm2(d2));
+                const double t = sqrt(0.5 * (r + fabs(d2.re))), o = r > 0.0 ? 0.5 * div_f64(d2.im, t) : 0.0;
+                const Cplx d = d2.re >= 0.0 ? Cplx{t, o} : Cplx{fabs(o), copysign(t, d2.im)};
+                const Cplx bp = bt + d, bm = bt - d;
+                const double bp2 = norm2(bp);
+                const Cplx Bm = bp2 >= norm2(bm) ? div_by(q, bp, div_f64(1.0, bp2)) : (1.0 / s2) * bm;
+                const Cplx om = -1.0 * cexpm1(-tau * d);
+                A = A + (R.r_drift * tau) * a + (kth * tau) * Bm;
+                sh.pre[it & 1][w][0][lane] = Bm;
+                sh.pre[it & 1][w][1][lane] = cx(1.0) - om;
+                sh.pre[it & 1][w][2][lane] = div_by((0.5 * s2) * om, d, div_f64(1.0, r));
+            }
+        } else if (it >= 1 && it <= chunks) {
+            const uint32_t m = min((uint32_t)kGeoHelpers, n - (it - 1) * kGeoHelpers);
+#pragma unroll
+            for (uint32_t h = 0; h < (uint32_t)kGeoHelpers; ++h) {
+                if (h < m) {
+                    const Cplx Bm = sh.pre[(it - 1) & 1][h][0][lane];
+                    const Cplx y = Bm - B, z = sh.pre[(it - 1) & 1][h][2][lane] * y;
+                    const Cplx v = cx(1.0 + z.re, z.im);
+                    sh.z[(it - 1) & 1][h][lane] = z;
+                    B = Bm - div_by(y * sh.pre[(it - 1) & 1][h][1][lane], v, div_f64(1.0, norm2(v)));
+                }
+            }
+        }
+        __syncthreads();
     }
+    if (w < kGeoHelpers) sh.A[w][lane] = A;
+    __syncthreads();
+    if (w < kGeoHelpers) return cx(0.0);
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int h = 0; h < kGeoHelpers; ++h) A = A + sh.A[h][lane];
     return cexp(A + R.v0 * B);
 }
 
@@ -89,10 +140,10 @@ __device__ __forceinline__ uint32_t find_item(const uint32_t* end, uint32_t n, u
     return lo;
 }
 
-// Panel p of an item, by one wavefront: lane q evaluates node q, u_q = (p + (x_q + 1)/2) h, and
-// phi(1/2 - i u_q) weighted by w_q (h/2) / (u_q^2 + 1/4); the 64 values go through LDS (sh: this
-// wave's 3 x 64 doubles) and lane i returns strike i's panel sum, node by node, of
-// Re(e^{i u_q k_i} weighted phi). *mag is the wave's max |phi| over the panel.
+// Panel p of an item, by one workgroup: lane q evaluates node q, u_q = (p + (x_q + 1)/2) h, and
+// phi(1/2 - i u_q) weighted by w_q (h/2) / (u_q^2 + 1/4); then lane i of each wavefront sums strike
+// i's Re(e^{i u_q k_i} weighted phi) over 8 nodes, node by node, and wavefront kGeoHelpers adds and
+// returns the eight sums in order, with the maximum of |phi| over the panel in *mag.
 // Panel 0 holds the integrand's 1/(u^2 + 1/4) peak at u = 0, which 64 nodes integrate to 1e-13
 // over [0, 16] but only to 1e-4 over [0, 120]: it is summed as n_sub = min(64, ceil(h / 16))
 // sub-panels of 64 nodes (wave-uniform, in order). The other panels keep width h.
@@ -100,28 +151,37 @@ __device__ __forceinline__ uint32_t first_panel_parts(double h) {
     return (uint32_t)fmin(64.0, ceil(h / 16.0));
 }
 
-__device__ double panel_sum(const GeoArgs& a, const DevGeo& G, const DevReq& R, const double* pts, uint32_t p, int lane,
-                            double k, bool has_k, double (*sh)[64], double* mag) {
+__device__ double panel_sum(const GeoArgs& a, const DevGeo& G, const DevReq& R, const double* pts, uint32_t p, int w,
+                            int lane, double k, bool has_k, GeoShared& sh, double* mag) {
     const uint32_t n_sub = p == 0 ? first_panel_parts(G.h) : 1u;
     const double hs = G.h / (double)n_sub;
+    constexpr int kNodes = 64 / kGeoWaves;  // per wavefront
     double sum = 0.0, mg = 0.0;
     for (uint32_t j = 0; j < n_sub; ++j) {
         const double u = ((double)(p + j) + 0.5 * (a.gl[lane] + 1.0)) * hs;  // p = 0 or j = 0
-        const Cplx ph = geo_cf(R, pts, G.n_pts, cx(0.5, -u));
-        const double f = 0.5 * hs * a.gl[64 + lane] / (u * u + 0.25);
-        sh[0][lane] = f * ph.re;
-        sh[1][lane] = f * ph.im;
-        sh[2][lane] = u;
-        mg = fmax(mg, wave_max(cabs_(ph)));
-        wave_sync_lds();
+        const Cplx ph = geo_cf(R, pts, G.n_pts, cx(0.5, -u), sh, w, lane);  // ends the use of node and part before
+        if (w == kGeoHelpers) {
+            const double f = 0.5 * hs * a.gl[64 + lane] / (u * u + 0.25);
+            sh.node[0][lane] = f * ph.re;
+            sh.node[1][lane] = f * ph.im;
+            sh.node[2][lane] = u;
+            mg = fmax(mg, wave_max(cabs_(ph)));
+        }
+        __syncthreads();
+        double part = 0.0;
         if (has_k) {
-            for (int q = 0; q < 64; ++q) {
+            for (int q = w * kNodes; q < (w + 1) * kNodes; ++q) {
                 double sn, cs;
-                sincos(sh[2][q] * k, &sn, &cs);
-                sum += cs * sh[0][q] - sn * sh[1][q];
+                sincos(sh.node[2][q] * k, &sn, &cs);
+                part += cs * sh.node[0][q] - sn * sh.node[1][q];
             }
         }
-        wave_sync_lds();  // sh is rewritten by the next sub-panel or panel
+        sh.part[w][lane] = part;
+        __syncthreads();
+        if (w == kGeoHelpers) {
+#pragma unroll
+            for (int v = 0; v < kGeoWaves; ++v) sum += sh.part[v][lane];
+        }
     }
     *mag = mg;
     return sum;
@@ -141,14 +201,13 @@ __device__ __forceinline__ void strike_of(const GeoArgs& a, const DevGeo& G, int
 constexpr int kGeoState = 64 + 4;
 constexpr int kGeoRounds = 3;  // parallel rounds of p0 panels before the serial continuation
 
-// Pass 1 of round r: every wavefront evaluates one panel of one unconverged item (round r covers
+// Pass 1 of round r: every workgroup evaluates one panel of one unconverged item (round r covers
 // that item's panels done .. done + p0 - 1) and stores each strike's panel sum; in the first round the
-// item's last wavefront evaluates E[e^L] instead.
-__global__ __launch_bounds__(256) void k_geo_panels(GeoArgs a, uint32_t round) {
-    __shared__ double sh[kGeoWaves][3][64];
-    const int w = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63u);
-    const uint32_t wv = blockIdx.x * kGeoWaves + (uint32_t)w;
-    if (wv >= a.n_waves) return;  // whole wavefronts only
+// item's last workgroup evaluates E[e^L] instead.
+__global__ __launch_bounds__(64 * kGeoWaves) void k_geo_panels(GeoArgs a, uint32_t round) {
+    __shared__ GeoShared sh;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
+    const uint32_t wv = blockIdx.x;
     const uint32_t item = __builtin_amdgcn_readfirstlane(find_item(a.wave_end, a.n_items, wv));
     const DevGeo& G = a.items[item];
     const DevReq& R = a.reqs[G.req];
@@ -160,8 +219,8 @@ __global__ __launch_bounds__(256) void k_geo_panels(GeoArgs a, uint32_t round) {
         if (j == G.p0 || st[66] != 0.0) return;  // E[e^L] is known; or the item has converged
         base = (uint32_t)st[65];
     } else if (j == G.p0) {
-        const Cplx e1 = geo_cf(R, pts, G.n_pts, cx(1.0));
-        if (lane == 0) a.panel_max[wv] = e1.re;
+        const Cplx e1 = geo_cf(R, pts, G.n_pts, cx(1.0), sh, w, lane);
+        if (w == kGeoHelpers && lane == 0) a.panel_max[wv] = e1.re;
         return;
     }
     const uint32_t p = base + j;
@@ -169,34 +228,38 @@ __global__ __launch_bounds__(256) void k_geo_panels(GeoArgs a, uint32_t round) {
     double K, k, mag;
     bool has_k;
     strike_of(a, G, lane, K, k, has_k);
-    a.panel[(size_t)wv * 64 + (uint32_t)lane] = panel_sum(a, G, R, pts, p, lane, k, has_k, sh[w], &mag);
+    const double sum = panel_sum(a, G, R, pts, p, w, lane, k, has_k, sh, &mag);
+    if (w != kGeoHelpers) return;
+    a.panel[(size_t)wv * 64 + (uint32_t)lane] = sum;
     if (lane == 0) a.panel_max[wv] = mag;
 }
 
-// Pass 2 of round r: one wavefront per item; lane i adds strike i's panel sums in panel order up
+// Pass 2 of round r: one workgroup per item; lane i of wavefront kGeoHelpers adds strike i's panel sums in panel order up
 // to the second of the first two consecutive panels (after the first) whose |phi| stays below
 // 1e-15 u0, u0 a panel's start: beyond u0 the integrand |phi| / (u^2 + 1/4) leaves at most
 // sup|phi| / u0 to the integral, and two panels in a row guard against a dip of a non-monotone
-// |phi|. An unconverged item keeps its sums for the next round; in the last round the wavefront
+// |phi|. An unconverged item keeps its sums for the next round; in the last round the workgroup
 // evaluates further panels itself. The price is the same ordered sum whatever p0 and the number of
 // rounds are.
-__global__ __launch_bounds__(256) void k_geo_sum(GeoArgs a, uint32_t round) {
-    __shared__ double sh[kGeoWaves][3][64];
-    const int w = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63u);
-    const uint32_t item = blockIdx.x * kGeoWaves + (uint32_t)w;
-    if (item >= a.n_items) return;  // whole wavefronts only
+__global__ __launch_bounds__(64 * kGeoWaves) void k_geo_sum(GeoArgs a, uint32_t round) {
+    __shared__ GeoShared sh;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
+    const uint32_t item = blockIdx.x;
     const DevGeo& G = a.items[item];
     const DevReq& R = a.reqs[G.req];
     const double* pts = a.pts + 2 * (size_t)G.pts_begin;
     double* st = a.state + (size_t)item * kGeoState;
-    if (round > 0 && st[66] != 0.0) return;
-    double K, k;
-    bool has_k;
-    strike_of(a, G, lane, K, k, has_k);
+    // every wavefront follows the same decisions; all have read the state before it is written
+    const bool done = round > 0 && st[66] != 0.0;
     const double e1 = round == 0 ? a.panel_max[G.wave_begin + G.p0] : st[64];  // E[e^L]
     double integ = round == 0 ? 0.0 : st[lane];
     const uint32_t base = round == 0 ? 0u : (uint32_t)st[65];
     bool below = round == 0 ? false : st[67] != 0.0;  // the previous panel was below the bound
+    __syncthreads();
+    if (done) return;
+    double K, k;
+    bool has_k;
+    strike_of(a, G, lane, K, k, has_k);
     bool converged = false;
     uint32_t p = base;
     for (uint32_t j = 0; j < G.p0 && p < G.max_panels && !converged; ++j, ++p) {
@@ -207,6 +270,7 @@ __global__ __launch_bounds__(256) void k_geo_sum(GeoArgs a, uint32_t round) {
     }
     const bool last = round + 1 == kGeoRounds;
     if (!converged && !last && p < G.max_panels) {
+        if (w != kGeoHelpers) return;
         st[lane] = integ;
         if (lane == 0) {
             st[64] = e1;
@@ -218,11 +282,14 @@ __global__ __launch_bounds__(256) void k_geo_sum(GeoArgs a, uint32_t round) {
     }
     for (; p < G.max_panels && !converged; ++p) {
         double mag;
-        integ += panel_sum(a, G, R, pts, p, lane, k, has_k, sh[w], &mag);
-        const bool now = p > 0 && mag < 1e-15 * (double)p * G.h;  // wave-uniform
+        integ += panel_sum(a, G, R, pts, p, w, lane, k, has_k, sh, &mag);
+        if (w == kGeoHelpers && lane == 0) sh.mag = mag;
+        __syncthreads();
+        const bool now = p > 0 && sh.mag < 1e-15 * (double)p * G.h;  // rewritten after the next panel's barriers
         converged = now && below;
         below = now;
     }
+    if (w != kGeoHelpers) return;
     if (lane == 0) st[66] = 1.0;  // later rounds skip the item
     if ((uint32_t)lane >= G.n_strikes) return;
     double price;
@@ -242,10 +309,10 @@ size_t geo_state_doubles(uint32_t n_items) { return (size_t)n_items * kGeoState;
 hipError_t launch_geo(const GeoArgs& a, hipStream_t st) {
     if (a.n_items == 0) return hipSuccess;
     for (uint32_t r = 0; r < (uint32_t)kGeoRounds; ++r) {
-        k_geo_panels<<<(a.n_waves + kGeoWaves - 1) / kGeoWaves, 64 * kGeoWaves, 0, st>>>(a, r);
+        k_geo_panels<<<a.n_waves, 64 * kGeoWaves, 0, st>>>(a, r);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        k_geo_sum<<<(a.n_items + kGeoWaves - 1) / kGeoWaves, 64 * kGeoWaves, 0, st>>>(a, r);
+        k_geo_sum<<<a.n_items, 64 * kGeoWaves, 0, st>>>(a, r);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

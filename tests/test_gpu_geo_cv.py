@@ -78,6 +78,20 @@ def test_exact_geometric_price_matches_oracle(ctx, oracle, name):
     np.testing.assert_allclose(g, o, rtol=0, atol=1e-9 * req.S0)
 
 
+@pytest.mark.parametrize("steps", [2, 6, 7, 8, 13, 14, 15, 21, 22, 50])
+def test_exact_geometric_price_at_chunk_edges(ctx, oracle, steps):
+    """Grids of fewer, as many and more steps than the 7 that the exact-price kernel prepares at a time
+    (one to eight chunks, full and ragged), two expiries, against the oracle as above."""
+    req = H.Request(**BASE, expiries=[0.6, 1.0], strikes=[[90.0, 110.0], [80.0, 100.0, 0.0]], steps=steps, n_paths=64,
+                    seed=2, r=0.02, flags=H.DRIFT)
+    say("gpu geo exact, steps", steps)
+    g = ctx.geo_asian_price(req)
+    o = oracle.geo_asian_price(req.params, req.S0, req.expiries, req.n_strikes(), req.flat_strikes(), steps=steps,
+                               r=req.r, flags=req.flags)
+    say(f"  max |gpu - oracle| / S0 = {np.abs(g - o).max() / req.S0:.2e}")
+    np.testing.assert_allclose(g, o, rtol=0, atol=1e-9 * req.S0)
+
+
 @pytest.mark.parametrize("name", sorted(geo_requests()))
 def test_fp64_control_variate_prices_equal_oracle(ctx, oracle, name):
     req = cv(geo_requests()[name], H.FP64, payoffs=H.ASIAN | H.ASIAN_GEO_CV)
