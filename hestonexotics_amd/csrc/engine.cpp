@@ -755,7 +755,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         return HEXO_ERR_HIP;
     }
     // the exact geometric prices depend on the requests only: computed once, before any run
-    if (ga.n_items && launch_geo(ga, stream) != hipSuccess) {
+    if (ga.n_items && launch_geo(ga, true, stream) != hipSuccess) {
         // the upload is in flight: the region and the (possibly shared) staging buffer are handed
         // back only once it is done
         (void)hipStreamSynchronize(stream);
@@ -768,27 +768,38 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         // variance process stays near 0 (v0 = 0 with a Feller ratio 2 kappa theta / sigma^2 near 0),
         // so the characteristic function of the geometric average's log hardly decays. The result
         // buffer is free until the first run.
-        if (hipMemcpyAsync(b->h_prices, ga.geo, sizeof(double) * n_out, hipMemcpyDeviceToHost, stream) != hipSuccess ||
-            hipStreamSynchronize(stream) != hipSuccess) {
+        auto read_back = [&] {
+            return hipMemcpyAsync(b->h_prices, ga.geo, sizeof(double) * n_out, hipMemcpyDeviceToHost, stream) == hipSuccess &&
+                   hipStreamSynchronize(stream) == hipSuccess;
+        };
+        // whether pred holds for a control-variate output of request i
+        auto any_price = [&](uint32_t i, auto pred) {
+            if (!(reqs[i].payoffs & HEXO_ASIAN_GEO_CV)) return false;
+            const uint64_t first = b->out_base[i] + n_payoffs(reqs[i].payoffs & (HEXO_ASIAN | HEXO_EUROPEAN)) * plans[i].n_opts;
+            for (uint64_t o = first; o < first + plans[i].n_opts; ++o)
+                if (pred(b->h_prices[o])) return true;
+            return false;
+        };
+        bool ok = read_back(), unfinished = false;
+        for (uint32_t i = 0; i < n && ok && !unfinished; ++i)
+            unfinished = any_price(i, [](double x) { return x == kGeoUnfinished; });
+        if (unfinished) ok = launch_geo(ga, false, stream) == hipSuccess && read_back();
+        if (!ok) {
             (void)hipStreamSynchronize(stream);
             batch_destroy(*b);
             err = "read-back of the geometric control-variate prices failed";
             return HEXO_ERR_HIP;
         }
         for (uint32_t i = 0; i < n; ++i) {
-            if (!(reqs[i].payoffs & HEXO_ASIAN_GEO_CV)) continue;
-            const uint64_t first = b->out_base[i] + n_payoffs(reqs[i].payoffs & (HEXO_ASIAN | HEXO_EUROPEAN)) * plans[i].n_opts;
-            for (uint64_t o = first; o < first + plans[i].n_opts; ++o)
-                if (std::isnan(b->h_prices[o])) {
-                    const hexo_request& q = reqs[i];
-                    err = "request " + std::to_string(i) +
-                          ": the geometric control variate's exact price did not converge (v0 " + std::to_string(q.v0) +
-                          ", Feller ratio 2 kappa theta / sigma^2 = " +
-                          std::to_string(2.0 * q.kappa * q.theta / (q.sigma * q.sigma)) +
-                          ": the variance stays near 0); price it without HEXO_ASIAN_GEO_CV";
-                    batch_destroy(*b);
-                    return HEXO_ERR_INVALID;
-                }
+            if (!any_price(i, [](double x) { return std::isnan(x); })) continue;
+            const hexo_request& q = reqs[i];
+            err = "request " + std::to_string(i) +
+                  ": the geometric control variate's exact price did not converge (v0 " + std::to_string(q.v0) +
+                  ", Feller ratio 2 kappa theta / sigma^2 = " +
+                  std::to_string(2.0 * q.kappa * q.theta / (q.sigma * q.sigma)) +
+                  ": the variance stays near 0); price it without HEXO_ASIAN_GEO_CV";
+            batch_destroy(*b);
+            return HEXO_ERR_INVALID;
         }
     }
     out = std::move(b);

@@ -20,9 +20,9 @@ hipError_t launch_paths(uint32_t precision, uint32_t ppt, PathMode mode, uint32_
 // (PathArgs.total_items tiles; partials stored per tile).
 hipError_t launch_paths_split(uint32_t precision, uint32_t n_draw, const PathArgs& a, bool mart, bool geo,
                               hipStream_t st);
-// Exact prices of the geometric control variates (geo.hip); GeoArgs.state holds
-// geo_state_doubles(n_items) doubles.
-hipError_t launch_geo(const GeoArgs& a, hipStream_t st);
+// Exact prices of the geometric control variates (geo.hip), the first round or the others for the
+// items that it left unfinished; GeoArgs.state holds geo_state_doubles(n_items) doubles.
+hipError_t launch_geo(const GeoArgs& a, bool first, hipStream_t st);
 size_t geo_state_doubles(uint32_t n_items);
 hipError_t launch_reduce(const ReduceArgs& a, uint64_t n_group_threads, uint64_t n_out_threads, hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t st);

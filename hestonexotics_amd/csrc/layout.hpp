@@ -123,12 +123,15 @@ struct DevGeo {
     uint32_t n_strikes;   // strikes of this block (<= 64)
     uint32_t opt;         // first option of the block (batch-global DevOpt index)
     uint32_t max_panels;  // bound on 64-node panels (the price is NaN if not converged by then)
-    uint32_t wave_begin;  // first wavefront of the item in the parallel panel pass
-    uint32_t p0;          // panels evaluated in parallel (that pass has p0 + 1 waves: the last one E[e^L])
+    uint32_t wave_begin;  // first workgroup of the item in the parallel panel pass
+    uint32_t p0;          // panels evaluated in parallel (that pass has p0 + 1 workgroups: the last one E[e^L])
     uint64_t out;         // geo[] index of the block's first control-variate output
     double c;             // W S0
     double h;             // width in u of one panel
 };
+
+// The exact geometric price of an item that the first round left unfinished.
+constexpr double kGeoUnfinished = -__builtin_huge_val();
 
 struct GeoArgs {
     const DevReq* reqs;
