@@ -277,6 +277,22 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
     return L;
 }
 
+// The most tiles for which a request with many outputs suits the split kernel. There the stepping wave
+// forms the payoff sums alone and stores a partial per tile, the persistent FP32 kernel's waves one per
+// pair of tiles; outputs then cost a fifth more. Persistent / split time with 1,500, 8,000, 16,000,
+// 30,000, 60,000 tiles, FP32, two payoffs (FP64 with 800, 1,600 and 3,200 tiles):
+//    64 strikes x   52 steps (2.5 outputs a step)  1.56 1.50 1.42 1.27 1.12   (1.35 1.27 1.22)
+//   200 strikes x   52 steps (7.7)                 1.37 1.23 1.17 1.00 0.93   (1.16 1.08 1.11)
+//   12 x 64 strikes x 61 steps (25)                1.23 0.98 0.88 0.83 0.81   (1.04 0.93 1.00)
+//  1000 strikes x   52 steps (38)                  1.15 0.90 0.84 0.78 0.79   (0.98 0.87 0.95)
+// Up to 256 outputs even short requests gain (64 strikes x 13 steps, 9.8 a step: 1.51 2.05 2.01 1.89
+// 1.72), since the persistent kernel's queue then sets its time.
+uint64_t split_most_tiles(const ReqPlan& p) {
+    const double per_step = (double)p.n_out / (double)p.total_steps;
+    if (p.n_out <= 256 || per_step <= 2.0) return ~0ull;
+    return per_step <= 16.0 ? 1u << 14 : p.cls == 0 ? 512u : 2048u;
+}
+
 // Drawing waves per tile of the split kernel for a class of `tiles` 64-path tiles, or 0 for the
 // persistent kernel. FP32, where the launch shape is left to the library (2 paths per thread, no
 // occupancy cap):
@@ -288,6 +304,9 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
 //    At 125,000 tiles the grid takes 1.72 ms against the persistent kernel's 1.80 and 64 uneven
 //    requests 8.6 to 8.8 ms against 8.7; at 370,000 tiles they take 25.8 ms against 25.3: there the
 //    persistent kernel's waves are full and it has no draws to carry through LDS.
+//  * up to 2^16 tiles with the geometric average, whose payoffs are more of the stepping wave's work:
+//    the grid with 64 strikes and 4, 3, 2 payoffs takes 2.35, 2.06, 1.98 ms at 125,000 tiles against
+//    2.23, 2.00, 1.97, and at 62,500 tiles 1.08, 0.99, 0.95 against 1.13, 1.04, 1.01.
 //  * up to 2,048 tiles where the stepping wave is much the longer one, leaving the drawing waves idle:
 //    the martingale correction on a variance that is mostly in the exponential branch
 //    (2 kappa theta / sigma^2 < 0.6). 1,563 tiles x 1,024 steps 0.605 ms against 0.734, 4,096 tiles
@@ -299,10 +318,12 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
 //    persistent; 50,000 paths 214, 195, 286); up to 3,328: one (k_path_fp64_split).
 //  * with the correction up to 256 tiles (1e4 paths: 223 us against 392, stiff parameters 332 against
 //    500; at 313 tiles stiff 521 against 501, at 1,563 and one drawing wave 610 against 561).
-uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, bool martingale, bool long_steps, const hexo_tuning& tun) {
+uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, uint64_t most_tiles, bool martingale, bool long_steps,
+                          const hexo_tuning& tun) {
+    if (tiles > most_tiles) return 0;
     if (cls == 0) return tiles > (martingale ? 256u : 3328u) ? 0 : tiles <= 512 ? 2 : 1;
     if (tun.paths_per_thread != 2 || tun.waves_per_simd != 0) return 0;
-    if (tiles > (long_steps ? 2048u : 1u << 17)) return 0;
+    if (tiles > (long_steps ? 2048u : class_geo(cls) ? 1u << 16 : 1u << 17)) return 0;
     return tiles <= 512 ? 2 : 1;
 }
 
@@ -377,6 +398,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint64_t n_geo_items = 0, n_geo_pts = 0, n_geo_waves = 0;
     uint32_t n_cls[kPathClasses] = {};
     uint64_t cls_tiles[kPathClasses] = {};
+    uint64_t cls_most[kPathClasses];  // split_most_tiles over the class's requests
+    std::fill(cls_most, cls_most + kPathClasses, ~0ull);
     bool cls_mart[kPathClasses] = {}, cls_long[kPathClasses] = {};  // requests with longer steps (split_draw_waves)
     for (uint32_t i = 0; i < n; ++i) {
         std::string why = validate(&reqs[i]);
@@ -403,6 +426,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         n_out += p.n_out;
         n_cls[p.cls]++;
         cls_tiles[p.cls] += p.n_tiles;
+        cls_most[p.cls] = std::min(cls_most[p.cls], split_most_tiles(p));
         const bool mart = (reqs[i].flags & HEXO_MARTINGALE) != 0;
         cls_mart[p.cls] |= mart;
         cls_long[p.cls] |= mart && 2.0 * reqs[i].kappa * reqs[i].theta < 0.6 * reqs[i].sigma * reqs[i].sigma;
@@ -413,7 +437,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint32_t cls_ppt[kPathClasses], cls_store[kPathClasses];
     uint32_t cls_draw[kPathClasses];
     for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
-        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_mart[cls], cls_long[cls], tun);
+        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_most[cls], cls_mart[cls], cls_long[cls], tun);
         cls_ppt[cls] = cls == 0 || cls_draw[cls] ? 1u : tun.paths_per_thread;
         cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;
     }

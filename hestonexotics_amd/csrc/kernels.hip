@@ -771,9 +771,10 @@ __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32
 
 // Registers for 5 waves per SIMD at 2 paths per lane (96), 4 with the martingale step: it needs 114,
 // and held to 96 it spilled 22 (4e6 paths x 252 steps 2.58 -> 2.48 ms, 2^20 stiff paths x 2,048 steps
-// 7.15 -> 6.90).
+// 7.15 -> 6.90). With the geometric average as well it spills as much, but its payoff sums want
+// the fifth wave more (1,000 strikes x 3 payoffs x 52 steps, 3.5e6 paths 3.79 -> 3.30 ms with it).
 template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 && !MART ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 && (!MART || GEO) ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
     extern __shared__ uint32_t lds_u32[];
     const int lane = (int)(threadIdx.x & 63u);
     // the wave's LDS region, at a wave-uniform address
