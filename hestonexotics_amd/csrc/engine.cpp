@@ -652,6 +652,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         b->nominal_path_steps += (double)q.n_paths * (double)q.steps * (double)q.n_expiries;
     }
     b->n_group_threads = ge;
+    b->small_reduce = ge <= kSmallGroupSums;
+    for (const ReqPlan& p : plans) b->small_reduce &= p.n_groups <= kSmallGroups;
     b->n_out_threads = out_i;
 
     // work queues: per kernel class, requests longest first
@@ -852,7 +854,7 @@ static int enqueue_body(Batch& b, PathMode mode, bool timed, double* d_finals, s
         ++b.path_launches;
     }
     if (timed) HIP_TRY(hipEventRecord(b.ev[1], b.stream));
-    HIP_TRY(launch_reduce(b.ra, b.n_group_threads, b.n_out_threads, b.stream));
+    HIP_TRY(launch_reduce(b.ra, b.n_group_threads, b.n_out_threads, b.small_reduce, b.stream));
     if (timed) HIP_TRY(hipEventRecord(b.ev[2], b.stream));
     HIP_TRY(hipMemcpyAsync(b.h_prices, b.ra.prices, sizeof(double) * b.n_out_total, hipMemcpyDeviceToHost, b.stream));
     HIP_TRY(hipMemcpyAsync(b.h_ses, b.ra.std_errs, sizeof(double) * b.n_out_total, hipMemcpyDeviceToHost, b.stream));

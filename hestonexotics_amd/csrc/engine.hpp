@@ -132,6 +132,7 @@ struct Batch {
     ReduceArgs ra{};
     GeoArgs ga{};  // exact geometric prices, computed once after the upload (n_items 0: none)
     uint64_t n_group_threads = 0, n_out_threads = 0;
+    bool small_reduce = false;  // one reduction kernel (layout.hpp, kSmallGroups)
     uint32_t* d_counters = nullptr;
     unsigned long long* d_counts = nullptr;
     // graph

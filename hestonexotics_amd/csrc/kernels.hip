@@ -127,6 +127,12 @@ struct TileSums<double> {  // FP64 sums (HEXO_FP32 and the FP64 kernel)
     __device__ __forceinline__ void store(void* partials, size_t slot) const {
         reinterpret_cast<double2*>(partials)[slot] = make_double2(s, ss);
     }
+    __device__ __forceinline__ TileSums of_lane(int l) const {
+        TileSums t;
+        t.s = __shfl(s, l);
+        t.ss = __shfl(ss, l);
+        return t;
+    }
 };
 
 template <>
@@ -157,6 +163,12 @@ struct TileSums<float> {  // compensated FP32 sums (HEXO_FP32_COMPENSATED)
     }
     __device__ __forceinline__ void store(void* partials, size_t slot) const {
         reinterpret_cast<float4*>(partials)[slot] = make_float4(s.s, s.c, ss.s, ss.c);
+    }
+    __device__ __forceinline__ TileSums of_lane(int l) const {
+        TileSums t;
+        t.s = CompF{__shfl(s.s, l), __shfl(s.c, l)};
+        t.ss = CompF{__shfl(ss.s, l), __shfl(ss.c, l)};
+        return t;
     }
 };
 
@@ -1151,34 +1163,37 @@ __device__ __forceinline__ TileSums<Acc> stored_sum(const ReduceArgs& a, const D
     return t;
 }
 
-// Sums the chunks of one 64-tile group in chunk order. Each chunk's sum completes the tree
-// ((t0 + t1) + (t2 + t3)) from the level the path kernel stored (store_tiles tiles per partial),
-// so a chunk's bits do not depend on the paths per thread the request ran with.
+// The sum of one chunk of tiles: completes the tree ((t0 + t1) + (t2 + t3)) from the level the path
+// kernel stored (store_tiles tiles per partial), so a chunk's bits do not depend on the paths per
+// thread the request ran with.
 template <typename Acc>
-__device__ __forceinline__ TileSums<Acc> group_sum(const ReduceArgs& a, const DevReq& R, uint32_t n_out, uint32_t g,
+__device__ __forceinline__ TileSums<Acc> chunk_sum(const ReduceArgs& a, const DevReq& R, uint32_t n_out, uint32_t c,
                                                    uint32_t o) {
     const uint32_t st = R.store_tiles;
     const uint32_t n_slots = (R.n_tiles + st - 1) / st;
-    const uint32_t t0 = g * kGroupTiles;
-    const uint32_t t1 = min(t0 + (uint32_t)kGroupTiles, R.n_tiles);
-    TileSums<Acc> acc;
-    for (uint32_t c = t0 / kChunkTiles; c < (t1 + kChunkTiles - 1) / kChunkTiles; ++c) {
-        TileSums<Acc> chunk;
-        if (st == kChunkTiles) {
-            chunk = stored_sum<Acc>(a, R, n_out, n_slots, c, o);
-        } else if (st == 2) {
-            TileSums<Acc> t[2] = {stored_sum<Acc>(a, R, n_out, n_slots, 2 * c, o),
-                                  stored_sum<Acc>(a, R, n_out, n_slots, 2 * c + 1, o)};
-            t[0].combine(t[1]);
-            chunk = t[0];
-        } else {
-            TileSums<Acc> t[kChunkTiles];
-#pragma unroll
-            for (int i = 0; i < kChunkTiles; ++i) t[i] = stored_sum<Acc>(a, R, n_out, n_slots, kChunkTiles * c + i, o);
-            chunk = chunk_level<kChunkTiles, Acc>(t);
-        }
-        acc.combine(chunk);
+    if (st == kChunkTiles) return stored_sum<Acc>(a, R, n_out, n_slots, c, o);
+    if (st == 2) {
+        TileSums<Acc> t[2] = {stored_sum<Acc>(a, R, n_out, n_slots, 2 * c, o),
+                              stored_sum<Acc>(a, R, n_out, n_slots, 2 * c + 1, o)};
+        t[0].combine(t[1]);
+        return t[0];
     }
+    TileSums<Acc> t[kChunkTiles];
+#pragma unroll
+    for (int i = 0; i < kChunkTiles; ++i) t[i] = stored_sum<Acc>(a, R, n_out, n_slots, kChunkTiles * c + i, o);
+    return chunk_level<kChunkTiles, Acc>(t);
+}
+
+__device__ __forceinline__ uint32_t chunks_of(const DevReq& R) { return (R.n_tiles + kChunkTiles - 1) / kChunkTiles; }
+constexpr uint32_t kGroupChunks = kGroupTiles / kChunkTiles;
+
+// Sums the chunks of one 64-tile group in chunk order.
+template <typename Acc>
+__device__ __forceinline__ TileSums<Acc> group_sum(const ReduceArgs& a, const DevReq& R, uint32_t n_out, uint32_t g,
+                                                   uint32_t o) {
+    TileSums<Acc> acc;
+    const uint32_t end = min((g + 1) * kGroupChunks, chunks_of(R));
+    for (uint32_t c = g * kGroupChunks; c < end; ++c) acc.combine(chunk_sum<Acc>(a, R, n_out, c, o));
     return acc;
 }
 
@@ -1198,18 +1213,17 @@ __global__ __launch_bounds__(256) void k_reduce_groups(ReduceArgs a, uint64_t to
         group_sum<double>(a, R, n_out, g, o).store(a.groups, gslot);
 }
 
-// Sum and sum of squares of output o over the request's groups, on one wavefront: lane l sums
-// groups l, l + 64, l + 128, ... in order and the 64 lane sums are combined by a fixed xor
+// Sum and sum of squares of an output over the request's groups (sums[first + g stride]), on one
+// wavefront: lane l sums groups l, l + 64, l + 128, ... in order and the 64 lane sums are combined by a fixed xor
 // butterfly (every lane ends with the same bits). The order depends only on the request's group
 // count, never on the launch.
-__device__ __forceinline__ void output_sums(const ReduceArgs& a, const DevReq& R, uint32_t o, uint32_t lane,
-                                            double& s, double& ss) {
-    const uint32_t n_out = R.n_opts * R.n_pay;
+__device__ __forceinline__ void output_sums(const void* sums, size_t first, uint32_t stride, const DevReq& R,
+                                            uint32_t lane, double& s, double& ss) {
     if (R.precision == kPrecComp) {
-        const float4* p = reinterpret_cast<const float4*>(a.groups);
+        const float4* p = reinterpret_cast<const float4*>(sums);
         CompF cs{0.f, 0.f}, css{0.f, 0.f};
         for (uint32_t g = lane; g < R.n_groups; g += kTile) {
-            const float4 v = p[(size_t)R.group_base + (size_t)g * n_out + o];
+            const float4 v = p[first + (size_t)g * stride];
             cs.merge(v.x, v.y);
             css.merge(v.z, v.w);
         }
@@ -1223,11 +1237,11 @@ __device__ __forceinline__ void output_sums(const ReduceArgs& a, const DevReq& R
         s = (double)cs.s + (double)cs.c;
         ss = (double)css.s + (double)css.c;
     } else {
-        const double2* p = reinterpret_cast<const double2*>(a.groups);
+        const double2* p = reinterpret_cast<const double2*>(sums);
         s = 0.0;
         ss = 0.0;
         for (uint32_t g = lane; g < R.n_groups; g += kTile) {
-            const double2 v = p[(size_t)R.group_base + (size_t)g * n_out + o];
+            const double2 v = p[first + (size_t)g * stride];
             s += v.x;
             ss += v.y;
         }
@@ -1246,25 +1260,68 @@ __device__ __forceinline__ void mean_var(double s, double ss, double n, double& 
     var = var > 0.0 ? var : 0.0;
 }
 
-// One wavefront per output. A control-variate output adds the exact geometric price to the mean of
-// A - G; with kCvRegression it is A - beta (G - E[G]) instead, beta = Cov(A, G) / Var G from the
-// same paths' Asian (block 0) and geometric outputs of the option: Cov from
-// Var(A - G) = Var A + Var G - 2 Cov(A, G), variance Var A - beta Cov(A, G).
+// The group sums of output o into LDS by a workgroup of 256 threads: 16 lanes take the chunks of a
+// group, and combine them in chunk order.
+template <typename Acc>
+__device__ __forceinline__ void group_sums_lds(const ReduceArgs& a, const DevReq& R, uint32_t o, void* sums) {
+    static_assert(kGroupChunks == 16, "a group's chunks are the 16 lanes of a row");
+    const uint32_t n_out = R.n_opts * R.n_pay, n_chunks = chunks_of(R), i = threadIdx.x % 16u;
+    for (uint32_t g0 = 0; g0 < R.n_groups; g0 += 16) {
+        const uint32_t g = g0 + threadIdx.x / 16u, c = g * kGroupChunks + i;
+        TileSums<Acc> t, acc;
+        if (c < n_chunks) t = chunk_sum<Acc>(a, R, n_out, c, o);
+#pragma unroll
+        for (uint32_t k = 0; k < kGroupChunks; ++k) {
+            const TileSums<Acc> u = t.of_lane((int)((threadIdx.x & 48u) + k));
+            if (g * kGroupChunks + k < n_chunks) acc.combine(u);
+        }
+        if (i == 0 && g < R.n_groups) acc.store(sums, g);
+    }
+}
+
+// One wavefront per output, or for small batches (SMALL, at most kSmallGroups groups a request) one
+// workgroup, whose threads form the group sums of what the output reads first: one kernel in place of
+// two, and a group's chunks in parallel lanes instead of one thread's serial loads (a request of 63
+// tiles: 11.5 us with the gap between them -> 6.8). In larger batches a wavefront's loads a whole row
+// of outputs apart cost more.
+// A control-variate output adds the exact geometric price to the mean of A - G; with kCvRegression
+// it is A - beta (G - E[G]) instead, beta = Cov(A, G) / Var G from the same paths' Asian (block 0)
+// and geometric outputs of the option: Cov from Var(A - G) = Var A + Var G - 2 Cov(A, G), variance
+// Var A - beta Cov(A, G).
+template <bool SMALL>
 __global__ __launch_bounds__(256) void k_reduce_final(ReduceArgs a, uint64_t total) {
-    const uint64_t t = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / (uint64_t)kTile;  // wave-uniform
+    __shared__ double2 lds[SMALL ? 3 : 1][SMALL ? kSmallGroups : 1];
+    const uint64_t t = SMALL ? blockIdx.x : ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / (uint64_t)kTile;  // wave-uniform
     const uint32_t lane = threadIdx.x % (uint32_t)kTile;
     if (t >= total) return;
     const uint32_t ri = find_req(a.out_end, a.n_req, t);
     const uint32_t o = (uint32_t)(t - (ri ? a.out_end[ri - 1] : 0ull));
     const DevReq& R = a.reqs[ri];
-    const uint32_t opt = o % R.n_opts;
+    const uint32_t opt = o % R.n_opts, n_out = R.n_opts * R.n_pay;
     const bool cv = a.geo && payoff_kind(R.payoffs, o / R.n_opts) == kAsianGeoCV;
     const bool reg = cv && (R.flags & kCvRegression);  // request-uniform
+    const uint32_t outs[3] = {o, opt, (uint32_t)__popc(R.payoffs & (kGeoAsian - 1u)) * R.n_opts + opt};
+    if constexpr (SMALL) {
+        for (int k = 0; k < (reg ? 3 : 1); ++k) {
+            if (R.precision == kPrecComp)
+                group_sums_lds<float>(a, R, outs[k], lds[k]);
+            else
+                group_sums_lds<double>(a, R, outs[k], lds[k]);
+        }
+        __syncthreads();
+        if (threadIdx.x >= (uint32_t)kTile) return;
+    }
+    auto sums = [&](int k, double& s, double& ss) {
+        if constexpr (SMALL)
+            output_sums(lds[k], 0, 1, R, lane, s, ss);
+        else
+            output_sums(a.groups, (size_t)R.group_base + outs[k], n_out, R, lane, s, ss);
+    };
     double s, ss, sa = 0.0, ssa = 0.0, sg = 0.0, ssg = 0.0;
-    output_sums(a, R, o, lane, s, ss);
+    sums(0, s, ss);
     if (reg) {
-        output_sums(a, R, opt, lane, sa, ssa);
-        output_sums(a, R, (uint32_t)__popc(R.payoffs & (kGeoAsian - 1u)) * R.n_opts + opt, lane, sg, ssg);
+        sums(1, sa, ssa);
+        sums(2, sg, ssg);
     }
     if (lane != 0) return;
     const double disc = a.opts[R.opt_begin + opt].disc;
@@ -1454,12 +1511,17 @@ hipError_t launch_paths(uint32_t precision, uint32_t ppt, PathMode mode, uint32_
     return hipGetLastError();
 }
 
-hipError_t launch_reduce(const ReduceArgs& a, uint64_t n_group_threads, uint64_t n_out_threads, hipStream_t st) {
+hipError_t launch_reduce(const ReduceArgs& a, uint64_t n_group_threads, uint64_t n_out_threads, bool small,
+                         hipStream_t st) {
+    if (small) {
+        if (n_out_threads) k_reduce_final<true><<<(uint32_t)n_out_threads, 256, 0, st>>>(a, n_out_threads);
+        return hipGetLastError();
+    }
     if (n_group_threads) k_reduce_groups<<<grid_for(n_group_threads, 256), 256, 0, st>>>(a, n_group_threads);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // one wavefront per output
-    if (n_out_threads) k_reduce_final<<<grid_for(n_out_threads * kTile, 256), 256, 0, st>>>(a, n_out_threads);
+    if (n_out_threads) k_reduce_final<false><<<grid_for(n_out_threads * kTile, 256), 256, 0, st>>>(a, n_out_threads);
     return hipGetLastError();
 }
 

@@ -24,7 +24,9 @@ hipError_t launch_paths_split(uint32_t precision, uint32_t n_draw, const PathArg
 // items that it left unfinished; GeoArgs.state holds geo_state_doubles(n_items) doubles.
 hipError_t launch_geo(const GeoArgs& a, bool first, hipStream_t st);
 size_t geo_state_doubles(uint32_t n_items);
-hipError_t launch_reduce(const ReduceArgs& a, uint64_t n_group_threads, uint64_t n_out_threads, hipStream_t st);
+// small: no request has more than kSmallGroups groups (one kernel instead of two).
+hipError_t launch_reduce(const ReduceArgs& a, uint64_t n_group_threads, uint64_t n_out_threads, bool small,
+                         hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t st);
 hipError_t launch_zero_u64(unsigned long long* p, uint32_t n, hipStream_t st);
 hipError_t launch_rng_fill(uint32_t* out, uint64_t seed, uint32_t stream, uint64_t path0, uint64_t n_paths,

@@ -148,6 +148,11 @@ struct GeoArgs {
     double* state;          // per item between rounds: strike sums, E[e^L], panels done, converged
 };
 
+// The one-kernel reduction's groups per request (its LDS), and the group sums of a batch up to which
+// it is used (median of both kernels / the one, us, at 1, 25, 600, 1,024, 1,800 group sums: 11.5/6.8,
+// 12.4/9.1, 16.3/9.8, 15.2/13.7, 16.8/11.0; at 2,560 to 4,096 16.2/17.9, 15.8/17.2, 17.4/18.9).
+constexpr uint32_t kSmallGroups = 64, kSmallGroupSums = 2048;
+
 struct ReduceArgs {
     const DevReq* reqs;
     const DevOpt* opts;

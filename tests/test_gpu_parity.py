@@ -493,3 +493,23 @@ def test_fp64_split_kernel_equals_persistent(ctx, n_paths, steps, T):
             got, want = ctx.price(req), ctx.price_batch([req, filler])[0]
             np.testing.assert_array_equal(got[0], want[0])
             np.testing.assert_array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("precision", [H.FP64, H.FP32, H.FP32_COMPENSATED])
+@pytest.mark.parametrize("n_paths", [1, 64, 65, 255, 257, 4096, 4097, 16384, 16385, 65537, 262144])
+def test_one_kernel_reduction_equals_two(ctx, precision, n_paths):
+    """A small batch's reduction (one kernel: group sums by 16 lanes a group) gives the bits of the
+    two-kernel one, which a batch with one request beyond 64 groups takes: at the edges of chunks
+    (256 paths), groups (4,096) and rounds of groups (65,536), with the regression control variate."""
+    say("gpu one-kernel reduction", precision, n_paths)
+    kw = dict(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, expiries=[0.5, 1.0],
+              strikes=[[95.0, 105.0], [100.0]], steps=4, seed=6, r=0.02, precision=precision)
+    control = H.ASIAN | H.ASIAN_GEO_CV | H.GEO_ASIAN
+    reqs = [H.Request(**kw, n_paths=n_paths, payoffs=H.ASIAN | H.EUROPEAN, flags=H.DRIFT | H.DISCOUNT),
+            H.Request(**kw, n_paths=n_paths, payoffs=control, flags=H.DRIFT | H.CV_REGRESSION)]
+    filler = H.Request(**kw, n_paths=262145, payoffs=H.ASIAN, flags=H.DRIFT)
+    beside = ctx.price_batch(reqs + [filler])
+    for req, (p, s) in zip(reqs, beside):
+        pa, sa = ctx.price(req)
+        np.testing.assert_array_equal(pa, p)
+        np.testing.assert_array_equal(sa, s)
