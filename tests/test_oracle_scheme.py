@@ -266,3 +266,16 @@ def test_path_offset_selects_the_same_paths():
     part = O.price(BASE, 100.0, [1.0], [1], [100.0], steps=12, n_paths=100, seed=8, path_offset=150,
                    want_finals=True)["finals"]
     np.testing.assert_array_equal(full[150:250], part)
+
+
+def test_fast_oracle_leaves_subnormals_to_the_checker():
+    """The timed build, compiled with -ffast-math, must not switch the process to flush-to-zero: at
+    S0 = 1e-305 the average's last interval (X - Xp)(T - tp) is subnormal, and the checker's finals
+    are 1e-305 times those at S0 = 1 (to 1e-9: ln X = -702 carries 1e-13 a step; flushed, they are off
+    by 8%)."""
+    kw = dict(steps=9, n_paths=130, seed=13, want_finals=True)
+    args = ([0.5], [1])
+    O.price(BASE, 1.0, *args, [1.0], steps=2, n_paths=64, seed=1, kind="fast")
+    one = O.price(BASE, 1.0, *args, [1.0], **kw)["finals"]
+    tiny = O.price(BASE, 1e-305, *args, [1e-305], **kw)["finals"]
+    np.testing.assert_allclose(tiny / 1e-305, one, rtol=1e-9)
