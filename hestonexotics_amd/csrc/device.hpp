@@ -101,42 +101,32 @@ __device__ __forceinline__ double normal_tail_f64(uint32_t j) {
     const double r = sqrt_f64(-log_f64(uniform_f64(j))) - 1.6;
     return div_f64(horner8(As241<double>::c, r), horner8(As241<double>::d, r));
 }
-// The central rational of N words at once: the coefficients are loaded once for all of them, and
-// their reciprocals come from one of the product (the denominators lie in [0.04, 1]); the residual
+// The central rational of a counter block's four words at once: the coefficients are loaded once for
+// all of them, and their reciprocals come from one of the product. Tail words take part (their results
+// are replaced afterwards): over all words the denominators lie in [0.0021, 94.1], positive throughout,
+// and their product in [2e-11, 8e7], so that no word spoils the other three. The residual
 // correction leaves each quotient within its last rounding whatever the reciprocal's.
-template <int N>
-__device__ __forceinline__ void normal_central_f64(const double (&q)[N], double (&z)[N]) {
-    static_assert(N == 1 || N == 4, "one word or a counter block's four");
-    double num[N], den[N], rec[N];
+__device__ __forceinline__ void normals_central_f64(const double (&q)[4], double (&z)[4]) {
+    double num[4], den[4], rec[4];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
+    for (int i = 0; i < 4; ++i) {
         const double r = __builtin_fma(-q[i], q[i], 0.180625);
         num[i] = q[i] * horner8(As241<double>::a, r);
         den[i] = horner8(As241<double>::b, r);
     }
-    if constexpr (N == 4) {
-        const double d01 = den[0] * den[1], d23 = den[2] * den[3], d = d01 * d23;
-        double r = __builtin_amdgcn_rcp(d);
-        r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-        const double r01 = r * d23, r23 = r * d01;
-        rec[0] = r01 * den[1];
-        rec[1] = r01 * den[0];
-        rec[2] = r23 * den[3];
-        rec[3] = r23 * den[2];
+    const double d01 = den[0] * den[1], d23 = den[2] * den[3], d = d01 * d23;
+    double r = __builtin_amdgcn_rcp(d);
+    r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+    const double r01 = r * d23, r23 = r * d01;
+    rec[0] = r01 * den[1];
+    rec[1] = r01 * den[0];
+    rec[2] = r23 * den[3];
+    rec[3] = r23 * den[2];
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const double v = num[i] * rec[i];
-            z[i] = __builtin_fma(__builtin_fma(-den[i], v, num[i]), rec[i], v);
-        }
-    } else {
-        z[0] = div_f64(num[0], den[0]);
+    for (int i = 0; i < 4; ++i) {
+        const double v = num[i] * rec[i];
+        z[i] = __builtin_fma(__builtin_fma(-den[i], v, num[i]), rec[i], v);
     }
-}
-__device__ __forceinline__ double normal_f64(uint32_t k) {
-    const double q[1] = {centred_f64(k)};
-    double z[1];
-    normal_central_f64<1>(q, z);
-    return is_tail_f64(q[0]) ? __builtin_copysign(normal_tail_f64(k ^ (uint32_t)((int32_t)k >> 31)), q[0]) : z[0];
 }
 
 // A value the compiler must keep in a vector register (it cannot prove the result wave-uniform and

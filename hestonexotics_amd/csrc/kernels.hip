@@ -948,7 +948,7 @@ __device__ __forceinline__ void normals4_f64(const u32x4& w, double (&z)[4], dou
         if (t) words[2 * pos[i]] = k[i] ^ (uint32_t)((int32_t)k[i] >> 31);
         n += (uint32_t)__builtin_popcountll(mask);
     }
-    normal_central_f64<4>(q, z);
+    normals_central_f64(q, z);
     wave_sync_lds();
     for (uint32_t b = 0; b < n; b += kTile) {  // wave-uniform
         const uint32_t t = b + (uint32_t)lane;
@@ -1379,10 +1379,23 @@ __global__ void k_philox(const uint32_t* ctr, const uint32_t* key, uint64_t n, u
     out[4 * i + 3] = b.w;
 }
 
-__global__ void k_normals(const uint32_t* words, uint64_t n, uint32_t precision, double* out) {
+__global__ void k_normals_fp32(const uint32_t* words, uint64_t n, double* out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    out[i] = precision == kPrecFP64 ? normal_f64(words[i]) : (double)normal_f32(words[i]);
+    out[i] = (double)normal_f32(words[i]);
+}
+
+// Words 4t .. 4t + 3 by thread t, as the FP64 path kernels take a lane's counter block. Words past n
+// (central ones) fill the last wavefront up.
+__global__ __launch_bounds__(256) void k_normals_fp64(const uint32_t* words, uint64_t n, double* out) {
+    __shared__ double queue[4][4 * kTile];
+    const uint64_t i = 4 * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    uint32_t k[4];
+    for (uint32_t j = 0; j < 4; ++j) k[j] = i + j < n ? words[i + j] : 0x80000000u;
+    double z[4];
+    normals4_f64(u32x4{k[0], k[1], k[2], k[3]}, z, queue[threadIdx.x >> 6], (int)(threadIdx.x & 63u));
+    for (uint32_t j = 0; j < 4; ++j)
+        if (i + j < n) out[i + j] = z[j];
 }
 
 __global__ void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n) {
@@ -1547,7 +1560,10 @@ hipError_t launch_philox(const uint32_t* ctr, const uint32_t* key, uint64_t n, u
 }
 
 hipError_t launch_normals(const uint32_t* words, uint64_t n, uint32_t precision, double* out, hipStream_t st) {
-    k_normals<<<grid_for(n, 256), 256, 0, st>>>(words, n, precision, out);
+    if (precision == kPrecFP64)
+        k_normals_fp64<<<grid_for((n + 3) / 4, 256), 256, 0, st>>>(words, n, out);
+    else
+        k_normals_fp32<<<grid_for(n, 256), 256, 0, st>>>(words, n, out);
     return hipGetLastError();
 }
 

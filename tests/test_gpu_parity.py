@@ -513,3 +513,23 @@ def test_one_kernel_reduction_equals_two(ctx, precision, n_paths):
         pa, sa = ctx.price(req)
         np.testing.assert_array_equal(pa, p)
         np.testing.assert_array_equal(sa, s)
+
+
+def tail_words(n):
+    """n words of the tail regions u < 0.075 and u > 0.925 alternately, the ends of both first."""
+    lo = np.unique(np.linspace(0, int(0.075 * 2**32) - 1, n).astype(np.uint64))
+    w = np.empty(n, np.uint64)
+    w[0::2], w[1::2] = lo[: (n + 1) // 2], 2**32 - 1 - lo[: n // 2]
+    return w.astype(np.uint32)
+
+
+@pytest.mark.parametrize("n_tail", [0, 1, 63, 64, 65, 128, 129, 255, 256])
+def test_fp64_normals_of_a_wavefront(ctx, oracle, n_tail):
+    """A wavefront's 256 words with n_tail of them in the tail (queued, 64 at a time), spread over the
+    lanes and over a block's four words: blocks of tail words beside central ones share a reciprocal.
+    Then a call that ends within a wavefront. The oracle's rounding, as over random words."""
+    rng = np.random.default_rng(n_tail)
+    w = (rng.integers(int(0.08 * 2**32), int(0.92 * 2**32), 256)).astype(np.uint32)
+    w[rng.permutation(256)[:n_tail]] = tail_words(n_tail)
+    for words in (w, np.concatenate([w, w[::-1], w[:37]])):
+        np.testing.assert_allclose(ctx.normals(words, H.FP64), oracle.normals_f64(words), rtol=2e-15, atol=1e-15)
