@@ -49,9 +49,16 @@ int run_single(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, double* pric
     if (rc == HEXO_ERR_NOMEM && need) {
         // grow; the arena is empty, every earlier call's batch being complete and released
         const size_t grown = std::max<size_t>({need, (size_t)16 << 20, 2 * ctx->sync_arena.capacity()});
-        if (!ctx->sync_arena.init(grown) && !ctx->sync_arena.init(need))
-            return ctx->set_error(HEXO_ERR_NOMEM, "hipMalloc of " + std::to_string(need) + " device bytes failed");
-        rc = hexo::batch_create(ctx, reqs, n, ctx->stream, mem, b, err);
+        hexo::LaunchPlan plan = hexo::plan_of(ctx->tuning_now());
+        if (!ctx->sync_arena.init(grown) && !ctx->sync_arena.init(need)) {
+            // half the partials with the persistent kernels
+            plan.split = false;
+            need = 0;
+            rc = hexo::batch_create(ctx, reqs, n, ctx->stream, mem, b, err, nullptr, &plan);
+            if (rc != HEXO_ERR_NOMEM || !need || !ctx->sync_arena.init(need))
+                return ctx->set_error(HEXO_ERR_NOMEM, "hipMalloc of " + std::to_string(need) + " device bytes failed");
+        }
+        rc = hexo::batch_create(ctx, reqs, n, ctx->stream, mem, b, err, nullptr, &plan);
     }
     if (rc != HEXO_OK) return ctx->set_error(rc, err);
     rc = hexo::batch_enqueue(*b, PathMode::Normal, false, nullptr, err);
@@ -469,9 +476,10 @@ int hexo_autotune(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, uint32_t 
         for (uint32_t b : blocks)
             for (uint32_t w : waves) {
                 const hexo_tuning trial{p, b, w, 0};
+                const hexo::LaunchPlan plan = hexo::plan_of(trial);
                 std::string err;
                 std::unique_ptr<hexo::Batch> bt;
-                int rc = hexo::batch_create(ctx, reqs, n, ctx->stream, hexo::BatchMemory(), bt, err, nullptr, &trial);
+                int rc = hexo::batch_create(ctx, reqs, n, ctx->stream, hexo::BatchMemory(), bt, err, nullptr, &plan);
                 if (rc != HEXO_OK) return ctx->set_error(rc, err);
                 double total = 0.0;
                 for (uint32_t r = 0; r <= reps && rc == HEXO_OK; ++r) {  // first run warms up

@@ -154,6 +154,7 @@ bool Arena::init(size_t bytes) {
     release();
     bytes = (bytes + 255) & ~(size_t)255;
     if (hipMalloc(reinterpret_cast<void**>(&base_), bytes) != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch would report it
         base_ = nullptr;
         return false;
     }
@@ -294,8 +295,7 @@ uint64_t split_most_tiles(const ReqPlan& p) {
 }
 
 // Drawing waves per tile of the split kernel for a class of `tiles` 64-path tiles, or 0 for the
-// persistent kernel. FP32, where the launch shape is left to the library (2 paths per thread, no
-// occupancy cap):
+// persistent kernel. FP32, where the plan allows it:
 //  * up to 512 tiles (half the SIMDs): two drawing waves; the tile's time is the stepping wave's
 //    (1e4 paths x 126 steps 28.5 -> 20.4 us against one). Beyond, the third wave competes with
 //    other tiles' stepping waves: 5% faster still for quadratic-branch steps at 1,500 tiles, 15%
@@ -319,10 +319,10 @@ uint64_t split_most_tiles(const ReqPlan& p) {
 //  * with the correction up to 256 tiles (1e4 paths: 223 us against 392, stiff parameters 332 against
 //    500; at 313 tiles stiff 521 against 501, at 1,563 and one drawing wave 610 against 561).
 uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, uint64_t most_tiles, bool martingale, bool long_steps,
-                          const hexo_tuning& tun) {
+                          bool fp32_split) {
     if (tiles > most_tiles) return 0;
     if (cls == 0) return tiles > (martingale ? 256u : 3328u) ? 0 : tiles <= 512 ? 2 : 1;
-    if (tun.paths_per_thread != 2 || tun.waves_per_simd != 0) return 0;
+    if (!fp32_split) return 0;
     if (tiles > (long_steps ? 2048u : class_geo(cls) ? 1u << 16 : 1u << 17)) return 0;
     return tiles <= 512 ? 2 : 1;
 }
@@ -388,12 +388,13 @@ PinnedBuf::~PinnedBuf() {
 
 int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_t stream, const BatchMemory& mem,
                  std::unique_ptr<Batch>& out, std::string& err, const uint64_t* finals_n,
-                 const hexo_tuning* tuning) {
+                 const LaunchPlan* given) {
     if (n == 0 || !reqs) {
         err = "empty batch";
         return HEXO_ERR_INVALID;
     }
-    const hexo_tuning tun = tuning ? *tuning : ctx->tuning_now();
+    const LaunchPlan plan = given ? *given : plan_of(ctx->tuning_now());
+    const hexo_tuning& tun = plan.shape;
     std::vector<ReqPlan> plans(n);
     uint64_t n_seg = 0, n_fin = 0, n_opt = 0, n_partials = 0, n_groups = 0, n_out = 0;
     uint64_t n_geo_items = 0, n_geo_pts = 0, n_geo_waves = 0;
@@ -437,8 +438,10 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     // kChunkTiles), or one per tile when its tiles do not divide a chunk (3 paths per thread).
     uint32_t cls_ppt[kPathClasses], cls_store[kPathClasses];
     uint32_t cls_draw[kPathClasses];
+    bool fp32_split = false;
     for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
-        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_most[cls], cls_mart[cls], cls_long[cls], tun);
+        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_most[cls], cls_mart[cls], cls_long[cls], plan.split);
+        fp32_split |= cls != 0 && n_cls[cls] && cls_draw[cls];
         cls_ppt[cls] = cls == 0 || cls_draw[cls] ? 1u : tun.paths_per_thread;
         cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;
     }
@@ -457,7 +460,13 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         make_layout(n, n_seg, n_fin, n_opt, n_cls, n_partials, n_groups, n_out, n_finals, n_geo_items, n_geo_pts,
                     n_geo_waves);
 
+    auto persistent = [&] {
+        LaunchPlan p = plan;
+        p.split = false;
+        return batch_create(ctx, reqs, n, stream, mem, out, err, finals_n, &p);
+    };
     // the device region must fit a fixed region or the arena before anything is staged
+    if (mem.region && L.total > mem.region_bytes && fp32_split) return persistent();
     if ((mem.region && L.total > mem.region_bytes) ||
         (!mem.region && mem.arena && L.total > mem.arena->capacity() - mem.arena->in_use())) {
         if (mem.need) *mem.need = L.total;
@@ -700,8 +709,10 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         }
         b->arena = mem.arena;
     } else if (hipMalloc(reinterpret_cast<void**>(&b->d_mem), L.total) != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch would report it
         b->d_mem = nullptr;
         batch_destroy(*b);
+        if (fp32_split) return persistent();
         err = "hipMalloc of " + std::to_string(L.total) + " bytes failed";
         return HEXO_ERR_NOMEM;
     }

@@ -106,6 +106,15 @@ inline uint32_t class_precision(uint32_t cls) { return cls == 0 ? HEXO_FP64 : HE
 inline bool class_martingale(uint32_t cls) { return cls == 2 || cls == 4; }
 inline bool class_geo(uint32_t cls) { return cls >= 3; }
 
+// How a batch's FP32 classes are launched: the persistent kernels' shape, and whether the kernels with
+// drawing and stepping waves may take a class instead (engine.cpp, split_draw_waves).
+struct LaunchPlan {
+    hexo_tuning shape{2, 256, 0, 0};
+    bool split = true;
+};
+// A shape set by the caller is used as given; the default one leaves the choice to the library.
+inline LaunchPlan plan_of(const hexo_tuning& t) { return {t, t.paths_per_thread == 2 && t.waves_per_simd == 0}; }
+
 struct Batch {
     hexo_ctx* ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -225,10 +234,12 @@ struct BatchMemory {
 };
 
 // Creates a batch: validates, builds the schedules, packs and uploads the tables, plans the
-// launches. tuning: the launch shape to plan with (null: the context's, read once under tuning_mu).
+// launches. plan: null for the context's shape (read once under tuning_mu). Where the device bytes do not
+// fit a fixed region, or cannot be allocated, the FP32 classes fall back to the persistent kernels, which
+// store half as many partials.
 int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_t stream, const BatchMemory& mem,
                  std::unique_ptr<Batch>& out, std::string& err, const uint64_t* finals_n = nullptr,
-                 const hexo_tuning* tuning = nullptr);
+                 const LaunchPlan* plan = nullptr);
 // Device bytes a set of requests needs (admission accounting).
 size_t batch_device_bytes(const hexo_request* reqs, uint32_t n);
 size_t request_device_bytes(const hexo_request* r);

@@ -2,18 +2,19 @@
 //
 // For callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
 // that forbid hipMalloc). The batch's device region (request tables, tile partials, group sums,
-// prices) lives in `scratch`, a file-scope device array of kScratchBytes that every GPU the
-// library runs on holds until the process ends; the host staging of the tables and results lives
-// in a file-scope host array. In host code `scratch` names a host-side stand-in, not a device
-// address: its address on each device is looked up once per device (hexo_ctx_create, with the
-// device current) and only that address is used.
+// prices) lives in `scratch`, a file-scope device array that every GPU the library runs on holds
+// until the process ends; the host staging of the tables and results lives in a file-scope host
+// array. In host code `scratch` names a host-side stand-in, not a device address: its address on
+// each device is looked up once per device (hexo_ctx_create, with the device current) and only that
+// address is used.
 //
 // Calls are serialised by the library (the array of a device and the host array are shared by
 // every call); each call overwrites the array's previous contents. What must start at zero (the
-// work-queue counters) is cleared by a fill kernel at every call. Requests whose region needs more
-// than kScratchBytes, or whose tables and results need more than kStageBytes of host staging, are
-// refused with HEXO_ERR_INVALID. Host-side planning (the time grid, the launch plan) uses the C++
-// heap, as in hexo_price.
+// work-queue counters) is cleared by a fill kernel at every call. A request whose partials do not fit
+// with one per tile (the kernels with drawing and stepping waves) runs on the persistent kernels, with
+// one per pair. Requests whose region needs more than the device array, or whose tables and results
+// need more than the host array, are refused with HEXO_ERR_INVALID. Host-side planning (the time
+// grid, the launch plan) uses the C++ heap, as in hexo_price.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -25,10 +26,12 @@ namespace {
 
 constexpr size_t kScratchBytes = (size_t)64 << 20;
 constexpr size_t kStageBytes = (size_t)16 << 20;
+// Room for the FP64 step's constants in the run records (56 bytes each, at most 4,096 runs a request).
+constexpr size_t kRunTableBytes = (size_t)256 << 10;
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) unsigned char scratch[kScratchBytes];
-alignas(256) unsigned char host_stage[kStageBytes];
+__device__ __align__(256) unsigned char scratch[kScratchBytes + kRunTableBytes];
+alignas(256) unsigned char host_stage[kStageBytes + kRunTableBytes];
 
 std::mutex g_mu;                       // serialises calls and the per-device lookup
 void* g_scratch[kMaxDevices] = {};     // this process's address of `scratch` on each device
@@ -46,7 +49,7 @@ int scratch_region(int device, void** ptr, size_t* bytes) {
         g_scratch[device] = p;
     }
     *ptr = g_scratch[device];
-    *bytes = kScratchBytes;
+    *bytes = sizeof(scratch);
     return HEXO_OK;
 }
 
@@ -64,7 +67,7 @@ extern "C" int hexo_price_noalloc(hexo_ctx* ctx, const hexo_request* req, double
     mem.region = ctx->scratch;
     mem.region_bytes = ctx->scratch_bytes;
     mem.host = hexo::host_stage;
-    mem.host_bytes = hexo::kStageBytes;
+    mem.host_bytes = sizeof(hexo::host_stage);
     mem.events = false;
     size_t need = 0;
     mem.need = &need;

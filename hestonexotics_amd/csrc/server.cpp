@@ -189,14 +189,17 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         lk.unlock();
         std::unique_ptr<hexo::Batch> b;
         std::string err;
-        hexo_tuning tun = ctx->tuning_now();
-        if (large && (tun.waves_per_simd == 0 || tun.waves_per_simd > kLargeWavesPerSimd))
-            tun.waves_per_simd = kLargeWavesPerSimd;
+        hexo::LaunchPlan plan = hexo::plan_of(ctx->tuning_now());
+        if (large) {
+            uint32_t& waves = plan.shape.waves_per_simd;
+            waves = waves ? std::min(waves, kLargeWavesPerSimd) : kLargeWavesPerSimd;
+            plan.split = false;
+        }
         hexo::BatchMemory mem;
         mem.arena = &arena;
         mem.stage = stages[slot].get();
         mem.events = false;
-        int rc = hexo::batch_create(ctx, reqs.data(), (uint32_t)reqs.size(), streams[slot], mem, b, err, nullptr, &tun);
+        int rc = hexo::batch_create(ctx, reqs.data(), (uint32_t)reqs.size(), streams[slot], mem, b, err, nullptr, &plan);
         if (rc == HEXO_ERR_NOMEM && !flights.empty()) {
             // fragmentation: put the requests back in arrival order and retry when a batch completes
             lk.lock();

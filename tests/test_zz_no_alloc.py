@@ -55,3 +55,32 @@ def test_noalloc_refuses_beyond_its_region(ctx):
     rc, p, s = noalloc(ctx, r)
     assert rc == 0
     np.testing.assert_array_equal(p, ctx.price(r)[0])
+
+
+@pytest.mark.parametrize("flags", [0, H.MARTINGALE])
+def test_noalloc_falls_back_to_the_kernel_with_fewer_partials(ctx, flags):
+    """93,750 tiles x 60 outputs: 86 MiB of partials a tile (the kernel with drawing and stepping waves),
+    43 MiB a pair of tiles (the persistent one): the second fits the region. The same bits."""
+    r = H.Request(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, expiries=[1.0],
+                  strikes=[list(np.linspace(70.0, 130.0, 30))], steps=52, n_paths=6_000_000, seed=4, flags=flags,
+                  payoffs=H.ASIAN | H.EUROPEAN, precision=H.FP32)
+    print("gpu noalloc fallback", flags, flush=True)
+    rc, p, s = noalloc(ctx, r)
+    assert rc == 0, ctx.lib.hexo_ctx_last_error(ctx.h)
+    p_ref, s_ref = ctx.price(r)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(s, s_ref)
+
+
+def test_noalloc_run_tables_do_not_count_against_the_partials(ctx):
+    """4,000 expiries x 1,016 tiles in FP64: 62 MiB of partials, 4,000 run records of 144 bytes (88 when
+    the region was laid out, which it then just held)."""
+    T = list(1.002 ** np.arange(4000))
+    r = H.Request(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, expiries=T, strikes=[[100.0]] * 4000,
+                  steps=1000, n_paths=1016 * 64, seed=4, payoffs=H.ASIAN, precision=H.FP64)
+    print("gpu noalloc run tables", flush=True)
+    rc, p, s = noalloc(ctx, r)
+    assert rc == 0, ctx.lib.hexo_ctx_last_error(ctx.h)
+    p_ref, s_ref = ctx.price(r)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(s, s_ref)
