@@ -772,8 +772,12 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
                                                           (int)block, lds) != hipSuccess ||
             bpc <= 0)
             bpc = std::max(1, 1024 / (int)block);
-        if (cls != 0 && tun.waves_per_simd)
-            bpc = std::max(1, std::min(bpc, (int)(tun.waves_per_simd * 4 * 64 / block)));
+        if (cls != 0) {
+            int most = bpc;
+            if (plan.free_waves) most -= (int)(plan.free_waves * 4 * kTile / block);
+            if (tun.waves_per_simd) most = std::min(most, (int)(tun.waves_per_simd * 4 * kTile / block));
+            bpc = std::max(1, most);
+        }
         const uint64_t waves_per_block = block / kTile;
         const uint64_t need = (b->pa[cls].total_items + waves_per_block - 1) / waves_per_block;
         b->grid[cls] = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(need, (uint64_t)n_cu * (uint64_t)bpc));

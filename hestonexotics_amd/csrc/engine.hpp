@@ -106,11 +106,13 @@ inline uint32_t class_precision(uint32_t cls) { return cls == 0 ? HEXO_FP64 : HE
 inline bool class_martingale(uint32_t cls) { return cls == 2 || cls == 4; }
 inline bool class_geo(uint32_t cls) { return cls >= 3; }
 
-// How a batch's FP32 classes are launched: the persistent kernels' shape, and whether the kernels with
-// drawing and stepping waves may take a class instead (engine.cpp, split_draw_waves).
+// How a batch's FP32 classes are launched: the persistent kernels' shape, whether the kernels with
+// drawing and stepping waves may take a class instead (engine.cpp, split_draw_waves), and how many of
+// the waves per SIMD that a persistent kernel could hold are left to other batches.
 struct LaunchPlan {
     hexo_tuning shape{2, 256, 0, 0};
     bool split = true;
+    uint32_t free_waves = 0;
 };
 // A shape set by the caller is used as given; the default one leaves the choice to the library.
 inline LaunchPlan plan_of(const hexo_tuning& t) { return {t, t.paths_per_thread == 2 && t.waves_per_simd == 0}; }

@@ -10,11 +10,13 @@
 //
 // Large and small requests are kept apart, because a batch's results are ready when its
 // longest request is. A request above kLargeWork path-steps runs in a batch of its own, one such
-// batch at a time, with its grid capped at kLargeWavesPerSimd waves per SIMD (the FP32 kernels
-// hold at most 5). The free wave slot on every SIMD lets a small batch launched later run beside
-// it at once, instead of waiting for the persistent grid to drain. Small requests are batched in
-// arrival order up to kSmallBatchWork path-steps, on the other streams. A large request waiting
-// for its turn does not hold up the small ones behind it.
+// batch at a time, with its grid one wave per SIMD short of what its FP32 kernel could hold and at most
+// kLargeWavesPerSimd: 4 of 5 (96 registers), 3 of 4 for the martingale step (120; at 4 only 32 registers
+// were left and small requests waited for the grid to drain). The free registers on every SIMD let a
+// small batch launched later run beside it at once: tiny requests behind a martingale one of 8e9
+// path-steps are done after 0.4 ms instead of 19, and it takes as long. Small requests are batched in arrival order
+// up to kSmallBatchWork path-steps, on the other streams. A large request waiting for its turn does
+// not hold up the small ones behind it.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -193,6 +195,7 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         if (large) {
             uint32_t& waves = plan.shape.waves_per_simd;
             waves = waves ? std::min(waves, kLargeWavesPerSimd) : kLargeWavesPerSimd;
+            plan.free_waves = 1;
             plan.split = false;
         }
         hexo::BatchMemory mem;

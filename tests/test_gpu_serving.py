@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import hestonexotics_amd as H
+import time
 from hestonexotics_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -208,3 +209,28 @@ def test_small_requests_pass_a_large_one(ctx):
     for r, (p, _, _) in zip(tiny, out_t):
         np.testing.assert_array_equal(p, ctx.price(r)[0])
     np.testing.assert_array_equal(p_big, ctx.price(big)[0])
+
+
+@pytest.mark.parametrize("flags", [0, H.MARTINGALE])
+@pytest.mark.parametrize("params", [dict(kappa=2.0, sigma=0.3), dict(kappa=0.5, sigma=0.9)])
+def test_small_requests_pass_a_large_martingale_one(ctx, flags, params):
+    """As above for a large request with the martingale step, whose kernel holds 4 waves per SIMD: tiny
+    requests (of both FP32 steps) run beside it from the start, not when its grid drains at the end."""
+    say("gpu serving: small requests pass a large martingale one", flags, params)
+    big = H.Request(v0=0.04, theta=0.04, rho=-0.7, S0=100.0, expiries=[2.0], strikes=[[100.0]], steps=4000,
+                    n_paths=2_000_000, seed=3, flags=H.MARTINGALE, precision=H.FP32, **params)
+    tiny = [dataclasses.replace(big, steps=10, n_paths=640, seed=10 + i, flags=flags) for i in range(6)]
+    ctx.server_start(streams=2)
+    try:
+        tb = ctx.submit(big)
+        tt = [ctx.submit(r) for r in tiny]
+        out_t = [ctx.wait(t, r.n_outputs) for t, r in zip(tt, tiny)]
+        _, _, info_big = ctx.wait(tb, big.n_outputs)
+    finally:
+        ctx.server_stop()
+    done_tiny = max(i["done_s"] for _, _, i in out_t) - info_big["arrival_s"]
+    done_big = info_big["done_s"] - info_big["arrival_s"]
+    say(f"  large done after {1e3 * done_big:.1f} ms, tiny after {1e3 * done_tiny:.1f} ms")
+    assert done_tiny < 0.5 * done_big
+    for r, (p, _, _) in zip(tiny, out_t):
+        np.testing.assert_array_equal(p, ctx.price(r)[0])
