@@ -14,9 +14,9 @@
 // kLargeWavesPerSimd: 4 of 5 (96 registers), 3 of 4 for the martingale step (120; at 4 only 32 registers
 // were left and small requests waited for the grid to drain). The free registers on every SIMD let a
 // small batch launched later run beside it at once: tiny requests behind a martingale one of 8e9
-// path-steps are done after 0.4 ms instead of 19, and it takes as long. Small requests are batched in arrival order
-// up to kSmallBatchWork path-steps, on the other streams. A large request waiting for its turn does
-// not hold up the small ones behind it.
+// path-steps are done after 0.4 ms instead of 19, and it takes as long. Small requests are batched
+// in arrival order up to kSmallBatchWork path-steps, on the other streams. A large request waiting
+// for its turn does not hold up the small ones behind it.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -41,6 +41,7 @@ struct hexo_server_state {
         uint64_t n_out = 0;
         double work = 0.0;  // request_work
         bool large = false;
+        bool building = false;  // its batch is being tried without the lock: launched, failed or queued again after
     };
     struct Flight {
         std::unique_ptr<hexo::Batch> b;
@@ -71,6 +72,7 @@ struct hexo_server_state {
     size_t budget = 0, reserved = 0, peak = 0;
     hexo_server_stats st{};
     uint32_t inject_launch = 0, inject_admit = 0;
+    uint32_t cancelling = 0;  // cancels that wait for a batch being built
     uint32_t batch_counter = 0;
     std::string worker_error;
 
@@ -185,9 +187,11 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         // launch calls), so that requests keep arriving meanwhile and the next batch takes them
         // together: with the lock held every submission waited for a launch and short requests ran
         // one or two to a batch (bursts of 2 to 48 requests of 1e3 to 4e5 paths took 1.0 to 1.7 times
-        // as long). The taken tickets are past cancelling, and only this thread touches the flights.
+        // as long). Only this thread touches the flights; a cancel of a taken ticket waits for the
+        // outcome, since a batch that finds no memory goes back to the queue.
         const bool fail_launch = inject_launch != 0;
-        for (uint64_t id : ids) tickets[id]->state = 1;
+        for (uint64_t id : ids) tickets[id]->building = true;
+        reserved += bytes;
         lk.unlock();
         std::unique_ptr<hexo::Batch> b;
         std::string err;
@@ -206,11 +210,13 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         if (rc == HEXO_ERR_NOMEM && !flights.empty()) {
             // fragmentation: put the requests back in arrival order and retry when a batch completes
             lk.lock();
+            reserved -= bytes;
             for (uint64_t id : ids) {
-                tickets[id]->state = 0;
+                tickets[id]->building = false;
                 queue.push_back(id);
             }
             std::sort(queue.begin(), queue.end());  // ticket ids grow with arrival
+            if (cancelling) cv.notify_all();
             return;
         }
         const bool injected = rc == HEXO_OK && fail_launch;
@@ -230,21 +236,23 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         }
         lk.lock();
         ++batch_counter;
+        for (uint64_t id : ids) tickets[id]->building = false;
+        if (cancelling || rc != HEXO_OK) cv.notify_all();
         if (rc != HEXO_OK) {
+            reserved -= bytes;
             if (injected && inject_launch) --inject_launch;
             worker_error = err;
             for (uint64_t id : ids) fail_ticket(*tickets[id], rc);
-            cv.notify_all();
             continue;
         }
         for (uint64_t id : ids) {
             Ticket& t = *tickets[id];
+            t.state = 1;
             t.info.admit_s = t_admit;
             t.info.launch_s = t_launch;
             t.info.batch_id = batch_counter;
             t.info.batch_size = (uint32_t)ids.size();
         }
-        reserved += bytes;
         peak = std::max(peak, reserved);
         st.batches++;
         slot_busy[slot] = true;
@@ -429,12 +437,18 @@ int hexo_cancel(hexo_ctx* ctx, uint64_t ticket) {
     if (!ctx) return HEXO_ERR_INVALID;
     const std::shared_ptr<hexo_server_state> s = ctx->server_ref();
     if (!s) return ctx->set_error(HEXO_ERR_STATE, "server not running");
-    std::lock_guard<std::mutex> lk(s->mu);
+    std::unique_lock<std::mutex> lk(s->mu);
     auto it = s->tickets.find(ticket);
     if (it == s->tickets.end()) return HEXO_ERR_NOT_FOUND;
-    if (it->second->state != 0) return ctx->set_error(HEXO_ERR_STATE, "ticket already launched or finished");
+    const std::shared_ptr<hexo_server_state::Ticket> t = it->second;
+    ++s->cancelling;
+    s->cv.wait(lk, [&] { return !t->building; });
+    --s->cancelling;
+    it = s->tickets.find(ticket);  // a waiter may have consumed it meanwhile
+    if (it == s->tickets.end()) return HEXO_ERR_NOT_FOUND;
+    if (t->state != 0) return ctx->set_error(HEXO_ERR_STATE, "ticket already launched or finished");
     s->queue.erase(std::remove(s->queue.begin(), s->queue.end(), ticket), s->queue.end());
-    fail_ticket(*it->second, HEXO_ERR_CANCELLED);
+    fail_ticket(*t, HEXO_ERR_CANCELLED);
     s->st.cancelled++;
     s->cv.notify_all();
     return HEXO_OK;

@@ -234,3 +234,33 @@ def test_small_requests_pass_a_large_martingale_one(ctx, flags, params):
     assert done_tiny < 0.5 * done_big
     for r, (p, _, _) in zip(tiny, out_t):
         np.testing.assert_array_equal(p, ctx.price(r)[0])
+
+
+def test_cancel_of_a_ticket_that_does_not_fit_yet(ctx):
+    """A request that finds the arena's free space in two pieces goes back to the queue until a batch
+    completes; a cancel that arrives while its batch is being tried takes effect. The arena: 24 MB of
+    a finished request, 16 MB of a running one, 24 MB free, a request of 32 MB waiting."""
+    def req(tiles, steps, n_strikes=100, **kw):
+        return H.Request(v0=0.04, theta=0.04, rho=-0.7, kappa=2.0, sigma=0.3, S0=100.0, expiries=[1.0],
+                         strikes=[list(np.linspace(70.0, 130.0, n_strikes))], steps=steps, n_paths=64 * tiles,
+                         payoffs=H.ASIAN, **kw)
+    first = req(15_000, 1000, seed=1, precision=H.FP32)       # about 2 ms, in the arena's first 24 MB
+    running = req(10_000, 100_000, seed=2, precision=H.FP64)  # about half a second, behind it
+    waiting = req(20_000, 2, seed=3, precision=H.FP32)
+    say("gpu serving: cancel while a batch is tried")
+    ctx.server_start(memory_budget_bytes=64_500_000, streams=3)
+    try:
+        tf, tr = ctx.submit(first), ctx.submit(running)
+        ctx.wait(tf, first.n_outputs)
+        for _ in range(20):
+            t = ctx.submit(waiting)
+            time.sleep(0.002)
+            ctx.cancel(t)
+            with pytest.raises(H.HexoError) as e:
+                ctx.wait(t, waiting.n_outputs)
+            assert e.value.code == -7  # HEXO_ERR_CANCELLED
+        assert not ctx.poll(tr), "the running request ended before the cancels"
+        assert ctx.server_stats()["cancelled"] == 20
+        ctx.wait(tr, running.n_outputs)
+    finally:
+        ctx.server_stop()
