@@ -49,7 +49,7 @@ int run_single(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, double* pric
     if (rc == HEXO_ERR_NOMEM && need) {
         // grow; the arena is empty, every earlier call's batch being complete and released
         const size_t grown = std::max<size_t>({need, (size_t)16 << 20, 2 * ctx->sync_arena.capacity()});
-        hexo::LaunchPlan plan = hexo::plan_of(ctx->tuning_now());
+        hexo::LaunchPlan plan = ctx->plan_now();
         if (!ctx->sync_arena.init(grown) && !ctx->sync_arena.init(need)) {
             // half the partials with the persistent kernels
             plan.split = false;
@@ -445,7 +445,7 @@ int hexo_normals(hexo_ctx* ctx, const uint32_t* words, uint64_t n, uint32_t prec
 
 int hexo_get_tuning(hexo_ctx* ctx, hexo_tuning* t) {
     if (!ctx || !t) return HEXO_ERR_INVALID;
-    *t = ctx->tuning_now();
+    *t = ctx->plan_now().shape;
     return HEXO_OK;
 }
 
@@ -455,7 +455,7 @@ int hexo_set_tuning(hexo_ctx* ctx, const hexo_tuning* t) {
     if (!(p >= 1 && p <= 4)) return ctx->set_error(HEXO_ERR_INVALID, "paths_per_thread must be 1, 2, 3 or 4");
     if (!(b == 64 || b == 128 || b == 256)) return ctx->set_error(HEXO_ERR_INVALID, "block_threads must be 64, 128 or 256");
     if (t->waves_per_simd > 8) return ctx->set_error(HEXO_ERR_INVALID, "waves_per_simd must be <= 8");
-    ctx->set_tuning(*t);
+    ctx->set_plan(hexo::plan_of(*t));
     return HEXO_OK;
 }
 
@@ -466,8 +466,10 @@ int hexo_autotune(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, uint32_t 
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
     DeviceGuard dg(ctx->device);
     // trial shapes are passed to the batches directly: the context's shape (which the serving
-    // thread may be reading) changes once, to the winner
-    hexo_tuning winner = ctx->tuning_now();
+    // thread may be reading) changes once, to the winner. A shape is the persistent kernels', so the
+    // trials run on them whatever the size of the batch, and the kernels with drawing and stepping
+    // waves keep their choice of small batches afterwards.
+    hexo_tuning winner = ctx->plan_now().shape;
     double best_ms = 1e300;
     const uint32_t ppts[] = {1, 2, 3, 4};
     const uint32_t blocks[] = {64, 128, 256};
@@ -476,7 +478,7 @@ int hexo_autotune(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, uint32_t 
         for (uint32_t b : blocks)
             for (uint32_t w : waves) {
                 const hexo_tuning trial{p, b, w, 0};
-                const hexo::LaunchPlan plan = hexo::plan_of(trial);
+                const hexo::LaunchPlan plan{trial, false, 0};
                 std::string err;
                 std::unique_ptr<hexo::Batch> bt;
                 int rc = hexo::batch_create(ctx, reqs, n, ctx->stream, hexo::BatchMemory(), bt, err, nullptr, &plan);
@@ -495,7 +497,7 @@ int hexo_autotune(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, uint32_t 
                     winner = trial;
                 }
             }
-    ctx->set_tuning(winner);
+    ctx->set_plan({winner, true, 0});
     if (best) *best = winner;
     return HEXO_OK;
 }

@@ -393,7 +393,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         err = "empty batch";
         return HEXO_ERR_INVALID;
     }
-    const LaunchPlan plan = given ? *given : plan_of(ctx->tuning_now());
+    const LaunchPlan plan = given ? *given : ctx->plan_now();
     const hexo_tuning& tun = plan.shape;
     std::vector<ReqPlan> plans(n);
     uint64_t n_seg = 0, n_fin = 0, n_opt = 0, n_partials = 0, n_groups = 0, n_out = 0;

@@ -164,7 +164,8 @@ struct hexo_ctx {
     int device = 0;
     hipDeviceProp_t prop{};
     hipStream_t stream = nullptr;
-    hexo_tuning tuning{2, 256, 0, 0};  // guarded by tuning_mu: the serving thread reads it too
+    // the launch plan of calls that bring none, guarded by tuning_mu: the serving thread reads it too
+    hexo::LaunchPlan plan;
     std::mutex tuning_mu;
     std::recursive_mutex mu;
     std::mutex err_mu;  // guards last_error: failures may be reported from several threads at once
@@ -199,14 +200,14 @@ struct hexo_ctx {
         last_error = msg;
         return code;
     }
-    hexo_tuning tuning_now() {
+    hexo::LaunchPlan plan_now() {
         std::lock_guard<std::mutex> g(tuning_mu);
-        return tuning;
+        return plan;
     }
-    void set_tuning(const hexo_tuning& t) {
+    void set_plan(const hexo::LaunchPlan& p) {
         std::lock_guard<std::mutex> g(tuning_mu);
-        tuning = t;
-        tuning.reserved = 0;
+        plan = p;
+        plan.shape.reserved = 0;
     }
     std::shared_ptr<struct hexo_server_state> server_ref() {
         std::lock_guard<std::mutex> g(server_mu);

@@ -195,7 +195,7 @@ void hexo_server_state::launch_ready(std::unique_lock<std::mutex>& lk) {
         lk.unlock();
         std::unique_ptr<hexo::Batch> b;
         std::string err;
-        hexo::LaunchPlan plan = hexo::plan_of(ctx->tuning_now());
+        hexo::LaunchPlan plan = ctx->plan_now();
         if (large) {
             uint32_t& waves = plan.shape.waves_per_simd;
             waves = waves ? std::min(waves, kLargeWavesPerSimd) : kLargeWavesPerSimd;

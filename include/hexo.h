@@ -109,7 +109,7 @@ typedef struct hexo_request {
 /* Launch shape of the FP32 path kernel. Results do not depend on it: every 64-path tile is
  * reduced on its own and tiles are combined in a fixed order. With 2 paths per thread and no cap
  * (the default) the library runs batches too small to fill the GPU on a kernel with more waves per
- * tile instead; any other shape is used as given. */
+ * tile instead; any other shape set by the caller is used as given. */
 typedef struct hexo_tuning {
     uint32_t paths_per_thread; /* 1, 2, 3 or 4 */
     uint32_t block_threads;    /* 64, 128 or 256 */
@@ -215,8 +215,9 @@ int hexo_normals(hexo_ctx* ctx, const uint32_t* words, uint64_t n, uint32_t prec
 /* ---- launch shape ---- */
 int hexo_get_tuning(hexo_ctx* ctx, hexo_tuning* t);
 int hexo_set_tuning(hexo_ctx* ctx, const hexo_tuning* t);
-/* Times the candidate launch shapes on the given requests and keeps the fastest;
- * *best receives it. reps: timed repetitions per candidate (>= 1). */
+/* Times the candidate launch shapes of the persistent FP32 kernels on the given requests and keeps the
+ * fastest; *best receives it. reps: timed repetitions per candidate (>= 1). Batches too small to fill
+ * the GPU stay on the kernels with more waves per tile, unlike after hexo_set_tuning with that shape. */
 int hexo_autotune(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, uint32_t reps, hexo_tuning* best);
 
 /* ---- measurement ---- */

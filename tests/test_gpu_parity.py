@@ -533,3 +533,34 @@ def test_fp64_normals_of_a_wavefront(ctx, oracle, n_tail):
     w[rng.permutation(256)[:n_tail]] = tail_words(n_tail)
     for words in (w, np.concatenate([w, w[::-1], w[:37]])):
         np.testing.assert_allclose(ctx.normals(words, H.FP64), oracle.normals_f64(words), rtol=2e-15, atol=1e-15)
+
+
+def test_autotuner_leaves_small_calls_on_their_kernel(ctx):
+    """The tuned shape is the persistent kernel's; a small batch keeps the kernel with drawing and
+    stepping waves (four times as fast at 1e4 paths), whichever shape wins."""
+    say("gpu autotune, small calls after")
+    small = W.c1(n_paths=10_000, precision=H.FP32)
+    base = ctx.get_tuning()
+
+    def path_ms():
+        b = ctx.batch([small])
+        times = []
+        for _ in range(5):
+            b.run_eager()
+            b.sync()
+            times.append(b.stats()["path_kernel_ms"])
+        b.close()
+        return min(times)
+
+    before = path_ms()
+    try:
+        for n_paths in (20_000, 10_000_000):
+            best = ctx.autotune(W.c2(n_paths=n_paths, maturities=[0.5], n_strikes=8, precision=H.FP32), reps=1)
+            after = path_ms()
+            say(f"  tuned on {n_paths} paths: {best}, small call {1e3 * before:.0f} -> {1e3 * after:.0f} us")
+            assert after < 2.0 * before
+        shape = dict(paths_per_thread=1, block_threads=64, waves_per_simd=0)
+        ctx.set_tuning(**shape)  # a shape given by the caller is used as given
+        assert path_ms() > 2.0 * before
+    finally:
+        ctx.set_tuning(**base)
