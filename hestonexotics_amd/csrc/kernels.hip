@@ -787,7 +787,8 @@ __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32
 // the fifth wave more (1,000 strikes x 3 payoffs x 52 steps, 3.5e6 paths 3.79 -> 3.30 ms with it).
 template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 && (!MART || GEO) ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
-    extern __shared__ uint32_t lds_u32[];
+    extern __shared__ __align__(16) uint32_t lds_u32[];
+    static_assert(__alignof__(lds_u32) >= alignof(float4), "path_fp32 stores float4 there");
     const int lane = (int)(threadIdx.x & 63u);
     // the wave's LDS region, at a wave-uniform address
     uint32_t* lds = lds_u32 + uniform(threadIdx.x >> 6) * WaveLds<PPT>::kWords;
@@ -853,7 +854,8 @@ __device__ __forceinline__ uint32_t stepping_first(uint32_t wave, uint32_t item,
 template <uint32_t NP, uint32_t C, bool MART, bool GEO>
 __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
     __shared__ DrawChunk<C> buf[2];
-    __shared__ uint32_t vals[WaveLds<1>::kWords];
+    __shared__ __align__(16) uint32_t vals[WaveLds<1>::kWords];
+    static_assert(__alignof__(vals) >= alignof(float4), "path_fp32 stores float4 there");
     const int lane = (int)(threadIdx.x & 63u);
     const uint32_t item = blockIdx.x;
     const uint32_t sp = uniform(find_sorted(a.item_end, a.n_sorted, item));
