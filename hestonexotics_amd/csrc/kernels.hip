@@ -25,6 +25,14 @@
 #include "kernels.hpp"
 #include "layout.hpp"
 
+// No implicit FMA contraction in this file: every fused multiply-add is written out. With contraction
+// the compiler fuses a product into a later add only where both land in one basic block, which depends
+// on how each instance of a kernel is laid out (one FP32 path per thread flattens the quadratic branch
+// and turned tt - 1 into fma(m^2, 1/s2h, -1); a branch added to the FP64 step changed which of its
+// sums were fused), so results would change by an ulp with the launch shape or the batch that a
+// request is in.
+#pragma clang fp contract(off)
+
 namespace hexo {
 
 namespace {
@@ -76,6 +84,13 @@ struct CompF {
     __device__ __forceinline__ void add(float x) {
         const float t = s + x;
         c += (__builtin_fabsf(s) >= __builtin_fabsf(x)) ? (s - t) + x : (x - t) + s;
+        s = t;
+    }
+    // x^2 enters every sum unrounded. (Fused by the compiler in some of them only, a wave's first square
+    // had its rounding error counted twice: standard errors off by 1.1e-8 on average, now 4.9e-9.)
+    __device__ __forceinline__ void add_square(float x) {
+        const float t = __builtin_fmaf(x, x, s);
+        c += (__builtin_fabsf(s) >= x * x) ? __builtin_fmaf(x, x, s - t) : __builtin_fmaf(x, x, -t) + s;
         s = t;
     }
     __device__ __forceinline__ void merge(float s2, float c2) {
@@ -140,7 +155,7 @@ struct TileSums<float> {  // compensated FP32 sums (HEXO_FP32_COMPENSATED)
     CompF s{0.f, 0.f}, ss{0.f, 0.f};
     __device__ __forceinline__ void add(float x) {
         s.add(x);
-        ss.add(x * x);
+        ss.add_square(x);
     }
     __device__ __forceinline__ void combine(const TileSums& o) {
         s.merge(o.s.s, o.s.c);
@@ -341,12 +356,6 @@ __device__ __forceinline__ void count_flush(unsigned long long* counts, uint32_t
 // ------------------------------------------------------------------------------------------
 // FP32 path kernel
 // ------------------------------------------------------------------------------------------
-// No implicit FMA contraction in the FP32 path: every fused multiply-add below is written out.
-// With contraction the compiler fuses a product into a later add only where both land in one basic
-// block, which depends on how each paths-per-thread instance is laid out (one path per thread
-// flattens the quadratic branch and turned tt - 1 into fma(m^2, 1/s2h, -1)), so the paths would
-// change by an ulp with the launch shape.
-#pragma clang fp contract(off)
 struct SegF {
     float omd, th, c1h, c2h, g0, ka, kb, k3;
     float mA, ma, mh, mr;
@@ -869,7 +878,6 @@ __global__ __launch_bounds__(64 * (NP + 1)) void k_path_fp32_split(PathArgs a) {
         draw_fp32<NP, C>(a.reqs[ri], tile, lane, role - 1, buf);
     }
 }
-#pragma clang fp contract(fast)
 // ------------------------------------------------------------------------------------------
 // Plain FP64 path kernel: the reference's step and policies in FP64 (src/HSimulation.tpp:52-86) with
 // the expressions that depend on the run only (e^-kappa dt, the variance's coefficients, K0..K4)
@@ -912,20 +920,23 @@ __device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, dou
     double k0 = c.k0;
     if (R.flags & kMartingale) {
         // Andersen's martingale-corrected K0* = -ln E[exp(A V') | V] - (K1 + K3/2) V, A = K2 + K4/2
-        const double A = c.k2 + 0.5 * c.k3;
-        const double beta = (m + m) / sm;
-        if (quad && 2.0 * A * aq < 1.0) {
-            const double lnM = A * bp2 * aq / (1.0 - 2.0 * A * aq) - 0.5 * ::log1p(-2.0 * A * aq);
-            k0 = -lnM - (c.k1 + 0.5 * c.k3) * Vp + R.r_drift * c.delta;
-        } else if (!quad && A < beta) {
+        const double A = __builtin_fma(0.5, c.k3, c.k2), K1h = __builtin_fma(0.5, c.k3, c.k1);
+        double lnM = 0.0;
+        bool exists;
+        if (quad) {
+            exists = 2.0 * A * aq < 1.0;
+            lnM = A * bp2 * aq / (1.0 - 2.0 * A * aq) - 0.5 * ::log1p(-2.0 * A * aq);
+        } else {
+            const double beta = (m + m) / sm;
+            exists = A < beta;
             const double omp = (m2 + m2) / sm;  // 1 - p
-            const double lnM = ::log((1.0 - omp) + beta * omp / (beta - A));
-            k0 = -lnM - (c.k1 + 0.5 * c.k3) * Vp + R.r_drift * c.delta;
+            lnM = ::log((1.0 - omp) + beta * omp / (beta - A));
         }
+        if (exists) k0 = __builtin_fma(R.r_drift, c.delta, __builtin_fma(-K1h, Vp, -lnM));
     }
     // V = V' = 0 makes the diffusion's variance 0: the floor keeps the root finite and moves nothing
     const double var = __builtin_fmax(__builtin_fma(c.k3, Vp, c.k3 * V), 1e-300);
-    logX = __builtin_fma(sqrt_f64(var), zx, logX + k0 + c.k1 * Vp + c.k2 * V);
+    logX = __builtin_fma(sqrt_f64(var), zx, __builtin_fma(c.k2, V, __builtin_fma(c.k1, Vp, logX + k0)));
     return quad;
 }
 
@@ -1030,8 +1041,8 @@ __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32
                 }
             }
             if (i + 1u < n) {
-                acc += c.delta * 0.5 * (X + Xp);  // AAsianCallNonAdaptive::accumulate_value
-                if (geo) accY += c.delta * 0.5 * ((logX - R.log_S0) + yp);
+                acc = __builtin_fma(c.delta * 0.5, X + Xp, acc);  // AAsianCallNonAdaptive::accumulate_value
+                if (geo) accY = __builtin_fma(c.delta * 0.5, (logX - R.log_S0) + yp, accY);
             }
         }
         for (uint32_t f = 0; f < S.fin_count; ++f) {
@@ -1043,7 +1054,8 @@ __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32
             if (geo) {
                 // the same functional on y, normalised by its weight sum W: G = W S0 exp(L / W)
                 const double y = logX - R.log_S0, wf = (F.T - F.tp) / F.dt;
-                const double L = (R.flags & kTrapezoid) ? (accY + (F.T - F.tp) * 0.5 * (yp + (yp + (y - yp) * wf))) / F.T
+                const double yt = __builtin_fma(y - yp, wf, yp);
+                const double L = (R.flags & kTrapezoid) ? (accY + (F.T - F.tp) * 0.5 * (yp + yt)) / F.T
                                                         : (accY + (y - yp) * wf) / F.T;
                 G = F.gW * R.S0 * ::exp(L / F.gW);
             }
@@ -1061,8 +1073,8 @@ __device__ __forceinline__ void path_fp64(const PathArgs& a, uint32_t ri, uint32
             reduce_tiles<1>(a, R, F, tile, lane, vals, nan);
             wave_sync_lds();
         }
-        acc += S.dnext * 0.5 * (X + Xp);
-        if (geo) accY += S.dnext * 0.5 * ((logX - R.log_S0) + yp);
+        acc = __builtin_fma(S.dnext * 0.5, X + Xp, acc);
+        if (geo) accY = __builtin_fma(S.dnext * 0.5, (logX - R.log_S0) + yp, accY);
     }
     if constexpr (COUNT) count_flush(a.counts, cq, ce, cc, ct, lane);
 }
@@ -1258,7 +1270,7 @@ __device__ __forceinline__ void output_sums(const void* sums, size_t first, uint
 // Sample mean and variance (n - 1 denominator, clamped at 0) from a sum and a sum of squares.
 __device__ __forceinline__ void mean_var(double s, double ss, double n, double& mean, double& var) {
     mean = s / n;
-    var = n > 1.0 ? (ss - n * mean * mean) / (n - 1.0) : 0.0;
+    var = n > 1.0 ? __builtin_fma(-(n * mean), mean, ss) / (n - 1.0) : 0.0;
     var = var > 0.0 ? var : 0.0;
 }
 
@@ -1331,15 +1343,15 @@ __global__ __launch_bounds__(256) void k_reduce_final(ReduceArgs a, uint64_t tot
     const double n = (double)R.n_paths;
     double mean, var;
     mean_var(s, ss, n, mean, var);
-    double price = scale * mean + (cv ? a.geo[R.out_base + o] : 0.0);
+    double price = __builtin_fma(scale, mean, cv ? a.geo[R.out_base + o] : 0.0);
     if (reg) {
         double ma, va, mg, vg;
         mean_var(sa, ssa, n, ma, va);
         mean_var(sg, ssg, n, mg, vg);
         const double cov = 0.5 * (va + vg - var);
         const double beta = vg > 0.0 ? cov / vg : 0.0;
-        price = scale * ma - beta * (scale * mg - a.geo[R.out_base + o]);
-        var = va - beta * cov;
+        price = __builtin_fma(scale, ma, -(beta * __builtin_fma(scale, mg, -a.geo[R.out_base + o])));
+        var = __builtin_fma(-beta, cov, va);
         var = var > 0.0 ? var : 0.0;
     }
     a.prices[R.out_base + o] = disc * price;
