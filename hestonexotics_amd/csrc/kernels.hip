@@ -922,11 +922,11 @@ __device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, dou
         // Andersen's martingale-corrected K0* = -ln E[exp(A V') | V] - (K1 + K3/2) V, A = K2 + K4/2
         const double A = __builtin_fma(0.5, c.k3, c.k2), K1h = __builtin_fma(0.5, c.k3, c.k1);
         double lnM = 0.0;
-        bool exists;
+        bool exists = false;
         if (quad) {
             exists = 2.0 * A * aq < 1.0;
             lnM = A * bp2 * aq / (1.0 - 2.0 * A * aq) - 0.5 * ::log1p(-2.0 * A * aq);
-        } else {
+        } else if (sm > 0.0) {  // where m^2 and s2 underflow to 0 there is no psi: the uncorrected step
             const double beta = (m + m) / sm;
             exists = A < beta;
             const double omp = (m2 + m2) / sm;  // 1 - p

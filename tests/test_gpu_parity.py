@@ -564,3 +564,12 @@ def test_autotuner_leaves_small_calls_on_their_kernel(ctx):
         assert path_ms() > 2.0 * before
     finally:
         ctx.set_tuning(**base)
+
+
+def test_fp64_martingale_of_a_vanishing_variance(ctx, oracle):
+    """A variance of 1e-170: m^2 and s2 underflow to 0, psi is 0 / 0, and the step is the uncorrected one."""
+    req = H.Request(v0=1e-170, theta=1e-170, rho=-0.7, kappa=2.0, sigma=1e-80, S0=100.0, expiries=[0.5],
+                    strikes=[[100.0]], steps=26, n_paths=130, seed=13, flags=H.MARTINGALE, precision=H.FP64)
+    o = oracle_for(oracle, req)["finals"]
+    assert np.isfinite(o).all()
+    np.testing.assert_allclose(ctx.paths(req, 0, req.n_paths), o, rtol=1e-12)
