@@ -894,6 +894,13 @@ struct SegD {
     double e, s2v, s2c, k0, k1, k2, k3, delta;
 };
 
+// a / b, for a b that may be subnormal where `tiny`: div_f64's reciprocal of it overflows.
+__device__ __forceinline__ double div_tiny_f64(double a, double b, bool tiny) {
+    double q = div_f64(a, b);
+    if (__builtin_amdgcn_ballot_w64(tiny)) q = tiny ? a / b : q;
+    return q;
+}
+
 __device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, double& V, double& logX, uint32_t wv,
                                              double zv, double zx) {
     const double m = __builtin_fma(V - R.theta, c.e, R.theta);
@@ -901,9 +908,10 @@ __device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, dou
     const double m2 = m * m;
     const double Vp = V;
     const bool quad = s2 < 1.5 * m2;  // psi = s2 / m^2 < 1.5
+    const bool tiny = s2 < 1e-290;    // so that (s2 + m^2)(1 - U) is normal where this is false
     double aq = 0.0, bp2 = 0.0, sm = 0.0, arg = 0.0;
     if (quad) {
-        const double tt = div_f64(m2 + m2, s2);  // 2 / psi
+        const double tt = div_tiny_f64(m2 + m2, s2, tiny);  // 2 / psi
         const double tm1 = tt - 1.0;
         bp2 = tm1 + sqrt_f64(tt * tm1);
         aq = div_f64(m, 1.0 + bp2);
@@ -913,7 +921,7 @@ __device__ __forceinline__ bool qe_step_fp64(const DevReq& R, const SegD& c, dou
         // p = (psi - 1)/(psi + 1), beta = 2/(m (psi + 1)): with sm = s2 + m^2, 1 - p = 2 m^2/sm and
         // 1/beta = sm/(2 m). U > p exactly when arg = (1 - p)/(1 - U) > 1; 1 - U comes from ~k
         sm = s2 + m2;
-        arg = div_f64(m2 + m2, sm * uniform_f64(~wv));
+        arg = div_tiny_f64(m2 + m2, sm * uniform_f64(~wv), tiny);
         const double v = log_f64(arg) * div_f64(sm, m + m);
         V = arg > 1.0 ? v : 0.0;
     }

@@ -573,3 +573,13 @@ def test_fp64_martingale_of_a_vanishing_variance(ctx, oracle):
     o = oracle_for(oracle, req)["finals"]
     assert np.isfinite(o).all()
     np.testing.assert_allclose(ctx.paths(req, 0, req.n_paths), o, rtol=1e-12)
+
+
+def test_fp64_subnormal_conditional_variance(ctx, oracle):
+    """s2 = Var[V' | V] = 1e-311 at psi = s2 / m^2 = 1e-151: the reciprocal of s2 overflows, the quotient
+    2 m^2 / s2 does not."""
+    req = H.Request(v0=1e-80, theta=1e-80, rho=0.0, kappa=2.0, sigma=2.3e-115, S0=100.0, expiries=[0.5],
+                    strikes=[[100.0]], steps=26, n_paths=130, seed=13, precision=H.FP64)
+    o = oracle_for(oracle, req)["finals"]
+    assert np.isfinite(o).all()
+    np.testing.assert_allclose(ctx.paths(req, 0, req.n_paths), o, rtol=1e-12)
