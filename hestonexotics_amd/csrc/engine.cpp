@@ -318,14 +318,23 @@ uint64_t split_most_tiles(const ReqPlan& p) {
 //    persistent; 50,000 paths 214, 195, 286); up to 3,328: one (k_path_fp64_split).
 //  * with the correction up to 256 tiles (1e4 paths: 223 us against 392, stiff parameters 332 against
 //    500; at 313 tiles stiff 521 against 501, at 1,563 and one drawing wave 610 against 561).
-uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, uint64_t most_tiles, bool martingale, bool long_steps,
-                          bool fp32_split) {
-    if (tiles > most_tiles) return 0;
+// Requests of 2^31 steps and more stay on the persistent kernel: a drawing wave counts the request's
+// steps in 32 bits. Less than a chunk below 2^32 its count would wrap and never end; beyond, it would meet
+// fewer barriers than the stepping wave, which counts run by run.
+constexpr uint64_t kSplitMaxSteps = 1ull << 31;
+constexpr uint32_t split_draw_waves(uint32_t cls, uint64_t tiles, uint64_t most_tiles, uint64_t most_steps,
+                                    bool martingale, bool long_steps, bool fp32_split) {
+    if (tiles > most_tiles || most_steps >= kSplitMaxSteps) return 0;
     if (cls == 0) return tiles > (martingale ? 256u : 3328u) ? 0 : tiles <= 512 ? 2 : 1;
     if (!fp32_split) return 0;
     if (tiles > (long_steps ? 2048u : class_geo(cls) ? 1u << 16 : 1u << 17)) return 0;
     return tiles <= 512 ? 2 : 1;
 }
+static_assert(kSplitMaxSteps <= 1ull << 31 && split_draw_waves(0, 1, 1, kSplitMaxSteps - 1, false, false, true) == 2 &&
+                  split_draw_waves(1, 1, 1, kSplitMaxSteps - 1, false, false, true) == 2 &&
+                  split_draw_waves(0, 1, 1, kSplitMaxSteps, false, false, true) == 0 &&
+                  split_draw_waves(1, 1, 1, (1ull << 32) + 2, false, false, true) == 0,
+              "a step count near or past 2^32 never reaches the drawing waves");
 
 bool plan_request(const hexo_request* r, ReqPlan& p) {
     if (!build_schedule(r->expiries, r->n_expiries, r->n_strikes, r->steps, p.segs, p.total_steps)) return false;
@@ -399,7 +408,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint64_t n_seg = 0, n_fin = 0, n_opt = 0, n_partials = 0, n_groups = 0, n_out = 0;
     uint64_t n_geo_items = 0, n_geo_pts = 0, n_geo_waves = 0;
     uint32_t n_cls[kPathClasses] = {};
-    uint64_t cls_tiles[kPathClasses] = {};
+    uint64_t cls_tiles[kPathClasses] = {}, cls_steps[kPathClasses] = {};
     uint64_t cls_most[kPathClasses];  // split_most_tiles over the class's requests
     std::fill(cls_most, cls_most + kPathClasses, ~0ull);
     bool cls_mart[kPathClasses] = {}, cls_long[kPathClasses] = {};  // requests with longer steps (split_draw_waves)
@@ -428,6 +437,7 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
         n_out += p.n_out;
         n_cls[p.cls]++;
         cls_tiles[p.cls] += p.n_tiles;
+        cls_steps[p.cls] = std::max(cls_steps[p.cls], p.total_steps);
         cls_most[p.cls] = std::min(cls_most[p.cls], split_most_tiles(p));
         const bool mart = (reqs[i].flags & HEXO_MARTINGALE) != 0;
         cls_mart[p.cls] |= mart;
@@ -440,7 +450,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     uint32_t cls_draw[kPathClasses];
     bool fp32_split = false;
     for (uint32_t cls = 0; cls < kPathClasses; ++cls) {
-        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_most[cls], cls_mart[cls], cls_long[cls], plan.split);
+        cls_draw[cls] = split_draw_waves(cls, cls_tiles[cls], cls_most[cls], cls_steps[cls], cls_mart[cls], cls_long[cls],
+                                         plan.split);
         fp32_split |= cls != 0 && n_cls[cls] && cls_draw[cls];
         cls_ppt[cls] = cls == 0 || cls_draw[cls] ? 1u : tun.paths_per_thread;
         cls_store[cls] = kChunkTiles % cls_ppt[cls] == 0 ? cls_ppt[cls] : 1u;

@@ -102,9 +102,9 @@ struct PinnedBuf {
 // kernel classes: 0 = FP64 kernel; FP32 kernels 1 + (martingale-corrected step) + 2 (geometric
 // control variate's accumulation)
 constexpr uint32_t kPathClasses = 5;
-inline uint32_t class_precision(uint32_t cls) { return cls == 0 ? HEXO_FP64 : HEXO_FP32; }
-inline bool class_martingale(uint32_t cls) { return cls == 2 || cls == 4; }
-inline bool class_geo(uint32_t cls) { return cls >= 3; }
+constexpr uint32_t class_precision(uint32_t cls) { return cls == 0 ? HEXO_FP64 : HEXO_FP32; }
+constexpr bool class_martingale(uint32_t cls) { return cls == 2 || cls == 4; }
+constexpr bool class_geo(uint32_t cls) { return cls >= 3; }
 
 // How a batch's FP32 classes are launched: the persistent kernels' shape, whether the kernels with
 // drawing and stepping waves may take a class instead (engine.cpp, split_draw_waves), and how many of
