@@ -405,12 +405,13 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
         ctx->swift_stream = nullptr;
         return ctx->set_error(HEXO_ERR_HIP, "hipStreamCreate failed");
     }
-    // Work arrays of each class for a pass of up to 256 or 1,024 chains, each chain with room for the
-    // largest J of its class: no second look at J, and the two streams share nothing that is written.
+    // Work arrays of each class for a pass of up to 256 or 1,024 of the call's chains, each chain with
+    // room for the largest J of its class: no second look at J, and the two streams share nothing that is
+    // written. (How many chains each class gets changes from call to call of a calibration; n does not.)
     const uint32_t rows = grads ? 6u : 1u;
     constexpr uint32_t kBigPass = 256, kSmallPass = 1024;
     const size_t row_bytes[2] = {sizeof(hexo::Cplx) * hexo::kSwiftFftMaxJ * std::min(n, kBigPass),
-                                 n_big < n ? sizeof(hexo::Cplx) * hexo::kSwiftSmallJ * kSmallPass : 0};
+                                 n_big < n ? sizeof(hexo::Cplx) * hexo::kSwiftSmallJ * std::min(n, kSmallPass) : 0};
     const size_t b_recs = align(sizeof(hexo::DevSwift) * kSmallPass);
     if (int rc = grow_device(ctx, ctx->swift_dev, ctx->swift_dev_bytes,
                              b_strk + 2 * b_blk + 2 * b_recs + (row_bytes[0] + row_bytes[1]) * (1 + rows)))

@@ -4,6 +4,7 @@ Pins: the reference's own golden prices and golden Jacobian (src/UnitTest.cpp:22
 tolerance sum |diff| < 1e-9), the oracle's SWIFT restatement (oracle/swift_oracle.c) on dynamic
 grids, batch invariance, and the Monte-Carlo European prices of the grid workload.
 """
+import ctypes as C
 import json
 import os
 
@@ -273,3 +274,22 @@ def test_swift_call_beyond_the_compute_units(ctx):
             assert res[k][2] == used
             if grads:
                 np.testing.assert_array_equal(res[k][1], gr)
+
+
+def test_swift_workspace_of_a_call_just_beyond_the_compute_units():
+    """257 chains with gradients: 256 of the largest transforms in flight (7 arrays of 64 KiB a chain)
+    and 257 small ones (16 KiB), half as much again to grow into: 210 MiB, kept by the context."""
+    say("gpu swift workspace")
+    chains = [H.SwiftChain(v0=0.04, theta=0.05, rho=-0.6, kappa=1.5, sigma=0.3, S0=100.0, r=0.02, T=1.0 + 0.01 * i,
+                           strikes=np.linspace(90.0, 110.0, 5)) for i in range(257)]
+    c = H.Context(0)
+    c.swift_price(chains, grads=True)
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert c.lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    held = free()
+    c.close()
+    assert 0 < free() - held < 230 << 20
