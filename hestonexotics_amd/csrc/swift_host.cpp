@@ -179,10 +179,44 @@ namespace {
 // trunc, times the width of the log-price range, about 20 standard deviations and the strikes'. Only
 // the order and the class of a chain's workgroup depend on it.
 double size_estimate(const hexo_swift_request& q) {
-    if (q.flags & HEXO_SWIFT_FIXED_GRID) return 0.6 * q.grid.J;  // 1,024 below the line at 630, 2,048 above it
+    if (q.flags & HEXO_SWIFT_FIXED_GRID) return 0.6 * q.grid.J;  // 1,024 below the line at 640, 2,048 above it
     const double u = -std::log(q.trunc) * q.sigma / ((q.v0 + q.kappa * q.theta * q.T) * std::sqrt(1.0 - q.rho * q.rho));
     const double size = u * (0.5 + 20.0 * std::sqrt(std::max(q.v0, q.theta) * q.T));
     return std::isfinite(size) ? size : 1e300;  // ordered in any case
+}
+
+// How the contraction of a pass with `blocks` groups of 16 strikes (of long chains, or in price_large)
+// divides its work: the six gradient rows on three groups of threads while half the CUs have nothing,
+// two strikes a thread where one fills them and a half and most of the second ones exist. Kernel, us:
+// split / plain / two strikes, 33 strikes a chain with gradients, J = 4,096, at 24, 96, 192, 384, 768,
+// 3,000 groups: 56/65/80, 62/68/82, 70/71/84, 129/93/91, 195/140/124, 761/530/410; 5 strikes, 1,000
+// groups 271/196/224.
+struct SumShape {
+    uint32_t strike_block;
+    bool split_rows;
+};
+SumShape sum_shape(const hexo_ctx* ctx, uint64_t blocks, uint64_t n_strikes, uint32_t n_chains) {
+    const uint64_t cus = (uint64_t)ctx->prop.multiProcessorCount;
+    const bool two = 2 * blocks > 3 * cus && n_strikes > 16ull * n_chains;
+    return {two ? hexo::kSwiftStrikeBlock2 : hexo::kSwiftStrikeBlock, 2 * blocks <= cus};
+}
+
+// The most chains of a pass. A pass is three kernels in a row, each with its own end on a half-empty
+// chip: 5,000 chains of 30 strikes with gradients 1,754, 1,598, 1,500 us at 256, 512, 1,024 large
+// (and four times as many small) ones, 2,000 of 21 755, 666, 581.
+constexpr uint32_t kBigPass = 1024, kSmallPass = 4096;
+
+// Quarter octaves of the size estimate, the longest last, from kSizeBig (640) on chains that may
+// exceed kSwiftSmallJ: the estimate is within a factor of 2 of J / 1.3 for nearly all, and of 6,000
+// calibration chains none with J = 2,048 was below 678. One that is after all runs once more.
+constexpr int kSizeClasses = 64, kSizeBig = 24;
+int size_class(double size) {
+    auto octave4 = [](double x) {
+        uint64_t b;
+        std::memcpy(&b, &x, 8);
+        return (int64_t)(b >> 50);  // exponent and the top two bits of the mantissa
+    };
+    return (int)std::clamp<int64_t>(octave4(size) - octave4(640.0) + kSizeBig, 0, kSizeClasses - 1);
 }
 
 // Chains whose transforms exceed the LDS (J > kSwiftFftMaxJ), given their grids, through the direct
@@ -198,7 +232,12 @@ int price_large(hexo_ctx* ctx, const hexo_swift_request* reqs, const std::vector
     std::vector<hexo::SwiftTable> tables;
     std::vector<uint64_t> ends(2 * (size_t)n);  // j, dens
     std::vector<uint32_t> blk_chain, blk_strike;
-    uint64_t n_pay = 0, n_dens = 0, n_pm = 0;
+    uint64_t n_pay = 0, n_dens = 0, n_pm = 0, n_blocks = 0, n_own = 0;
+    for (uint32_t i : idx) {
+        n_blocks += (reqs[i].n_strikes + hexo::kSwiftStrikeBlock - 1u) / hexo::kSwiftStrikeBlock;
+        n_own += reqs[i].n_strikes;
+    }
+    const SumShape shape = sum_shape(ctx, n_blocks, n_own, n);
     hexo::SwiftTotals tot{0, 0, 0};
     for (uint32_t i = 0; i < n; ++i) {
         const hexo_swift_request& q = reqs[idx[i]];
@@ -243,7 +282,7 @@ int price_large(hexo_ctx* ctx, const hexo_swift_request* reqs, const std::vector
         n_dens += nk;
         n_pm += (uint64_t)rows * g.J;
         tot.j += g.J;
-        for (uint32_t o = 0; o < q.n_strikes; o += hexo::kSwiftStrikeBlock) {
+        for (uint32_t o = 0; o < q.n_strikes; o += shape.strike_block) {
             blk_chain.push_back(i);
             blk_strike.push_back(o);
         }
@@ -295,8 +334,8 @@ int price_large(hexo_ctx* ctx, const hexo_swift_request* reqs, const std::vector
     off += b_blk;
     a.block_strike = reinterpret_cast<const uint32_t*>(dev + off);
     a.n_blocks = (uint32_t)blk_chain.size();
-    a.strike_block = hexo::kSwiftStrikeBlock;
-    a.split_rows = true;
+    a.strike_block = shape.strike_block;
+    a.split_rows = shape.split_rows;
     off += b_blk;
     double* d_strikes = reinterpret_cast<double*>(dev + off);
     a.strikes = d_strikes;
@@ -368,18 +407,19 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
     // calibration batch, and one of 4,096 begun last holds up the rest), and those that will not
     // exceed kSwiftSmallJ several to a CU. The others' chain of kernels is as long as the rest of the
     // batch takes, so it runs beside it on a stream of its own.
+    // Sorted into quarter octaves of the estimate only: comparing 5,000 chains took 160 us of the host.
     const bool sorted = n > (uint32_t)ctx->prop.multiProcessorCount;
     uint32_t n_big = n;
     if (sorted) {
-        std::vector<double> size(n);
-        for (uint32_t i = 0; i < n; ++i) {
-            size[i] = size_estimate(reqs[i]);
-            order[i] = i;
+        std::vector<uint8_t> key(n);
+        uint32_t count[kSizeClasses] = {}, first[kSizeClasses];
+        for (uint32_t i = 0; i < n; ++i) ++count[key[i] = (uint8_t)size_class(size_estimate(reqs[i]))];
+        uint32_t at = 0;
+        for (int k = kSizeClasses - 1; k >= 0; at += count[k--]) {
+            first[k] = at;
+            if (k == kSizeBig) n_big = at + count[k];
         }
-        std::stable_sort(order, order + n, [&](uint32_t x, uint32_t y) { return size[x] > size[y]; });
-        // The estimate is within a factor of 2 of J / 1.3 for nearly all: of 6,000 calibration chains
-        // none with J = 2,048 was below 678. One that is after all runs once more (below).
-        n_big = (uint32_t)(std::lower_bound(order, order + n, 630.0, [&](uint32_t x, double v) { return size[x] >= v; }) - order);
+        for (uint32_t i = 0; i < n; ++i) order[first[key[i]]++] = i;
     }
     auto fail = [&](int code, const std::string& msg) {
         // drain what was queued before the pinned stages are reused
@@ -405,72 +445,86 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
         ctx->swift_stream = nullptr;
         return ctx->set_error(HEXO_ERR_HIP, "hipStreamCreate failed");
     }
-    // Work arrays of each class for a pass of up to 256 or 1,024 of the call's chains, each chain with
-    // room for the largest J of its class: no second look at J, and the two streams share nothing that is
-    // written. (How many chains each class gets changes from call to call of a calibration; n does not.)
+    // Work arrays of each class for a pass of the call's chains, each chain with room for the largest J of
+    // its class: no second look at J, and the two streams share nothing that is written. At most
+    // 2 x 470 MB with gradients, 2 x 134 MB without. (How many chains each class gets changes from call to
+    // call of a calibration; n does not.)
     const uint32_t rows = grads ? 6u : 1u;
-    constexpr uint32_t kBigPass = 256, kSmallPass = 1024;
-    const size_t row_bytes[2] = {sizeof(hexo::Cplx) * hexo::kSwiftFftMaxJ * std::min(n, kBigPass),
-                                 n_big < n ? sizeof(hexo::Cplx) * hexo::kSwiftSmallJ * std::min(n, kSmallPass) : 0};
-    const size_t b_recs = align(sizeof(hexo::DevSwift) * kSmallPass);
+    const uint32_t big_pass = std::min(n, kBigPass), small_pass = std::min(n, kSmallPass);
+    const size_t row_bytes[2] = {sizeof(hexo::Cplx) * hexo::kSwiftFftMaxJ * big_pass,
+                                 n_big < n ? sizeof(hexo::Cplx) * hexo::kSwiftSmallJ * small_pass : 0};
+    const size_t b_recs[2] = {align(sizeof(hexo::DevSwift) * big_pass), align(sizeof(hexo::DevSwift) * small_pass)};
     if (int rc = grow_device(ctx, ctx->swift_dev, ctx->swift_dev_bytes,
-                             b_strk + 2 * b_blk + 2 * b_recs + (row_bytes[0] + row_bytes[1]) * (1 + rows)))
+                             b_strk + 2 * b_blk + b_recs[0] + b_recs[1] + (row_bytes[0] + row_bytes[1]) * (1 + rows)))
         return rc;
     unsigned char* dev = reinterpret_cast<unsigned char*>(ctx->swift_dev);
     double* dev_strikes = reinterpret_cast<double*>(dev);
     uint32_t* block_chain = reinterpret_cast<uint32_t*>(dev + b_strk);
     uint32_t* block_strike = reinterpret_cast<uint32_t*>(dev + b_strk + b_blk);
-    // one class of chains, order[k0 .. k1), its contraction workgroups numbered from blk on
-    auto run = [&](int small, uint32_t k0, uint32_t k1, uint32_t& blk, hipStream_t s) {
-        // Two strikes a thread in the contraction where one would already fill the device (2 workgroups
-        // a CU) and most of the second ones exist; not for long chains, which are bound by their own
-        // serial sums. 1,000 chains of J = 512 and 64 strikes with gradients: 107 us instead of 147.
-        const bool two = small && n_blocks > 2ull * ctx->prop.multiProcessorCount && n_strk > 16ull * n;
+    // the next pass of a class of chains, order[k .. end), its contraction workgroups numbered from blk on
+    uint32_t blk = 0;
+    auto run = [&](int small, uint32_t& k, uint32_t end, hipStream_t s) {
+        const uint32_t m = std::min(end - k, small ? small_pass : big_pass), b0 = blk;
+        SumShape shape{hexo::kSwiftStrikeBlock, false};
+        if (small) {
+            // Two strikes a thread where the call would already fill the device with one (2 workgroups a
+            // CU) and most of the second ones exist. 1,000 chains of J = 512 and 64 strikes with gradients:
+            // 107 us instead of 147.
+            if (n_blocks > 2ull * ctx->prop.multiProcessorCount && n_strk > 16ull * n)
+                shape.strike_block = hexo::kSwiftStrikeBlock2;
+        } else if (sorted) {
+            uint64_t blocks = 0, strikes = 0;
+            for (uint32_t i = k; i < k + m; ++i) {
+                const uint32_t ns = chains[order[i]].n_strikes;
+                blocks += (ns + hexo::kSwiftStrikeBlock - 1u) / hexo::kSwiftStrikeBlock;
+                strikes += ns;
+            }
+            shape = sum_shape(ctx, blocks, strikes, m);
+        }
         hexo::SwiftChainArgs c{};
         c.chains = chains;
+        c.order = sorted ? order + k : nullptr;
         c.strikes = h_strikes;
         c.roots = static_cast<const hexo::Cplx*>(ctx->swift_roots);
         c.grids = gout;
         c.dev_strikes = dev_strikes;
         c.block_chain = block_chain;
         c.block_strike = block_strike;
-        c.recs = reinterpret_cast<hexo::DevSwift*>(dev + b_strk + 2 * b_blk + small * b_recs);
-        c.coeff = reinterpret_cast<hexo::Cplx*>(dev + b_strk + 2 * b_blk + 2 * b_recs + (small ? row_bytes[0] * (1 + rows) : 0));
+        c.recs = reinterpret_cast<hexo::DevSwift*>(dev + b_strk + 2 * b_blk + (small ? b_recs[0] : 0));
+        c.coeff = reinterpret_cast<hexo::Cplx*>(dev + b_strk + 2 * b_blk + b_recs[0] + b_recs[1] + (small ? row_bytes[0] * (1 + rows) : 0));
+        c.n_req = m;
         c.max_J = small ? hexo::kSwiftSmallJ : hexo::kSwiftFftMaxJ;
         c.rows = rows;
-        c.strike_block = two ? hexo::kSwiftStrikeBlock2 : hexo::kSwiftStrikeBlock;
+        c.strike_block = shape.strike_block;
+        for (uint32_t i = k; i < k + m; ++i) {
+            hexo::SwiftChainIn& q = chains[sorted ? order[i] : i];
+            q.block_off = blk;
+            blk += (q.n_strikes + c.strike_block - 1u) / c.strike_block;
+        }
+        k += m;
         hexo::SwiftArgs a{};
         a.reqs = c.recs;
+        a.n_req = m;
         a.strikes = dev_strikes;
+        a.block_chain = block_chain + b0;
+        a.block_strike = block_strike + b0;
+        a.n_blocks = blk - b0;
         a.strike_block = c.strike_block;
-        a.split_rows = !small && sorted;
+        a.split_rows = shape.split_rows;
         a.coeff = c.coeff;
         a.pm = c.coeff + row_bytes[small] / sizeof(hexo::Cplx);
         a.prices = h_prices;
         a.grads = h_grads;
-        for (uint32_t k = k0, m; k < k1; k += m) {
-            m = std::min(k1 - k, small ? kSmallPass : kBigPass);
-            const uint32_t b0 = blk;
-            for (uint32_t i = k; i < k + m; ++i) {
-                hexo::SwiftChainIn& q = chains[sorted ? order[i] : i];
-                q.block_off = blk;
-                blk += (q.n_strikes + c.strike_block - 1u) / c.strike_block;
-            }
-            c.order = sorted ? order + k : nullptr;
-            c.n_req = a.n_req = m;
-            a.block_chain = block_chain + b0;
-            a.block_strike = block_strike + b0;
-            a.n_blocks = blk - b0;
-            if (hexo::launch_swift_transform(c, s) != hipSuccess ||
-                hexo::launch_swift_prices(a, c.max_J, s) != hipSuccess)
-                return false;
-        }
-        return true;
+        return hexo::launch_swift_transform(c, s) == hipSuccess && hexo::launch_swift_prices(a, c.max_J, s) == hipSuccess;
     };
+    // the two classes' passes in turn, so that both streams have work from the start
     const bool beside = n_big && n_big < n;
-    uint32_t blk = 0;
-    if (!run(0, 0, n_big, blk, beside ? ctx->swift_stream : st) || !run(1, n_big, n, blk, st) ||
-        (beside && hipStreamSynchronize(ctx->swift_stream) != hipSuccess) || hipStreamSynchronize(st) != hipSuccess)
+    bool ok = true;
+    for (uint32_t big = 0, small = n_big; ok && (big < n_big || small < n);) {
+        if (big < n_big) ok = run(0, big, n_big, beside ? ctx->swift_stream : st);
+        if (ok && small < n) ok = run(1, small, n, st);
+    }
+    if (!ok || (beside && hipStreamSynchronize(ctx->swift_stream) != hipSuccess) || hipStreamSynchronize(st) != hipSuccess)
         return fail(HEXO_ERR_HIP, "SWIFT launch failed");
     // chains that were larger than their class
     uint32_t missed = 0;
@@ -479,8 +533,8 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
             gout[order[k]].g.J <= hexo::kSwiftFftMaxJ)
             order[missed++] = order[k];
     blk = 0;
-    if (missed && (!run(0, 0, missed, blk, st) || hipStreamSynchronize(st) != hipSuccess))
-        return fail(HEXO_ERR_HIP, "SWIFT launch failed");
+    for (uint32_t k = 0; ok && k < missed;) ok = run(0, k, missed, st);
+    if (!ok || (missed && hipStreamSynchronize(st) != hipSuccess)) return fail(HEXO_ERR_HIP, "SWIFT launch failed");
     std::vector<hexo_swift_grid> grids(n);
     std::vector<uint32_t> large;
     for (uint32_t i = 0; i < n; ++i) {

@@ -293,3 +293,19 @@ def test_swift_workspace_of_a_call_just_beyond_the_compute_units():
     held = free()
     c.close()
     assert 0 < free() - held < 230 << 20
+
+
+def test_swift_call_of_several_passes(ctx):
+    """More chains of each class than a pass takes (1,024 of long transforms, 4,096 of short ones), whose
+    contractions split their work in every way: each chain has the bits that it has alone."""
+    kw = dict(v0=0.04, theta=0.05, rho=-0.6, kappa=1.5, sigma=0.3, S0=100.0, r=0.02)
+    g = list(H.swift_grid(H.SwiftChain(**kw, T=1.0, strikes=[80.0, 120.0])))[:7]
+    say("gpu swift call of several passes")
+    for n_long, n_strikes in ((1030, 33), (1030, 5), (40, 33)):
+        chains = [H.SwiftChain(**kw, T=1.0 + 1e-4 * i, strikes=np.linspace(80.0, 120.0, n_strikes),
+                               grid=g + [2048 if i < n_long else 256]) for i in range(n_long + 4100)]
+        res = ctx.swift_price(chains, grads=True)
+        for k in (0, n_long // 2, n_long - 1, n_long, n_long + 4095, n_long + 4099):
+            p, gr, _ = ctx.swift_price([chains[k]], grads=True)[0]
+            np.testing.assert_array_equal(res[k][0], p)
+            np.testing.assert_array_equal(res[k][1], gr)
