@@ -233,7 +233,7 @@ struct ReqPlan {
 struct Layout {
     size_t reqs, segs, fins, opts, order[kPathClasses], item_end[kPathClasses], group_end, out_end;  // uploaded
     size_t upload_end;
-    size_t geo_items, geo_pts, gl, geo_wave_end;                                      // uploaded
+    size_t geo_items, geo_pts, gl;                                                    // uploaded
     size_t counters, counts, partials, groups, prices, ses, finals, geo, geo_panel, geo_pmax, geo_state;  // device
     size_t total;
 };
@@ -261,7 +261,6 @@ Layout make_layout(uint32_t n_req, uint64_t n_seg, uint64_t n_fin, uint64_t n_op
     L.geo_items = take(sizeof(DevGeo) * std::max<uint64_t>(n_geo_items, 1));
     L.geo_pts = take(2 * sizeof(double) * std::max<uint64_t>(n_geo_pts, 1));
     L.gl = take(128 * sizeof(double));
-    L.geo_wave_end = take(sizeof(uint32_t) * std::max<uint64_t>(n_geo_items, 1));
     L.upload_end = o;
     L.counters = take(256);
     L.counts = take(256);
@@ -524,7 +523,6 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     DevGeo* hgi = reinterpret_cast<DevGeo*>(H + L.geo_items);
     double* hgp = reinterpret_cast<double*>(H + L.geo_pts);
     gauss_legendre64(reinterpret_cast<double*>(H + L.gl), reinterpret_cast<double*>(H + L.gl) + 64);
-    uint32_t* hgw = reinterpret_cast<uint32_t*>(H + L.geo_wave_end);
     uint64_t geo_i = 0, geo_p = 0, geo_w = 0;
 
     const double L2E = 1.4426950408889634074;  // log2(e)
@@ -655,7 +653,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
                 g.wave_begin = (uint32_t)geo_w;
                 g.p0 = it.p0;
                 geo_w += it.p0 + 1;
-                hgw[geo_i - 1] = (uint32_t)geo_w;
+                b->ga.max_p0 = std::max(b->ga.max_p0, it.p0);
+                b->ga.max_pts = std::max(b->ga.max_pts, it.n_pts);
             }
             std::memcpy(hgp + 2 * geo_p, p.geo.pts.data(), sizeof(double) * p.geo.pts.size());
             geo_p += p.geo.pts.size() / 2;
@@ -755,8 +754,6 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     ga.gl = reinterpret_cast<const double*>(D + L.gl);
     ga.geo = reinterpret_cast<double*>(D + L.geo);
     ga.n_items = (uint32_t)geo_i;
-    ga.n_waves = (uint32_t)geo_w;
-    ga.wave_end = reinterpret_cast<const uint32_t*>(D + L.geo_wave_end);
     ga.panel = reinterpret_cast<double*>(D + L.geo_panel);
     ga.panel_max = reinterpret_cast<double*>(D + L.geo_pmax);
     ga.state = reinterpret_cast<double*>(D + L.geo_state);

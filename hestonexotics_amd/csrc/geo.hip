@@ -128,22 +128,15 @@ __device__ __forceinline__ double wave_max(double x) {
     return x;  // every lane holds the wave's maximum
 }
 
-__device__ __forceinline__ uint32_t find_item(const uint32_t* end, uint32_t n, uint32_t t) {
-    uint32_t lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (end[mid] > t)
-            hi = mid;
-        else
-            lo = mid + 1;
-    }
-    return lo;
-}
-
 // Panel p of an item, by one workgroup: lane q evaluates node q, u_q = (p + (x_q + 1)/2) h, and
-// phi(1/2 - i u_q) weighted by w_q (h/2) / (u_q^2 + 1/4); then lane i of each wavefront sums strike
-// i's Re(e^{i u_q k_i} weighted phi) over 8 nodes, node by node, and wavefront kGeoHelpers adds and
-// returns the eight sums in order, with the maximum of |phi| over the panel in *mag.
+// phi(1/2 - i u_q) weighted by w_q (h/2) / (u_q^2 + 1/4); then each wavefront sums
+// Re(e^{i u_q k_i} weighted phi) over 8 nodes for every strike i, and wavefront kGeoHelpers adds and
+// returns the eight sums in order, with the maximum of |phi| over the panel in *mag. Up to 32 strikes
+// are taken eight at a time, a lane per strike and node, the nodes added by a fixed tree: a lane per
+// strike that goes through the nodes has eight sine-cosine pairs for one strike too, most of the
+// time of a panel of a short grid (324 items of 2 steps and a strike 1,007 -> 819 us). With more it
+// saves less than the exchanges cost (222 items of 28 steps, whole call: 21 strikes 3,788 -> 3,708 us, 40
+// strikes 3,868 -> 3,892).
 // Panel 0 holds the integrand's 1/(u^2 + 1/4) peak at u = 0, which 64 nodes integrate to 1e-13
 // over [0, 16] but only to 1e-4 over [0, 120]: it is summed as n_sub = min(64, ceil(h / 16))
 // sub-panels of 64 nodes (wave-uniform, in order). The other panels keep width h.
@@ -156,6 +149,7 @@ __device__ double panel_sum(const GeoArgs& a, const DevGeo& G, const DevReq& R, 
     const uint32_t n_sub = p == 0 ? first_panel_parts(G.h) : 1u;
     const double hs = G.h / (double)n_sub;
     constexpr int kNodes = 64 / kGeoWaves;  // per wavefront
+    constexpr uint32_t kTreeStrikes = 32;
     double sum = 0.0, mg = 0.0;
     for (uint32_t j = 0; j < n_sub; ++j) {
         const double u = ((double)(p + j) + 0.5 * (a.gl[lane] + 1.0)) * hs;  // p = 0 or j = 0
@@ -168,17 +162,30 @@ __device__ double panel_sum(const GeoArgs& a, const DevGeo& G, const DevReq& R, 
             mg = fmax(mg, wave_max(cabs_(ph)));
         }
         __syncthreads();
-        double part = 0.0;
-        if (has_k) {
-            for (int q = w * kNodes; q < (w + 1) * kNodes; ++q) {
+        if (G.n_strikes > kTreeStrikes) {
+            double part = 0.0;
+            if (has_k) {
+                for (int q = w * kNodes; q < (w + 1) * kNodes; ++q) {
+                    double sn, cs;
+                    sincos(sh.node[2][q] * k, &sn, &cs);
+                    part += cs * sh.node[0][q] - sn * sh.node[1][q];
+                }
+            }
+            sh.part[w][lane] = part;
+        } else {
+            const int q = w * kNodes + lane % kNodes;
+            for (int i = lane / kNodes; i - lane / kNodes < (int)G.n_strikes; i += 64 / kNodes) {
+                const double ki = __shfl(k, i);
                 double sn, cs;
-                sincos(sh.node[2][q] * k, &sn, &cs);
-                part += cs * sh.node[0][q] - sn * sh.node[1][q];
+                sincos(sh.node[2][q] * ki, &sn, &cs);
+                double part = cs * sh.node[0][q] - sn * sh.node[1][q];
+#pragma unroll
+                for (int m = 1; m < kNodes; m <<= 1) part += __shfl_xor(part, m);
+                if (lane % kNodes == 0) sh.part[w][i] = part;
             }
         }
-        sh.part[w][lane] = part;
         __syncthreads();
-        if (w == kGeoHelpers) {
+        if (w == kGeoHelpers && has_k) {
 #pragma unroll
             for (int v = 0; v < kGeoWaves; ++v) sum += sh.part[v][lane];
         }
@@ -204,15 +211,24 @@ constexpr int kGeoRounds = 3;  // parallel rounds of p0 panels before the serial
 // Pass 1 of round r: every workgroup evaluates one panel of one unconverged item (round r covers
 // that item's panels done .. done + p0 - 1) and stores each strike's panel sum; in the first round the
 // item's last workgroup evaluates E[e^L] instead.
+// The grid is items x panels, without those past an item's p0: found from a prefix sum over the items, a
+// workgroup's item cost it nine dependent loads at 324 items. Item by item, or where all grids are short
+// panel by panel, so that the first panels, which take longest, begin first: 324 items of 2, 6, 12,
+// 24, 52, 252 steps 913/831, 1,103/1,076, 1,314/1,298, 1,744/1,764, 2,971/3,001, 10,864/11,534 us.
+constexpr uint32_t kShortGrid = 16;     // points
+constexpr uint32_t kGridItems = 65535;  // the most blocks in y and z of a grid
 __global__ __launch_bounds__(64 * kGeoWaves) void k_geo_panels(GeoArgs a, uint32_t round) {
     __shared__ GeoShared sh;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
-    const uint32_t wv = blockIdx.x;
-    const uint32_t item = __builtin_amdgcn_readfirstlane(find_item(a.wave_end, a.n_items, wv));
+    const bool panels_first = a.max_pts <= kShortGrid;
+    const uint32_t item = panels_first ? blockIdx.x : blockIdx.z * kGridItems + blockIdx.y;
+    const uint32_t j = panels_first ? blockIdx.y : blockIdx.x;
+    if (item >= a.n_items) return;
     const DevGeo& G = a.items[item];
+    if (j > G.p0) return;
+    const uint32_t wv = G.wave_begin + j;
     const DevReq& R = a.reqs[G.req];
     const double* pts = a.pts + 2 * (size_t)G.pts_begin;
-    const uint32_t j = wv - G.wave_begin;
     const double* st = a.state + (size_t)item * kGeoState;
     uint32_t base = 0;
     if (round > 0) {
@@ -312,7 +328,11 @@ size_t geo_state_doubles(uint32_t n_items) { return (size_t)n_items * kGeoState;
 hipError_t launch_geo(const GeoArgs& a, bool first, hipStream_t st) {
     if (a.n_items == 0) return hipSuccess;
     for (uint32_t r = first ? 0u : 1u; r < (first ? 1u : (uint32_t)kGeoRounds); ++r) {
-        k_geo_panels<<<a.n_waves, 64 * kGeoWaves, 0, st>>>(a, r);
+        const uint32_t per_item = a.max_p0 + 1;
+        const dim3 grid = a.max_pts <= kShortGrid ? dim3(a.n_items, per_item)
+                                                  : dim3(per_item, a.n_items < kGridItems ? a.n_items : kGridItems,
+                                                         (a.n_items + kGridItems - 1) / kGridItems);
+        k_geo_panels<<<grid, 64 * kGeoWaves, 0, st>>>(a, r);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         k_geo_sum<<<a.n_items, 64 * kGeoWaves, 0, st>>>(a, r);

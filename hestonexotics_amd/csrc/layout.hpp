@@ -141,8 +141,7 @@ struct GeoArgs {
     const double* gl;   // 64 Gauss-Legendre nodes on [-1, 1], then their 64 weights
     double* geo;        // exact geometric prices (undiscounted, absolute units), per output
     uint32_t n_items;
-    uint32_t n_waves;       // workgroups of the parallel panel pass (sum over items of p0 + 1)
-    const uint32_t* wave_end;  // inclusive prefix over items of p0 + 1
+    uint32_t max_p0, max_pts;  // over the items
     double* panel;          // per panel: each strike's panel sum (64 doubles)
     double* panel_max;      // per panel: max |phi| over its nodes; E[e^L] in the item's last
     double* state;          // per item between rounds: strike sums, E[e^L], panels done, converged

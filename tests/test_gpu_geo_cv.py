@@ -275,3 +275,22 @@ def test_exact_price_near_deterministic(ctx, oracle, case):
     np.testing.assert_allclose(g, o, rtol=0, atol=1e-9 * 100.0)
     tol = 1e-9 * EG
     assert np.all(g >= -tol) and np.all(g >= EG - np.array(K) - tol) and np.all(np.diff(g) <= tol)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 129])
+def test_exact_geometric_price_of_n_strikes(ctx, oracle, n):
+    """The panels' sums take up to 32 strikes eight at a time, more one a lane, 64 to a block; some strikes
+    are 0 or negative (no integral). Against the oracle as above, and the same bits in a batch of items of other sizes."""
+    K = np.linspace(70.0, 130.0, n)
+    K[n // 2:: 5] = (0.0, -5.0)[n % 2]
+    req = H.Request(**BASE, expiries=[1.0], strikes=[list(K)], steps=12, n_paths=64, seed=2, r=0.02, flags=H.DRIFT,
+                    payoffs=H.ASIAN_GEO_CV, precision=H.FP64)
+    say("gpu geo exact, strikes", n)
+    g = ctx.geo_asian_price(req)
+    o = oracle.geo_asian_price(req.params, req.S0, req.expiries, req.n_strikes(), req.flat_strikes(), steps=12,
+                               r=req.r, flags=req.flags)
+    np.testing.assert_allclose(g, o, rtol=0, atol=1e-9 * req.S0)
+    others = [H.Request(**BASE, expiries=[0.2, 2.0], strikes=[[90.0] * k, [100.0]], steps=s, n_paths=64, seed=1, r=0.02,
+                        payoffs=H.ASIAN_GEO_CV, precision=H.FP64) for k, s in ((3, 5), (70, 30))]
+    alone = ctx.price(req)
+    np.testing.assert_array_equal(ctx.price_batch([others[0], req, others[1]])[1][0], alone[0])
