@@ -54,14 +54,20 @@ __device__ __forceinline__ Cplx ccosh(Cplx a) {
     return Cplx{cosh(a.re) * c, sinh(a.re) * s};
 }
 
+__device__ __forceinline__ Cplx mul_add(Cplx a, Cplx b, double c) {  // a b + c
+    return Cplx{__builtin_fma(a.re, b.re, __builtin_fma(-a.im, b.im, c)),
+                __builtin_fma(a.re, b.im, a.im * b.re)};
+}
+
 // log(1 + z) and exp(w) - 1 without cancellation for small arguments (short series below 1e-3,
 // whose truncation error is below 1e-15 relative)
 __device__ __forceinline__ Cplx clog1p(Cplx z) {
     if (hypot(z.re, z.im) < 1e-3) {
         // z (1 - z (1/2 - z (1/3 - z/4)))
-        Cplx t = cx(1.0 / 3.0) - 0.25 * z;
-        t = cx(0.5) - z * t;
-        t = cx(1.0) - z * t;
+        const Cplx m = cx(-z.re, -z.im);
+        Cplx t = cx(__builtin_fma(0.25, m.re, 1.0 / 3.0), 0.25 * m.im);
+        t = mul_add(m, t, 0.5);
+        t = mul_add(m, t, 1.0);
         return z * t;
     }
     return clog(cx(1.0 + z.re, z.im));
@@ -69,13 +75,15 @@ __device__ __forceinline__ Cplx clog1p(Cplx z) {
 __device__ __forceinline__ Cplx cexpm1(Cplx w) {
     if (hypot(w.re, w.im) < 1e-3) {
         // w (1 + w (1/2 + w (1/6 + w/24)))
-        Cplx t = cx(1.0 / 6.0) + (1.0 / 24.0) * w;
-        t = cx(0.5) + w * t;
-        t = cx(1.0) + w * t;
+        Cplx t = cx(__builtin_fma(1.0 / 24.0, w.re, 1.0 / 6.0), 1.0 / 24.0 * w.im);
+        t = mul_add(w, t, 0.5);
+        t = mul_add(w, t, 1.0);
         return w * t;
     }
-    const Cplx e = cexp(w);
-    return Cplx{e.re - 1.0, e.im};
+    double s, c;
+    sincos(w.im, &s, &c);
+    const double e = exp(w.re);
+    return Cplx{__builtin_fma(e, c, -1.0), e * s};
 }
 
 }  // namespace hexo

@@ -335,6 +335,20 @@ static_assert(kSplitMaxSteps <= 1ull << 31 && split_draw_waves(0, 1, 1, kSplitMa
                   split_draw_waves(1, 1, 1, (1ull << 32) + 2, false, false, true) == 0,
               "a step count near or past 2^32 never reaches the drawing waves");
 
+// Whether the exact geometric prices' panels are evaluated by a wavefront each, eight to a CU, or by a
+// workgroup each, one to a CU, in a third of the time on a long grid (geo.hip). By the number of panels
+// as long as the longest that make up the work. Kernel time, us, workgroup / wavefront, at
+// 174, 348, 696, 1,392, 28,188 equal panels on 256 CUs (long grids: 786 and 1,347 unequal ones of 1,000
+// steps, whole call: 4,430/4,651 and 7,561/6,733):
+//    2 steps  12/14    19/13    29/13    55/19    972/200
+//   12 steps  16/26    29/26    41/26    80/40    1,369/495
+//   24 steps  20/41    36/41    56/43    109/73   1,834/876
+//   52 steps  30/74    57/76    88/79    176/132  3,047/1,724
+//  252 steps  105/320  211/330  318/344  613/563  11,301/7,708
+bool geo_by_wave(double panels, double steps, int n_cu) {
+    return panels > n_cu * (0.7 + 3.4 * steps / (steps + 50.0));
+}
+
 bool plan_request(const hexo_request* r, ReqPlan& p) {
     if (!build_schedule(r->expiries, r->n_expiries, r->n_strikes, r->steps, p.segs, p.total_steps)) return false;
     p.n_opts = n_opts_of(r);
@@ -524,6 +538,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     double* hgp = reinterpret_cast<double*>(H + L.geo_pts);
     gauss_legendre64(reinterpret_cast<double*>(H + L.gl), reinterpret_cast<double*>(H + L.gl) + 64);
     uint64_t geo_i = 0, geo_p = 0, geo_w = 0;
+    uint32_t geo_pts_max = 0;
+    double geo_work = 0.0;  // panels times steps (and 8 steps' time for the rest of a panel)
 
     const double L2E = 1.4426950408889634074;  // log2(e)
     uint64_t seg_i = 0, fin_i = 0, opt_i = 0, part_i = 0, grp_i = 0, out_i = 0, ge = 0;
@@ -650,11 +666,12 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
                 g.out = out_i + cvpay * p.n_opts + it.opt;
                 g.c = it.c;
                 g.h = it.h;
-                g.wave_begin = (uint32_t)geo_w;
+                g.slot_begin = (uint32_t)geo_w;
                 g.p0 = it.p0;
                 geo_w += it.p0 + 1;
                 b->ga.max_p0 = std::max(b->ga.max_p0, it.p0);
-                b->ga.max_pts = std::max(b->ga.max_pts, it.n_pts);
+                geo_pts_max = std::max(geo_pts_max, it.n_pts);
+                geo_work += (it.p0 + 1.0) * (it.n_pts + 8.0);
             }
             std::memcpy(hgp + 2 * geo_p, p.geo.pts.data(), sizeof(double) * p.geo.pts.size());
             geo_p += p.geo.pts.size() / 2;
@@ -754,6 +771,8 @@ int batch_create(hexo_ctx* ctx, const hexo_request* reqs, uint32_t n, hipStream_
     ga.gl = reinterpret_cast<const double*>(D + L.gl);
     ga.geo = reinterpret_cast<double*>(D + L.geo);
     ga.n_items = (uint32_t)geo_i;
+    ga.by_wave = geo_by_wave(geo_work / (geo_pts_max + 8.0), geo_pts_max,
+                             ctx->prop.multiProcessorCount > 0 ? ctx->prop.multiProcessorCount : 256);
     ga.panel = reinterpret_cast<double*>(D + L.geo_panel);
     ga.panel_max = reinterpret_cast<double*>(D + L.geo_pmax);
     ga.state = reinterpret_cast<double*>(D + L.geo_state);

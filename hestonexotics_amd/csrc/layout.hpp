@@ -115,7 +115,7 @@ struct PathArgs {
 // Geometric-average control variate (payoff HEXO_ASIAN_GEO_CV). The Asian functional of an
 // expiry, A = sum_j w_j X_{t_j} over the grid points, has weight sum W; its geometric counterpart
 // is G = W S0 exp(sum_j v_j ln(X_{t_j}/S0)) with v = w / W, whose exact price under the Heston
-// model is computed once per batch: one wavefront per (request, expiry, block of <= 64 strikes).
+// model is computed once per batch, per (request, expiry, block of <= 64 strikes).
 struct DevGeo {
     uint32_t req;         // request index
     uint32_t pts_begin;   // first point (t_0 = 0) of the expiry's (t_j, v_j) list
@@ -123,8 +123,8 @@ struct DevGeo {
     uint32_t n_strikes;   // strikes of this block (<= 64)
     uint32_t opt;         // first option of the block (batch-global DevOpt index)
     uint32_t max_panels;  // bound on 64-node panels (the price is NaN if not converged by then)
-    uint32_t wave_begin;  // first workgroup of the item in the parallel panel pass
-    uint32_t p0;          // panels evaluated in parallel (that pass has p0 + 1 workgroups: the last one E[e^L])
+    uint32_t slot_begin;  // first of the item's p0 + 1 slots in GeoArgs.panel and panel_max
+    uint32_t p0;          // panels evaluated in parallel (and E[e^L], in the last slot)
     uint64_t out;         // geo[] index of the block's first control-variate output
     double c;             // W S0
     double h;             // width in u of one panel
@@ -141,7 +141,8 @@ struct GeoArgs {
     const double* gl;   // 64 Gauss-Legendre nodes on [-1, 1], then their 64 weights
     double* geo;        // exact geometric prices (undiscounted, absolute units), per output
     uint32_t n_items;
-    uint32_t max_p0, max_pts;  // over the items
+    uint32_t max_p0;  // over the items
+    bool by_wave;     // a panel per wavefront, not per workgroup
     double* panel;          // per panel: each strike's panel sum (64 doubles)
     double* panel_max;      // per panel: max |phi| over its nodes; E[e^L] in the item's last
     double* state;          // per item between rounds: strike sums, E[e^L], panels done, converged

@@ -294,3 +294,24 @@ def test_exact_geometric_price_of_n_strikes(ctx, oracle, n):
                         payoffs=H.ASIAN_GEO_CV, precision=H.FP64) for k, s in ((3, 5), (70, 30))]
     alone = ctx.price(req)
     np.testing.assert_array_equal(ctx.price_batch([others[0], req, others[1]])[1][0], alone[0])
+
+
+@pytest.mark.parametrize("n", [1, 9, 32, 33, 64, 70])
+@pytest.mark.parametrize("steps", [2, 7, 8, 15, 61])
+def test_exact_price_by_a_wavefront_equals_by_a_workgroup(ctx, steps, n):
+    """A batch with panels enough to fill the GPU evaluates each by one wavefront, a request alone by a
+    workgroup: the same bits, for parameters that converge in the first round and (a variance near 0)
+    in later ones."""
+    K = np.linspace(70.0, 130.0, n)
+    K[n // 2:: 7] = 0.0
+    say("gpu geo exact by a wavefront", steps, n)
+    reqs = []
+    for model in (BASE, dict(BASE, kappa=0.5, sigma=0.9, rho=-0.9), dict(BASE, v0=0.004, theta=0.004, kappa=0.5, sigma=1.0, rho=-0.9)):
+        for e in ([1.0], [0.4, 1.0]):
+            reqs.append(H.Request(**model, expiries=e, strikes=[list(K)] * len(e), steps=steps, n_paths=64, seed=2, r=0.02,
+                                  flags=H.DRIFT, payoffs=H.ASIAN_GEO_CV, precision=H.FP64))
+    alone = [ctx.price(r) for r in reqs]
+    batch = [dataclasses.replace(r) for r in reqs * 3]  # a request holds the arrays of one C struct
+    for (p, s), (q, t) in zip(alone, ctx.price_batch(batch)[len(reqs):]):
+        np.testing.assert_array_equal(p, q)
+        np.testing.assert_array_equal(s, t)
