@@ -299,9 +299,12 @@ uint64_t split_most_tiles(const ReqPlan& p) {
 //    (1e4 paths x 126 steps 28.5 -> 20.4 us against one). Beyond, the third wave competes with
 //    other tiles' stepping waves: 5% faster still for quadratic-branch steps at 1,500 tiles, 15%
 //    slower where the stepping wave is the longer one (martingale correction, exponential branch).
-//  * up to 2^17 tiles (1e6 paths for each of the grid workload's 8 maturities): one drawing wave.
-//    At 125,000 tiles the grid takes 1.72 ms against the persistent kernel's 1.80 and 64 uneven
-//    requests 8.6 to 8.8 ms against 8.7; at 370,000 tiles they take 25.8 ms against 25.3: there the
+//  * up to 2^17 tiles (1e6 paths for each of the grid workload's 8 maturities): one drawing wave. A batch
+//    persistent / split, ms, at 31,000, 62,500, 94,000, 125,000, 156,000, 187,500, 375,000 tiles:
+//      8 x 52 steps, 64 strikes  .373/.321  .576/.518  .799/.748  1.02/.98  1.24/1.23  1.46/1.48  2.80/2.93
+//      8 x 52 steps, 1 strike    .333/.254  .524/.435  .706/.632  .91/.83   1.09/1.02  1.29/1.21  2.43/2.38
+//      8 x 252 steps, 21 strikes 1.04/.98   1.89/1.88  2.80/2.79  3.66/3.68 4.53/4.59  5.43/5.49  10.6/10.9
+//    64 uneven requests of 252 steps take 3.58/3.59 at 125,000 and 10.4/10.6 at 375,000. There the
 //    persistent kernel's waves are full and it has no draws to carry through LDS.
 //  * up to 2^16 tiles with the geometric average, whose payoffs are more of the stepping wave's work:
 //    the grid with 64 strikes and 4, 3, 2 payoffs takes 2.35, 2.06, 1.98 ms at 125,000 tiles against

@@ -790,17 +790,31 @@ __device__ __forceinline__ void path_fp32(const PathArgs& a, uint32_t ri, uint32
     if constexpr (COUNT) count_flush(a.counts, cnt.quad, cnt.exp, cnt.central, cnt.tail, lane);
 }
 
+// The workgroup's LDS, aligned for path_fp32's values of an expiry. Without the geometric average these are
+// float2: declared 16-byte aligned, its reads of two of them become single 16-byte ones, and the 512
+// uneven requests take 682.5 ms against 676.5.
+template <bool GEO>
+__device__ __forceinline__ uint32_t* path_lds() {
+    if constexpr (GEO) {
+        extern __shared__ __align__(16) uint32_t lds_16[];
+        static_assert(__alignof__(lds_16) >= alignof(float4));
+        return lds_16;
+    } else {
+        extern __shared__ __align__(8) uint32_t lds_8[];
+        static_assert(__alignof__(lds_8) >= alignof(float2));
+        return lds_8;
+    }
+}
+
 // Registers for 5 waves per SIMD at 2 paths per lane (96), 4 with the martingale step: it needs 114,
 // and held to 96 it spilled 22 (4e6 paths x 252 steps 2.58 -> 2.48 ms, 2^20 stiff paths x 2,048 steps
 // 7.15 -> 6.90). With the geometric average as well it spills as much, but its payoff sums want
 // the fifth wave more (1,000 strikes x 3 payoffs x 52 steps, 3.5e6 paths 3.79 -> 3.30 ms with it).
 template <int PPT, bool DEBUG, bool COUNT, bool MART, bool GEO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PPT == 2 && (!MART || GEO) ? 5 : 4, 8))) void k_path_fp32(PathArgs a) {
-    extern __shared__ __align__(16) uint32_t lds_u32[];
-    static_assert(__alignof__(lds_u32) >= alignof(float4), "path_fp32 stores float4 there");
     const int lane = (int)(threadIdx.x & 63u);
     // the wave's LDS region, at a wave-uniform address
-    uint32_t* lds = lds_u32 + uniform(threadIdx.x >> 6) * WaveLds<PPT>::kWords;
+    uint32_t* lds = path_lds<GEO>() + uniform(threadIdx.x >> 6) * WaveLds<PPT>::kWords;
     for (;;) {
         const uint32_t item = next_item(a.counter, lane);
         if (item >= a.total_items) break;
