@@ -102,7 +102,6 @@ int check_grid(const hexo_swift_grid& g, std::string& err) {
     return HEXO_OK;
 }
 
-// SwiftParameters constructor (src/SWIFT.cpp:21-35).
 // The extreme strikes and the rest of a chain's grid-choice inputs.
 hexo::SwiftGridIn grid_input(const hexo_swift_request& q) {
     hexo::SwiftGridIn in{{q.v0, q.theta, q.rho, q.kappa, q.sigma}, q.T, q.r, q.S0, q.strikes[0], q.strikes[0], q.trunc};
@@ -185,12 +184,13 @@ double size_estimate(const hexo_swift_request& q) {
     return std::isfinite(size) ? size : 1e300;  // ordered in any case
 }
 
-// How the contraction of a pass with `blocks` groups of 16 strikes (of long chains, or in price_large)
-// divides its work: the six gradient rows on three groups of threads while half the CUs have nothing,
+// How the contraction of a pass with `blocks` groups of 16 strikes (of long chains, or in price_large; as
+// many as would take as long if all chains were the longest) divides its work: the six gradient rows on three groups of threads while half the CUs have nothing,
 // two strikes a thread where one fills them and a half and most of the second ones exist. Kernel, us:
 // split / plain / two strikes, 33 strikes a chain with gradients, J = 4,096, at 24, 96, 192, 384, 768,
 // 3,000 groups: 56/65/80, 62/68/82, 70/71/84, 129/93/91, 195/140/124, 761/530/410; 5 strikes, 1,000
-// groups 271/196/224.
+// groups 271/196/224. 512 calibration chains, whose 676 groups of J up to 4,096 count as fewer than 384:
+// whole call 306 us, 318 with two strikes a thread.
 struct SumShape {
     uint32_t strike_block;
     bool split_rows;
@@ -410,8 +410,8 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
     // Sorted into quarter octaves of the estimate only: comparing 5,000 chains took 160 us of the host.
     const bool sorted = n > (uint32_t)ctx->prop.multiProcessorCount;
     uint32_t n_big = n;
+    std::vector<uint8_t> key(sorted ? n : 0);
     if (sorted) {
-        std::vector<uint8_t> key(n);
         uint32_t count[kSizeClasses] = {}, first[kSizeClasses];
         for (uint32_t i = 0; i < n; ++i) ++count[key[i] = (uint8_t)size_class(size_estimate(reqs[i]))];
         uint32_t at = 0;
@@ -473,13 +473,16 @@ extern "C" int hexo_swift_price(hexo_ctx* ctx, const hexo_swift_request* reqs, u
             if (n_blocks > 2ull * ctx->prop.multiProcessorCount && n_strk > 16ull * n)
                 shape.strike_block = hexo::kSwiftStrikeBlock2;
         } else if (sorted) {
-            uint64_t blocks = 0, strikes = 0;
+            uint64_t blocks[kSizeClasses] = {}, strikes = 0;
             for (uint32_t i = k; i < k + m; ++i) {
                 const uint32_t ns = chains[order[i]].n_strikes;
-                blocks += (ns + hexo::kSwiftStrikeBlock - 1u) / hexo::kSwiftStrikeBlock;
+                blocks[key[order[i]]] += (ns + hexo::kSwiftStrikeBlock - 1u) / hexo::kSwiftStrikeBlock;
                 strikes += ns;
             }
-            shape = sum_shape(ctx, blocks, strikes, m);
+            double longest = 0.0;
+            for (int c = 0; c <= key[order[k]]; ++c)
+                longest += (double)blocks[c] * std::exp2(0.25 * (c - key[order[k]]));
+            shape = sum_shape(ctx, (uint64_t)longest, strikes, m);
         }
         hexo::SwiftChainArgs c{};
         c.chains = chains;
