@@ -108,7 +108,8 @@ __device__ __forceinline__ Cplx geo_advance(Cplx Bm, Cplx e, Cplx Z, Cplx& B) {
     return z;
 }
 // A: the helpers' sums of dA, then of the logarithms.
-__device__ __forceinline__ Cplx geo_phi(const DevReq& R, const Cplx (&A)[2][kGeoHelpers][64], Cplx B, int lane) {
+__device__ __forceinline__ Cplx geo_phi(const DevReq& R, const Cplx (&A)[2][kGeoHelpers][64], Cplx B,
+                                        int lane) {
     const double k2 = 2.0 * R.kappa * R.theta / (R.sigma * R.sigma);
     Cplx dA = cx(0.0), lg = cx(0.0);
 #pragma unroll
@@ -119,8 +120,11 @@ __device__ __forceinline__ Cplx geo_phi(const DevReq& R, const Cplx (&A)[2][kGeo
     return cexp((dA - k2 * lg) + R.v0 * B);
 }
 
-// By a wavefront, the sums of a lane in LDS.
-__device__ Cplx geo_cf_wave(const DevReq& R, const double* pts, uint32_t n, Cplx s, Cplx (&A)[2][kGeoHelpers][64], int lane) {
+// By a wavefront, the sums of a lane in LDS: at 250 registers two wavefronts share a SIMD, and a batch
+// with panels enough to fill them needs no helpers to wait for (324 items of 2 steps 972 -> 200 us, of
+// 252 steps 11.3 -> 7.7 ms against a workgroup per panel; the rule is in engine.cpp).
+__device__ Cplx geo_cf_wave(const DevReq& R, const double* pts, uint32_t n, Cplx s,
+                            Cplx (&A)[2][kGeoHelpers][64], int lane) {
 #pragma unroll
     for (int h = 0; h < kGeoHelpers; ++h) A[0][h][lane] = A[1][h][lane] = cx(0.0);
     const GeoModel M(R);
@@ -219,7 +223,8 @@ __device__ __forceinline__ uint32_t first_panel_parts(double h) {
 __device__ __forceinline__ double node_u(const GeoArgs& a, uint32_t panel, double h, int lane) {
     return ((double)panel + 0.5 * (a.gl[lane] + 1.0)) * h;
 }
-__device__ __forceinline__ void store_node(const GeoArgs& a, double (&node)[3][64], Cplx phi, double u, double h, int lane) {
+__device__ __forceinline__ void store_node(const GeoArgs& a, double (&node)[3][64], Cplx phi, double u,
+                                           double h, int lane) {
     const double f = 0.5 * h * a.gl[64 + lane] / (u * u + 0.25);
     node[0][lane] = f * phi.re;
     node[1][lane] = f * phi.im;
@@ -477,7 +482,8 @@ hipError_t launch_geo(const GeoArgs& a, bool first, hipStream_t st) {
         const uint32_t per_item = a.max_p0 + 1, rows = a.n_items < kGridItems ? a.n_items : kGridItems;
         const uint32_t layers = (a.n_items + kGridItems - 1) / kGridItems;
         if (a.by_wave)
-            k_geo_panels_wave<<<dim3((per_item + kPanelWaves - 1) / kPanelWaves, rows, layers), 64 * kPanelWaves, 0, st>>>(a, r);
+            k_geo_panels_wave<<<dim3((per_item + kPanelWaves - 1) / kPanelWaves, rows, layers),
+                                64 * kPanelWaves, 0, st>>>(a, r);
         else
             k_geo_panels<<<dim3(per_item, rows, layers), 64 * kGeoWaves, 0, st>>>(a, r);
         hipError_t e = hipGetLastError();

@@ -55,7 +55,9 @@ __device__ __forceinline__ double exp_f64(double y) {
     return __builtin_amdgcn_ldexp(e, (int)n);
 }
 
-// ln x for x > 0 in the normal range: x = 2^e m, f = m - 1, ln m = f - s (f - s^2 P(s^2)).
+// ln x for x > 0 in the normal range: x = 2^e m, f = m - 1, ln m = f - s (f - s^2 P(s^2)). This form, and
+// ln 2 in two parts, are those of the logarithm of fdlibm (Sun Microsystems, 1993); the coefficients are
+// from math_f64_fit.py.
 __device__ __forceinline__ double log_f64(double x) {
     double m = __builtin_amdgcn_frexp_mant(x);  // [1/2, 1)
     const bool low = m < 0.70710678118654752440;

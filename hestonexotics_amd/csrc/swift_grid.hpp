@@ -1,6 +1,6 @@
 // swift_grid.hpp -- the dynamic SWIFT grid (the reference's SwiftParameters constructor,
-// src/SWIFT.cpp:21-35), shared by the host (hexo_swift_grid_for) and the GPU grid kernel that
-// hexo_swift_price runs for all of a call's chains at once.
+// src/SWIFT.cpp:21-35), shared by the host (hexo_swift_grid_for) and k_swift_transform, whose first
+// wavefront chooses its chain's grid.
 #pragma once
 
 #include <hip/hip_runtime.h>

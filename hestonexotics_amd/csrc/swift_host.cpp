@@ -185,8 +185,9 @@ double size_estimate(const hexo_swift_request& q) {
 }
 
 // How the contraction of a pass with `blocks` groups of 16 strikes (of long chains, or in price_large; as
-// many as would take as long if all chains were the longest) divides its work: the six gradient rows on three groups of threads while half the CUs have nothing,
-// two strikes a thread where one fills them and a half and most of the second ones exist. Kernel, us:
+// many as would take as long if all chains were the longest) divides its work: the six gradient rows on
+// three groups of threads while half the CUs have nothing, two strikes a thread where one fills them
+// and a half and most of the second ones exist. Kernel, us:
 // split / plain / two strikes, 33 strikes a chain with gradients, J = 4,096, at 24, 96, 192, 384, 768,
 // 3,000 groups: 56/65/80, 62/68/82, 70/71/84, 129/93/91, 195/140/124, 761/530/410; 5 strikes, 1,000
 // groups 271/196/224. 512 calibration chains, whose 676 groups of J up to 4,096 count as fewer than 384:
