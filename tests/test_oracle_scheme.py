@@ -268,9 +268,9 @@ def test_path_offset_selects_the_same_paths():
     np.testing.assert_array_equal(full[150:250], part)
 
 
-def test_fast_oracle_leaves_subnormals_to_the_checker():
+def test_fast_oracle_leaves_subnormals_to_the_strict_one():
     """The timed build, compiled with -ffast-math, must not switch the process to flush-to-zero: at
-    S0 = 1e-305 the average's last interval (X - Xp)(T - tp) is subnormal, and the checker's finals
+    S0 = 1e-305 the average's last interval (X - Xp)(T - tp) is subnormal, and the strict oracle's finals
     are 1e-305 times those at S0 = 1 (to 1e-9: ln X = -702 carries 1e-13 a step; flushed, they are off
     by 8%)."""
     kw = dict(steps=9, n_paths=130, seed=13, want_finals=True)
